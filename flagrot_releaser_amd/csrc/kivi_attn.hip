@@ -1,5 +1,6 @@
 // extern "C" surface of libflagrot_kivi.so (declared in include/flagrot_kivi.h) and the split merge of the decode
-// attention.  The writers, the dequantiser and the LSE merge are in kivi_write.hip, the decode splits in kivi_decode.hip, everything of head dim 256 in kivi_wide.hip.
+// attention.  The value writer, the dequantiser and the LSE merge are in kivi_write.hip, the key group encoder in
+// kivi_kenc.hip, the decode splits in kivi_decode.hip, the rest of head dim 256 in kivi_wide.hip.
 // Semantics follow integrations/vllm_flagrot/csrc/kivi.cu:1908-1931 (k_merge) and :1933-2342 (C ABI).
 #include <cstdio>
 #include <cstring>
@@ -54,12 +55,7 @@ int kv_k_encode(const void* src, long long src_rs, const void* src2, long long s
                 int ident, const void* kfix, int f8, void* stream) {
   if (N <= 0) return 0;
   if (D != 128 && D != 256) return bad("kv_k_encode: head dim 128 or 256");
-  if (D == 256)
-    return launched(k_encode256_launch(src, src_rs, src2, src2_rs, static_cast<const long long*>(sidx),
-                                       static_cast<const long long*>(dslot), N, Hkv, static_cast<const float*>(qs),
-                                       static_cast<const float*>(lz), NQ, qsc, static_cast<uint8_t*>(pool), ident,
-                                       static_cast<const int*>(kfix), f8 & 1, static_cast<hipStream_t>(stream)), "kv_k_encode");
-  return launched(k_encode_launch(src, src_rs, src2, src2_rs, static_cast<const long long*>(sidx),
+  return launched(k_encode_launch(D, src, src_rs, src2, src2_rs, static_cast<const long long*>(sidx),
                                   static_cast<const long long*>(dslot), N, Hkv, static_cast<const float*>(qs),
                                   static_cast<const float*>(lz), NQ, qsc, static_cast<uint8_t*>(pool), ident,
                                   static_cast<const int*>(kfix), f8 & 1, static_cast<hipStream_t>(stream)), "kv_k_encode");

@@ -1,5 +1,6 @@
 // Launcher prototypes shared by the translation units of libflagrot_kivi.so (f8: FP8-meta pages).  The plain names are
-// the 128-d kernels (kivi_write.hip, kivi_decode.hip), the *256 ones the 256-d kernels (kivi_wide.hip).
+// the 128-d kernels (kivi_write.hip, kivi_decode.hip), the *256 ones the 256-d kernels (kivi_wide.hip); the key group
+// encoder (kivi_kenc.hip) takes the head dim.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -8,7 +9,7 @@ namespace frkv {
 
 int v_write_launch(const void* kv, long long kv_rs, int n, int Hkv, const long long* slots, const float* co, uint8_t* pool,
                    const float* M, int ident, const int* vfix, int f8, hipStream_t st);
-int k_encode_launch(const void* src, long long src_rs, const void* src2, long long src2_rs, const long long* sidx,
+int k_encode_launch(int D, const void* src, long long src_rs, const void* src2, long long src2_rs, const long long* sidx,
                     const long long* dslot, int N, int Hkv, const float* qs, const float* lz, int NQ, float qsc,
                     uint8_t* pool, int ident, const int* kfix, int f8, hipStream_t st);
 int dequant_launch(const uint8_t* pool, const int* bt, int g0, int g1, int nvalid, int Hkv, int fp32, void* ok, void* ov,
@@ -24,9 +25,6 @@ int attn_splits_launch(int G, const void* q, long long q_rs, const void* pool, c
 
 int v_write256_launch(const void* kv, long long kv_rs, int n, int Hkv, const long long* slots, const float* co, uint8_t* pool,
                       const float* M, int ident, const int* vfix, int f8, hipStream_t st);
-int k_encode256_launch(const void* src, long long src_rs, const void* src2, long long src2_rs, const long long* sidx,
-                       const long long* dslot, int N, int Hkv, const float* qs, const float* lz, int NQ, float qsc,
-                       uint8_t* pool, int ident, const int* kfix, int f8, hipStream_t st);
 int dequant256_launch(const uint8_t* pool, const int* bt, int g0, int g1, int nvalid, int Hkv, int fp32, void* ok, void* ov,
                       int f8, hipStream_t st);
 // splits and merge in one call: out bf16 rows of Hkv G 256 values

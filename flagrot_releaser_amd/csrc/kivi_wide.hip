@@ -1,6 +1,6 @@
-// KIVI-style FlagRot INT2 pages at head dim 256 for gfx950: value writer, key group encoder, page dequantiser and the
-// decode attention with its split merge (integrations/vllm_flagrot/csrc/kivi.cu:163-328 k_v_write<256>, :343-663
-// k_k_encode<256>, :2067-2300 the dequantisers, :1997-2036 the 256-d attention launches).  Compiled with
+// KIVI-style FlagRot INT2 pages at head dim 256 for gfx950: value writer, page dequantiser and the decode attention
+// with its split merge (integrations/vllm_flagrot/csrc/kivi.cu:163-328 k_v_write<256>, :2067-2300 the dequantisers,
+// :1997-2036 the 256-d attention launches); the key group encoder is in kivi_kenc.hip.  Compiled with
 // -ffp-contract=off like the 128-d writers: the quantiser rounds every operation on its own.
 //
 // Page chunk per (16-token page, KV head), D = 256, NV = 8 sub-vectors (kivi.cu:15-35):
@@ -125,21 +125,6 @@ __global__ void __launch_bounds__(256) k_v_write256(const uint16_t* __restrict__
   }
 }
 
-// ------------------------------------------------------------------------------------------------ key group encoder
-constexpr int LD2 = 260;                                  // padded row of 256 floats
-constexpr int QT2 = 8;                                    // calibration queries per tile
-struct KEnc2 {
-  float xs[32][LD2];
-  float es[3][32][LD2];
-  float qt[QT2][LD2];
-  float lzt[QT2];
-  float par[3][2][D2];                                    // per candidate (min, scale) per channel
-  float red[4][20];
-  int valid[32];
-  int choice[9];                                          // sub-vectors 0..7: H32; [8]: whole head
-  float ef;
-};
-
 DEVI void lds_row(const float* row, int l32, float (&x)[2][4]) {
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -150,203 +135,6 @@ DEVI void lds_row(const float* row, int l32, float (&x)[2][4]) {
 DEVI void lds_put(float* row, int l32, const float (&x)[2][4]) {
 #pragma unroll
   for (int s = 0; s < 2; ++s) *reinterpret_cast<float4*>(row + 128 * s + 4 * l32) = make_float4(x[s][0], x[s][1], x[s][2], x[s][3]);
-}
-
-template <bool F8>
-__global__ void __launch_bounds__(256) k_k_encode256(const uint16_t* __restrict__ src, long long src_rs,
-                                                     const uint16_t* __restrict__ src2, long long src2_rs,
-                                                     const long long* __restrict__ sidx, const long long* __restrict__ dslot,
-                                                     int Hkv, const float* __restrict__ qs, const float* __restrict__ lz,
-                                                     int NQ, float qsc, uint8_t* __restrict__ pool, int ident,
-                                                     const int* __restrict__ kfix) {
-  extern __shared__ __align__(16) uint8_t lds[];
-  KEnc2& S = *reinterpret_cast<KEnc2*>(lds);
-  const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, hw = tid >> 5, l32 = tid & 31;
-  const long long* si = sidx + static_cast<long long>(item) * 32;
-  const long long* ds = dslot + static_cast<long long>(item) * 32;
-  if (ds[0] < 0) return;
-  if (tid < 32) S.valid[tid] = si[tid] != -1;
-  __syncthreads();
-  for (int e = tid; e < 32 * D2; e += 256) {
-    const int t = e >> 8, c = e & 255;
-    const long long r = si[t];
-    float v = 0.f;
-    if (r >= 0) v = bf16_lo(src[r * src_rs + h * D2 + c]);
-    else if (r <= -2) v = bf16_lo(src2[(-r - 2) * src2_rs + h * D2 + c]);
-    S.xs[t][c] = v;
-  }
-  __syncthreads();
-  // candidates in their bases: one half wave per token
-  for (int t = hw; t < 32; t += 8) {
-    float xv[2][4];
-    lds_row(S.xs[t], l32, xv);
-    lds_put(S.es[0][t], l32, xv);
-    float y[2][4];
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) y[s][i] = xv[s][i];
-    to_basis2<1>(y, l32);
-    lds_put(S.es[1][t], l32, y);
-    to_basis2<2>(xv, l32);
-    lds_put(S.es[2][t], l32, xv);
-  }
-  __syncthreads();
-  // per (candidate, channel): range over the valid tokens, parameters, reconstruction in place
-  for (int e = tid; e < 3 * D2; e += 256) {
-    const int c = e >> 8, ch = e & 255;
-    float mn = INFINITY, mx = -INFINITY;
-    for (int t = 0; t < 32; ++t)
-      if (S.valid[t]) { const float v = S.es[c][t][ch]; mn = fminf(mn, v); mx = fmaxf(mx, v); }
-    float s = kv_scale(mn, mx);
-    kv_params<F8>(mn, s);
-    S.par[c][0][ch] = mn; S.par[c][1][ch] = s;
-    for (int t = 0; t < 32; ++t)
-      if (S.valid[t]) S.es[c][t][ch] = kv_rec(kv_code(S.es[c][t][ch], mn, s), mn, s);
-  }
-  __syncthreads();
-  if (ident) {
-    if (tid < 9) S.choice[tid] = 0;
-  } else if (kfix != nullptr) {
-    if (tid < 9) S.choice[tid] = tid < 8 ? (kfix[h] >> tid) & 1 : (kfix[h] >> 16) & 1;
-  } else {
-    // errors e = rec - x in the original basis (0 for tokens outside the group)
-    for (int t = hw; t < 32; t += 8) {
-      float xx[2][4];
-      lds_row(S.xs[t], l32, xx);
-      const bool v = S.valid[t];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        float y[2][4];
-        lds_row(S.es[c][t], l32, y);
-        if (c == 1) to_basis2<1>(y, l32);
-        if (c == 2) to_basis2<2>(y, l32);
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) y[s][i] = v ? y[s][i] - xx[s][i] : 0.f;
-        lds_put(S.es[c][t], l32, y);
-      }
-    }
-    __syncthreads();
-    // thread <-> (token t, query slot qi of the tile)
-    const int t = tid & 31, qi = tid >> 5;
-    const bool tv = S.valid[t];
-    const float* qh = qs + static_cast<long long>(h) * NQ * D2;
-    const float* lzh = lz + static_cast<long long>(h) * NQ;
-    for (int pass = 0; pass < 2; ++pass) {
-      float acc[18];                                      // [0..7] identity, [8..15] H32 per sub-vector, [16] whole, [17] base
-#pragma unroll
-      for (int k = 0; k < 18; ++k) acc[k] = 0.f;
-      for (int q0 = 0; q0 < NQ; q0 += QT2) {
-        __syncthreads();
-        for (int e = tid; e < QT2 * D2; e += 256) {
-          const int qq = e >> 8, c = e & 255;
-          S.qt[qq][c] = q0 + qq < NQ ? qh[static_cast<long long>(q0 + qq) * D2 + c] : 0.f;
-        }
-        if (tid < QT2) S.lzt[tid] = q0 + tid < NQ ? lzh[q0 + tid] : 0.f;
-        __syncthreads();
-        float lg = 0.f;
-        for (int c = 0; c < D2; ++c) lg += S.xs[t][c] * S.qt[qi][c];
-        const float w = (tv && q0 + qi < NQ) ? fminf(expf(qsc * lg - S.lzt[qi]), 1.f) : 0.f;
-        if (pass == 0) {
-          float pf = 0.f;
-#pragma unroll
-          for (int j = 0; j < NV2; ++j) {
-            float p0 = 0.f, p1 = 0.f;
-            for (int c = 32 * j; c < 32 * j + 32; ++c) {
-              const float qv = S.qt[qi][c];
-              p0 += S.es[0][t][c] * qv; p1 += S.es[1][t][c] * qv; pf += S.es[2][t][c] * qv;
-            }
-            acc[j] += w * p0 * p0; acc[8 + j] += w * p1 * p1;
-          }
-          acc[16] += w * pf * pf;
-        } else {
-          float pb = 0.f;
-          for (int c = 0; c < D2; ++c) pb += S.es[0][t][c] * S.qt[qi][c];
-          acc[17] += w * pb * pb;
-        }
-      }
-      // block reduction: half waves by exchange, then the four wavefronts in order
-#pragma unroll
-      for (int k = 0; k < 18; ++k) {
-#pragma unroll
-        for (int m = 1; m < 32; m <<= 1) acc[k] += hx(acc[k], m);
-        acc[k] += __shfl_xor(acc[k], 32, 64);
-      }
-      __syncthreads();
-      if ((tid & 63) == 0)
-#pragma unroll
-        for (int k = 0; k < 18; ++k) S.red[tid >> 6][k] = acc[k];
-      __syncthreads();
-      if (pass == 0) {
-        if (tid < 8) {
-          const float a = ((S.red[0][tid] + S.red[1][tid]) + S.red[2][tid]) + S.red[3][tid];
-          const float b = ((S.red[0][8 + tid] + S.red[1][8 + tid]) + S.red[2][8 + tid]) + S.red[3][8 + tid];
-          S.choice[tid] = b < a ? 1 : 0;                          // identity on ties
-        }
-        if (tid == 32) S.ef = ((S.red[0][16] + S.red[1][16]) + S.red[2][16]) + S.red[3][16];
-        __syncthreads();
-        for (int e = tid; e < 32 * D2; e += 256) {                // errors of the chosen sub-vector candidates
-          const int tt = e >> 8, c = e & 255;
-          if (S.choice[c >> 5]) S.es[0][tt][c] = S.es[1][tt][c];
-        }
-      } else if (tid == 0) {
-        const float b = ((S.red[0][17] + S.red[1][17]) + S.red[2][17]) + S.red[3][17];
-        S.choice[8] = S.ef < b ? 1 : 0;                           // base on ties
-      }
-    }
-  }
-  __syncthreads();
-  const bool useF = S.choice[8] != 0;
-  // codes of the valid tokens in the chosen bases
-  for (int t = hw; t < 32; t += 8) {
-    if (!S.valid[t]) continue;
-    float yi[2][4], yh[2][4], yf[2][4];
-    lds_row(S.xs[t], l32, yi);
-    lds_row(S.xs[t], l32, yh);
-    lds_row(S.xs[t], l32, yf);
-    to_basis2<1>(yh, l32);
-    to_basis2<2>(yf, l32);
-    const long long slot = ds[t];
-    uint8_t* chunk = pool + ((slot / 16) * Hkv + h) * CHUNK2<F8>;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int cand = useF ? 2 : S.choice[4 * s + (l32 >> 3)];
-      uint32_t word = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = 128 * s + 4 * l32 + i;
-        const float y = cand == 0 ? yi[s][i] : cand == 1 ? yh[s][i] : yf[s][i];
-        const int ci = c & 15;
-        word |= static_cast<uint32_t>(kv_code(y, S.par[cand][0][c], S.par[cand][1][c]) & 3) << (2 * (ci >> 1) + 16 * (ci & 1));
-      }
-      word |= __shfl_xor(word, 1, 32);
-      word |= __shfl_xor(word, 2, 32);
-      if ((l32 & 3) == 0) reinterpret_cast<uint32_t*>(chunk + (slot % 16) * 64)[8 * s + (l32 >> 2)] = word;
-    }
-  }
-  // meta of all 32 cells: cell i holds channels [8 i, 8 i + 8)
-  {
-    const int c = tid;
-    const int cand = useF ? 2 : S.choice[c >> 5];
-    const long long slot = ds[c >> 3];
-    if (slot >= 0) {
-      uint8_t* chunk = pool + ((slot / 16) * Hkv + h) * CHUNK2<F8>;
-      if (F8) {                                                     // flags at slot 0 of cells 0 .. 8
-        const bool neg = (c & 7) == 0 && (c < 64 ? (!useF && S.choice[c >> 3] != 0) : (c == 64 ? useF : false));
-        uint8_t* at = chunk + KM2 + (slot % 16) * 16 + 2 * (c & 7);
-        uint32_t sb = e4m3_bits(S.par[cand][1][c]) | (neg ? 0x80u : 0u);
-        if ((c & 7) == 7) sb |= at[0] & 0x80u;                      // the value row's whole-head flag lives here
-        *reinterpret_cast<uint16_t*>(at) = static_cast<uint16_t>(sb | (e4m3_bits(S.par[cand][0][c]) << 8));
-      } else {
-        uint32_t sb = f16_bits_rn(S.par[cand][1][c]) & 0x7FFFu;
-        const bool neg = c < 8 ? (!useF && S.choice[c] != 0) : (c == 8 ? useF : false);
-        if (neg) sb |= 0x8000u;
-        reinterpret_cast<uint32_t*>(chunk + KM2 + (slot % 16) * 32)[c & 7] = sb | (f16_bits_rn(S.par[cand][0][c]) << 16);
-      }
-    }
-  }
 }
 
 // ------------------------------------------------------------------------------------------------ dequantiser
@@ -662,20 +450,6 @@ int v_write256_launch(const void* kv, long long kv_rs, int n, int Hkv, const lon
                          : (f8 ? k_v_write256<true, false> : k_v_write256<false, false>);
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((items + 7) / 8)), dim3(256), 0, st, static_cast<const uint16_t*>(kv),
                      kv_rs, n, Hkv, slots, co, M, pool, ident, vfix);
-  return hipPeekAtLastError() == hipSuccess ? 0 : 1;
-}
-
-int k_encode256_launch(const void* src, long long src_rs, const void* src2, long long src2_rs, const long long* sidx,
-                       const long long* dslot, int N, int Hkv, const float* qs, const float* lz, int NQ, float qsc,
-                       uint8_t* pool, int ident, const int* kfix, int f8, hipStream_t st) {
-  static bool attr = false;
-  if (!attr) {
-    if (!carve(&k_k_encode256<false>, sizeof(KEnc2)) || !carve(&k_k_encode256<true>, sizeof(KEnc2))) return 1;
-    attr = true;
-  }
-  const auto kern = f8 ? k_k_encode256<true> : k_k_encode256<false>;
-  hipLaunchKernelGGL(kern, dim3(N, Hkv), dim3(256), sizeof(KEnc2), st, static_cast<const uint16_t*>(src), src_rs,
-                     static_cast<const uint16_t*>(src2), src2_rs, sidx, dslot, Hkv, qs, lz, NQ, qsc, pool, ident, kfix);
   return hipPeekAtLastError() == hipSuccess ? 0 : 1;
 }
 

@@ -1,5 +1,5 @@
-// KIVI-style FlagRot INT2 pages for gfx950: per-token value writer, per-(32-token group, KV head) key encoder,
-// page dequantiser and the bf16 LSE merge.  Compiled with -ffp-contract=off: the quantiser (scale, codes,
+// KIVI-style FlagRot INT2 pages for gfx950: per-token value writer, page dequantiser and the bf16 LSE merge (the key
+// group encoder is in kivi_kenc.hip).  Compiled with -ffp-contract=off: the quantiser (scale, codes,
 // reconstruction) rounds every operation on its own, as the reference's (integrations/vllm_flagrot/csrc/kivi.cu:94-125).
 //
 // Page chunk per (16-token page, KV head), D = 128: KC @0 [16][32] key codes (32-bit words of 16 channels, channel i at
@@ -79,202 +79,6 @@ __global__ void __launch_bounds__(256) k_v_write(const uint16_t* __restrict__ kv
       uint8_t* kb = chunk + 512 + off * 8 + 6;
       *kb = static_cast<uint8_t>((*kb & 0x7Fu) | (pk.whole ? 0x80u : 0u));
     } else chunk[1536 + off] = pk.whole ? 1 : 0;
-  }
-}
-
-// ------------------------------------------------------------------------------------------------ key group encoder
-constexpr int LD = 132;                                   // padded row of 128 floats
-constexpr int QT = 8;                                     // calibration queries per tile
-struct KEnc {
-  float xs[32][LD];
-  float es[3][32][LD];
-  float qt[QT][LD];
-  float lzt[QT];
-  float par[3][2][128];                                   // per candidate (min, scale) per channel
-  float red[4][12];
-  int valid[32];
-  int choice[5];
-  float ef;
-};
-
-template <bool F8>
-__global__ void __launch_bounds__(256) k_k_encode(const uint16_t* __restrict__ src, long long src_rs,
-                                                  const uint16_t* __restrict__ src2, long long src2_rs,
-                                                  const long long* __restrict__ sidx, const long long* __restrict__ dslot,
-                                                  int Hkv, const float* __restrict__ qs, const float* __restrict__ lz,
-                                                  int NQ, float qsc, uint8_t* __restrict__ pool, int ident,
-                                                  const int* __restrict__ kfix) {
-  extern __shared__ __align__(16) uint8_t lds[];
-  KEnc& S = *reinterpret_cast<KEnc*>(lds);
-  const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, hw = tid >> 5, l32 = tid & 31;
-  const long long* si = sidx + static_cast<long long>(item) * 32;
-  const long long* ds = dslot + static_cast<long long>(item) * 32;
-  if (ds[0] < 0) return;
-  if (tid < 32) S.valid[tid] = si[tid] != -1;
-  __syncthreads();
-  for (int e = tid; e < 32 * 128; e += 256) {
-    const int t = e >> 7, c = e & 127;
-    const long long r = si[t];
-    float v = 0.f;
-    if (r >= 0) v = bf16_lo(src[r * src_rs + h * 128 + c]);
-    else if (r <= -2) v = bf16_lo(src2[(-r - 2) * src2_rs + h * 128 + c]);
-    S.xs[t][c] = v;
-  }
-  __syncthreads();
-  // candidates in their bases: one half wave per token
-  for (int t = hw; t < 32; t += 8) {
-    const float4 xv = *reinterpret_cast<const float4*>(&S.xs[t][4 * l32]);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      float y[4] = {xv.x, xv.y, xv.z, xv.w};
-      if (c == 1) fwht<32>(y, l32);
-      if (c == 2) fwht<128>(y, l32);
-      *reinterpret_cast<float4*>(&S.es[c][t][4 * l32]) = make_float4(y[0], y[1], y[2], y[3]);
-    }
-  }
-  __syncthreads();
-  // per (candidate, channel): range over the valid tokens, parameters, reconstruction in place
-  for (int e = tid; e < 3 * 128; e += 256) {
-    const int c = e >> 7, ch = e & 127;
-    float mn = INFINITY, mx = -INFINITY;
-    for (int t = 0; t < 32; ++t)
-      if (S.valid[t]) { const float v = S.es[c][t][ch]; mn = fminf(mn, v); mx = fmaxf(mx, v); }
-    float s = kv_scale(mn, mx);
-    kv_params<F8>(mn, s);
-    S.par[c][0][ch] = mn; S.par[c][1][ch] = s;
-    for (int t = 0; t < 32; ++t)
-      if (S.valid[t]) S.es[c][t][ch] = kv_rec(kv_code(S.es[c][t][ch], mn, s), mn, s);
-  }
-  __syncthreads();
-  if (ident) {
-    if (tid < 5) S.choice[tid] = 0;
-  } else if (kfix != nullptr) {
-    if (tid < 5) S.choice[tid] = tid < 4 ? (kfix[h] >> tid) & 1 : (kfix[h] >> 16) & 1;
-  } else {
-    // errors e = rec - x in the original basis (0 for tokens outside the group)
-    for (int t = hw; t < 32; t += 8) {
-      const float4 xv = *reinterpret_cast<const float4*>(&S.xs[t][4 * l32]);
-      const float xx[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const float4 yv = *reinterpret_cast<const float4*>(&S.es[c][t][4 * l32]);
-        float y[4] = {yv.x, yv.y, yv.z, yv.w};
-        if (c == 1) fwht<32>(y, l32);
-        if (c == 2) fwht<128>(y, l32);
-        const bool v = S.valid[t];
-        *reinterpret_cast<float4*>(&S.es[c][t][4 * l32]) =
-            make_float4(v ? y[0] - xx[0] : 0.f, v ? y[1] - xx[1] : 0.f, v ? y[2] - xx[2] : 0.f, v ? y[3] - xx[3] : 0.f);
-      }
-    }
-    __syncthreads();
-    // thread <-> (token t, query slot qi of the tile)
-    const int t = tid & 31, qi = tid >> 5;
-    const bool tv = S.valid[t];
-    const float* qh = qs + static_cast<long long>(h) * NQ * 128;
-    const float* lzh = lz + static_cast<long long>(h) * NQ;
-    for (int pass = 0; pass < 2; ++pass) {
-      float accI[4] = {0.f, 0.f, 0.f, 0.f}, accH[4] = {0.f, 0.f, 0.f, 0.f}, accF = 0.f, accB = 0.f;
-      for (int q0 = 0; q0 < NQ; q0 += QT) {
-        __syncthreads();
-        for (int e = tid; e < QT * 128; e += 256) {
-          const int qq = e >> 7, c = e & 127;
-          S.qt[qq][c] = q0 + qq < NQ ? qh[static_cast<long long>(q0 + qq) * 128 + c] : 0.f;
-        }
-        if (tid < QT) S.lzt[tid] = q0 + tid < NQ ? lzh[q0 + tid] : 0.f;
-        __syncthreads();
-        float lg = 0.f;
-        for (int c = 0; c < 128; ++c) lg += S.xs[t][c] * S.qt[qi][c];
-        const float w = (tv && q0 + qi < NQ) ? fminf(expf(qsc * lg - S.lzt[qi]), 1.f) : 0.f;
-        if (pass == 0) {
-          float pf = 0.f;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            float p0 = 0.f, p1 = 0.f;
-            for (int c = 32 * j; c < 32 * j + 32; ++c) {
-              const float qv = S.qt[qi][c];
-              p0 += S.es[0][t][c] * qv; p1 += S.es[1][t][c] * qv; pf += S.es[2][t][c] * qv;
-            }
-            accI[j] += w * p0 * p0; accH[j] += w * p1 * p1;
-          }
-          accF += w * pf * pf;
-        } else {
-          float pb = 0.f;
-          for (int c = 0; c < 128; ++c) pb += S.es[0][t][c] * S.qt[qi][c];
-          accB += w * pb * pb;
-        }
-      }
-      // block reduction: half waves by exchange, then the four wavefronts in order
-      float v[10] = {accI[0], accI[1], accI[2], accI[3], accH[0], accH[1], accH[2], accH[3], accF, accB};
-#pragma unroll
-      for (int k = 0; k < 10; ++k) {
-#pragma unroll
-        for (int m = 1; m < 32; m <<= 1) v[k] += hx(v[k], m);
-        v[k] += __shfl_xor(v[k], 32, 64);
-      }
-      __syncthreads();
-      if ((tid & 63) == 0)
-        for (int k = 0; k < 10; ++k) S.red[tid >> 6][k] = v[k];
-      __syncthreads();
-      if (pass == 0) {
-        if (tid < 4) {
-          const float a = ((S.red[0][tid] + S.red[1][tid]) + S.red[2][tid]) + S.red[3][tid];
-          const float b = ((S.red[0][4 + tid] + S.red[1][4 + tid]) + S.red[2][4 + tid]) + S.red[3][4 + tid];
-          S.choice[tid] = b < a ? 1 : 0;                          // identity on ties
-        }
-        if (tid == 32) S.ef = ((S.red[0][8] + S.red[1][8]) + S.red[2][8]) + S.red[3][8];
-        __syncthreads();
-        for (int e = tid; e < 32 * 128; e += 256) {               // errors of the chosen sub-vector candidates
-          const int tt = e >> 7, c = e & 127;
-          if (S.choice[c >> 5]) S.es[0][tt][c] = S.es[1][tt][c];
-        }
-      } else if (tid == 0) {
-        const float b = ((S.red[0][9] + S.red[1][9]) + S.red[2][9]) + S.red[3][9];
-        S.choice[4] = S.ef < b ? 1 : 0;                           // base on ties
-      }
-    }
-  }
-  __syncthreads();
-  const bool useF = S.choice[4] != 0;
-  // codes of the valid tokens in the chosen bases
-  for (int t = hw; t < 32; t += 8) {
-    if (!S.valid[t]) continue;
-    const float4 xv = *reinterpret_cast<const float4*>(&S.xs[t][4 * l32]);
-    float yi[4] = {xv.x, xv.y, xv.z, xv.w}, yh[4] = {xv.x, xv.y, xv.z, xv.w}, yf[4] = {xv.x, xv.y, xv.z, xv.w};
-    fwht<32>(yh, l32);
-    fwht<128>(yf, l32);
-    const int cand = useF ? 2 : S.choice[l32 >> 3];
-    uint32_t word = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = 4 * l32 + i;
-      const float y = cand == 0 ? yi[i] : cand == 1 ? yh[i] : yf[i];
-      const int ci = c & 15;
-      word |= static_cast<uint32_t>(kv_code(y, S.par[cand][0][c], S.par[cand][1][c]) & 3) << (2 * (ci >> 1) + 16 * (ci & 1));
-    }
-    word |= __shfl_xor(word, 1, 32);
-    word |= __shfl_xor(word, 2, 32);
-    const long long slot = ds[t];
-    uint8_t* chunk = pool + ((slot / 16) * Hkv + h) * CHUNK<F8>;
-    if ((l32 & 3) == 0) reinterpret_cast<uint32_t*>(chunk + (slot % 16) * 32)[l32 >> 2] = word;
-  }
-  // meta of all 32 cells: cell i holds channels [4 i, 4 i + 4)
-  for (int c = tid; c < 128; c += 256) {
-    const int cand = useF ? 2 : S.choice[c >> 5];
-    const long long slot = ds[c >> 2];
-    if (slot < 0) continue;
-    uint8_t* chunk = pool + ((slot / 16) * Hkv + h) * CHUNK<F8>;
-    if (F8) {                                                     // flags at slot 0 of cells 0 .. 4
-      const bool neg = (c & 3) == 0 && (c < 16 ? (!useF && S.choice[c >> 2] != 0) : (c == 16 ? useF : false));
-      uint8_t* at = chunk + 512 + (slot % 16) * 8 + 2 * (c & 3);
-      uint32_t sb = e4m3_bits(S.par[cand][1][c]) | (neg ? 0x80u : 0u);
-      if ((c & 3) == 3) sb |= at[0] & 0x80u;                      // the value row's whole-head flag lives here
-      *reinterpret_cast<uint16_t*>(at) = static_cast<uint16_t>(sb | (e4m3_bits(S.par[cand][0][c]) << 8));
-    } else {
-      uint32_t sb = f16_bits_rn(S.par[cand][1][c]) & 0x7FFFu;
-      const bool neg = c < 4 ? (!useF && S.choice[c] != 0) : (c == 4 ? useF : false);
-      if (neg) sb |= 0x8000u;
-      reinterpret_cast<uint32_t*>(chunk + 512 + (slot % 16) * 16)[c & 3] = sb | (f16_bits_rn(S.par[cand][0][c]) << 16);
-    }
   }
 }
 
@@ -409,23 +213,6 @@ int v_write_launch(const void* kv, long long kv_rs, int n, int Hkv, const long l
   const auto kern = wmat ? (f8 ? k_v_write<true, true> : k_v_write<false, true>) : (f8 ? k_v_write<true, false> : k_v_write<false, false>);
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((items + 7) / 8)), dim3(256), 0, st,
                      static_cast<const uint16_t*>(kv), kv_rs, n, Hkv, slots, co, M, pool, ident, vfix);
-  return hipPeekAtLastError() == hipSuccess ? 0 : 1;
-}
-
-int k_encode_launch(const void* src, long long src_rs, const void* src2, long long src2_rs, const long long* sidx,
-                    const long long* dslot, int N, int Hkv, const float* qs, const float* lz, int NQ, float qsc,
-                    uint8_t* pool, int ident, const int* kfix, int f8, hipStream_t st) {
-  static bool attr = false;
-  if (!attr) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_k_encode<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(sizeof(KEnc))) != hipSuccess) return 1;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_k_encode<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(sizeof(KEnc))) != hipSuccess) return 1;
-    attr = true;
-  }
-  const auto kern = f8 ? k_k_encode<true> : k_k_encode<false>;
-  hipLaunchKernelGGL(kern, dim3(N, Hkv), dim3(256), sizeof(KEnc), st, static_cast<const uint16_t*>(src), src_rs,
-                     static_cast<const uint16_t*>(src2), src2_rs, sidx, dslot, Hkv, qs, lz, NQ, qsc, pool, ident, kfix);
   return hipPeekAtLastError() == hipSuccess ? 0 : 1;
 }
 
