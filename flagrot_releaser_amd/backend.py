@@ -147,15 +147,6 @@ class RingGeometry:
             return p
         return S + (p - S) % W if W > 0 else -1
 
-    def kept(self, n: int, device):
-        """positions of an n-token prompt that stay in BF16 (sinks and the newest W), and their slots"""
-        pos = torch.arange(n, device=device)
-        keep = pos < self.S
-        if self.W > 0:
-            keep = keep | (pos >= n - self.W)
-        pos = pos[keep]
-        return keep, self.slot(pos)
-
     def paged_tokens(self, L, out=None):
         """tokens of a length-L sequence that decode reads from pages: [S, L - W) with the sinks masked by kv_start,
         nothing while the sequence still fits the BF16 rows"""
@@ -335,26 +326,21 @@ class DecodeLayer:
 
     def prefill(self, kv, slots, req: int):
         """a prompt of request row `req`: every token to its page; sinks and the newest W tokens also to the BF16 row"""
-        self.write_pages(kv, slots)
-        if self.ring is not None:
-            keep, where = self.geo.kept(kv.shape[0], kv.device)
-            self.ring[req].index_copy_(0, where, self.center_rows(kv[keep]))
+        self.prefill_chunk(kv, slots, req, 0)
 
     def prefill_chunk(self, kv, slots, req: int, start: int):
         """the next n tokens of request row `req`'s prompt, positions [start, start + n): every token to its page; the
         sinks among them and the newest W of the prompt so far also to the BF16 row"""
         self.write_pages(kv, slots)
         if self.ring is not None:
-            n = kv.shape[0]
-            pos = start + torch.arange(n, device=kv.device)
-            keep = (pos < self.geo.S) | (pos >= start + n - self.geo.W)
-            self.ring[req].index_copy_(0, self.geo.slot(pos[keep]), self.center_rows(kv[keep]))
+            K.ring_rows(kv, self.ring, kmu=self.kmu, base=int(req) * self.geo.slots, sink=self.geo.S, window=self.geo.W,
+                        start=start)
 
     def update(self, kv, sp: StepPlan):
         """cache update of a decode step: the new tokens to their pages and to their BF16 slots"""
         self.write_pages(kv, sp.slots)
         if self.ring is not None:
-            self.ring.view(-1, 2 * self.Hkv, D).index_copy_(0, sp.ring_dest, self.center_rows(kv))
+            K.ring_rows(kv, self.ring, kmu=self.kmu, dest=sp.ring_dest)
 
     def decode(self, q, sp: StepPlan, out):
         n = q.shape[0]
@@ -396,20 +382,24 @@ class KiviDecodeLayer:
         dev = pool.device
         self.ring = torch.zeros((planner.spare + 1) * self.geo.slots, 2 * Hkv, D, dtype=torch.bfloat16, device=dev)
         self.ws = kivi_workspace(dev, planner.max_rows, Hkv, G, D, planner.plan)
+        self._rows = None                                  # made by the first prompt, for prompts up to max_len
 
     def prefill(self, kv, slots, req: int):
         """a fresh prompt of n tokens: values of every token, the whole key groups, sinks and newest W rows in BF16"""
         n = kv.shape[0]
         KIVI.v_write(kv, slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
-        keep, where = self.geo.kept(n, kv.device)
-        row = self.ring.view(self.planner.spare + 1, self.geo.slots, 2 * self.Hkv, D)[req]
-        row.index_copy_(0, where, kv[keep])
+        K.ring_rows(kv, self.ring, base=int(req) * self.geo.slots, sink=self.geo.S, window=self.geo.W)
         whole = n // GROUP
         if whole:
-            pos = torch.arange(whole * GROUP, device=kv.device).view(whole, GROUP)
-            src = torch.where(pos < self.geo.S, torch.full_like(pos, -1), pos).contiguous()     # sinks stay BF16 only
-            KIVI.k_encode(kv, src, slots[:whole * GROUP].view(whole, GROUP).contiguous(), self.qs, self.lz, self.scale,
-                          self.pool, self.Hkv, D, f8=self.f8)
+            KIVI.k_encode(kv, self._prompt_rows(whole), slots[:whole * GROUP].view(whole, GROUP).contiguous(), self.qs,
+                          self.lz, self.scale, self.pool, self.Hkv, D, f8=self.f8)
+
+    def _prompt_rows(self, groups: int):
+        """row of every token of the leading groups of a prompt, -1 for the sinks (they stay BF16 only)"""
+        if self._rows is None or self._rows.shape[0] < groups:
+            pos = torch.arange(max(groups, -(-self.planner.max_len // GROUP)) * GROUP, device=self.pool.device)
+            self._rows = pos.masked_fill_(pos < self.geo.S, -1).view(-1, GROUP)
+        return self._rows[:groups]
 
     def prefill_chunk(self, kv, slots, req: int, start: int, table_row):
         """the next n tokens of request `req`'s prompt, positions [start, start + n): values of every token, the key
@@ -422,13 +412,11 @@ class KiviDecodeLayer:
         if groups is not None:
             KIVI.k_encode(kv, groups[0], groups[1], self.qs, self.lz, self.scale, self.pool, self.Hkv, D, src2=flat,
                           f8=self.f8)
-        pos = start + torch.arange(n, device=kv.device)
-        keep = (pos < self.geo.S) | (pos >= start + n - self.geo.W)
-        flat.index_copy_(0, req * self.geo.slots + self.geo.slot(pos[keep]), kv[keep])
+        K.ring_rows(kv, self.ring, base=int(req) * self.geo.slots, sink=self.geo.S, window=self.geo.W, start=start)
 
     def update(self, kv, sp: StepPlan):
         KIVI.v_write(kv, sp.slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
-        self.ring.index_copy_(0, sp.ring_dest, kv)
+        K.ring_rows(kv, self.ring, dest=sp.ring_dest)
         KIVI.k_encode(self.ring, sp.group_src, sp.group_dst, self.qs, self.lz, self.scale, self.pool, self.Hkv, D,
                       f8=self.f8)
 

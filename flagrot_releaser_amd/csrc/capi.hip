@@ -193,6 +193,23 @@ int fr_v2_write(int fmt, const void* kv, long long kv_ts, const long long* slots
   return launched(static_write_launch(fmt, p, static_cast<hipStream_t>(stream)), "fr_v2_write");
 }
 
+int fr_ring_rows(const void* kv, long long kv_ts, int T, int Hkv, int Dh, const float* kmu, void* ring, const long long* dest,
+                 long long base, int S, int W, int start, void* stream) {
+  if (T <= 0) return 0;
+  if (Dh != 128 && Dh != 256) return fail(-8, "fr_ring_rows: head dim 128 | 256");
+  if (S < 0 || W < 0 || start < 0) return fail(-3, "fr_ring_rows: bad ring geometry");
+  RingRowsParams p{};
+  p.kv = kv; p.kv_ts = kv_ts; p.width = 2 * Hkv * Dh; p.kmu = kmu; p.ring = ring; p.dest = dest; p.base = base;
+  p.S = S; p.W = W; p.start = start;
+  if (dest != nullptr) p.rows = p.sinks = T;
+  else {      // positions below S, and the newest W of the rest
+    p.sinks = start < S ? (S - start < T ? S - start : T) : 0;
+    p.win0 = T - W > p.sinks ? T - W : p.sinks;
+    p.rows = p.sinks + T - p.win0;
+  }
+  return launched(ring_rows_launch(p, static_cast<hipStream_t>(stream)), "fr_ring_rows");
+}
+
 // What the host split planner multiplies by the CU count to get the number of workgroups that run at once.  The answer
 // is 1: the fastest launch shape is ONE large workgroup per CU (decode_launch takes it whenever the plan's workgroups
 // fit the CUs once with >= 1024 tokens each), and a planner that fills "1 x CUs" slots with the longest chunks that

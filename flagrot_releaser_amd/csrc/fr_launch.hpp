@@ -36,6 +36,19 @@ int k2_write_lds_bytes(int hd);
 int head_fwht_launch(const void* x, long long x_ts, void* out, long long o_ts, int T, int H, const uint8_t* flags,
                      float scale, hipStream_t st, int D);
 
+struct RingRowsParams {
+  const void* kv;          // bf16 [T, width], token stride kv_ts
+  long long kv_ts;
+  int width;               // elements of a row: 2 * Hkv * head dim
+  const float* kmu;        // [width / 2] subtracted from the key half, or null
+  void* ring;              // bf16 [*, width]
+  const long long* dest;   // ring row of every token (< 0: skip), or null: the rule below
+  long long base;          // first ring row of the request
+  int S, W, start;         // sinks, window, position of token 0
+  int rows, sinks, win0;   // rows copied: tokens [0, sinks) and [win0, win0 + rows - sinks)
+};
+int ring_rows_launch(const RingRowsParams& p, hipStream_t st);
+
 struct DecodeParams {
   const void* q;
   long long q_bs;

@@ -37,6 +37,7 @@ NOALLOC_MAX_PARTS = 8192     # FR_NOALLOC_MAX_PARTS of include/flagrot_kernels.h
 NATIVE = Library("kernels", "FLAGROT_LIB", "fr_abi_version", ABI, "fr_last_error", {
     "fr_v2_attn": "i p l p p i p i i i i i f p p i i i i i p p p p l p p p l l p i i",
     "fr_v2_write": "i p l p i i i p i p p i p",
+    "fr_ring_rows": "p l i i i p p p l i i i p",
     "fr_v2_occupancy": "i i i i",
     "fr_v2_chunk_bytes": "i i",
     "fr_cb_nsg": "",
@@ -401,6 +402,25 @@ def cb_attn_noalloc(q, pool, block_table, seq_lens, out, nsplit, chunk, qscale, 
             CB_KINDS[kind], out, out.stride(0), *_tail_args(tail, tail_len, tail_idx, tail_bs, tail_ts), current_stream(),
             G, int(kv_start))
     return _decode("fr_cb_attn_noalloc", args, bound)
+
+
+def ring_rows(kv, ring, kmu=None, dest=None, base=0, sink=0, window=0, start=0):
+    """The BF16 rows a request keeps beside its pages: rows kv bf16 [T, 2 Hkv, Dh] into ring, a contiguous bf16 tensor of
+    rows of 2 Hkv Dh elements; kmu fp32 [Hkv, Dh] is subtracted from the keys (FP32, one rounding).  dest int64 [T] names
+    the ring row of every token (negative: skip).  Without it the tokens are positions start .. start + T - 1 of the
+    request whose ring starts at row `base`: positions below `sink` go to their own slot, the newest `window` of the rest
+    to slot sink + (p - sink) % window."""
+    T = kv.shape[0]
+    if T == 0:
+        return
+    assert kv.dtype == torch.bfloat16 and ring.dtype == torch.bfloat16 and ring.is_contiguous()
+    rows, width = _loadable(kv), kv.shape[1] * kv.shape[2]
+    if dest is None:
+        assert (base + sink + window) * width <= ring.numel(), "the request's rows lie outside the ring"
+    else:
+        assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.shape[0] == T
+    NATIVE.run("fr_ring_rows", rows, rows.stride(0), T, kv.shape[1] // 2, kv.shape[2], _centre(kmu, rows), ring, dest,
+               base, sink, window, start, current_stream())
 
 
 def head_fwht(x, flags, scale, out=None):
