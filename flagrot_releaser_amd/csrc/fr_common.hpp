@@ -222,21 +222,28 @@ DEVI void place4(uint32_t c, bool isB, int i, uint32_t& mask, uint32_t& bits) {
   }
 }
 
-// V^T fields of one token by 32-bit atomics (tokens of a page may arrive from different waves): the lane's 4 codes
+// V^T fields of one token by 32-bit atomics (tokens of a page may arrive from different waves): the lane's 4 codes.  The
+// dims dd and dd + 8 share a word of the 2-bit format: the lane of dd takes both (half the atomics, none on one address).
 template <int QM, int P>
 DEVI void store_v_codes(uint8_t* chunk, int pos, const uint32_t (&code)[4], int l32) {
   using L = Lay<QM, P>;
   const int c8 = pos >> 3, ii = (pos & 7) >> 1;
   const bool isB = pos & 1;
+  uint32_t cb[4];
+  if constexpr (QM == QM_ASYM2) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cb[i] = hdown(code[i], 2);
+    if (l32 & 2) return;
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int dd = 4 * l32 + i;
     const int e = ((dd & 63) >> 4) * 8 + (dd & 7);
     if constexpr (QM == QM_ASYM2) {
       uint32_t* wp = reinterpret_cast<uint32_t*>(chunk + L::V_OFF + (e * (P / 8) + c8) * 8 + 4 * (dd >> 6));
-      const int sh = 8 * ii + 4 * ((dd & 15) >> 3) + 2 * (isB ? 1 : 0);
-      atomicAnd(wp, ~(3u << sh));
-      atomicOr(wp, code[i] << sh);
+      const int sh = 8 * ii + 2 * (isB ? 1 : 0);
+      atomicAnd(wp, ~(0x33u << sh));
+      atomicOr(wp, (code[i] | (cb[i] << 4)) << sh);
     } else {
       const int sub = 2 * (dd >> 6) + ((dd & 15) >> 3);
       uint32_t* wp = reinterpret_cast<uint32_t*>(chunk + L::V_OFF + (e * (P / 8) + c8) * 16 + 4 * sub);
