@@ -31,4 +31,86 @@ DEVI float tree32_lanes(float v) {        // the same tree, one element per lane
   return v;
 }
 
+// orthonormal H_D of a row held by the wavefront (D = 256: lane = dims 4 lane + i; D = 128: both half waves hold it)
+template <int D>
+DEVI void head_transform(float (&y)[4], int lane) {
+  if constexpr (D == 128) {
+    fwht<128>(y, lane & 31);
+  } else {
+    butterflies<128>(y, lane & 31);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float o = xor32(y[i]);
+      y[i] = (lane >= 32 ? o - y[i] : y[i] + o) * 0.0625f;
+    }
+  }
+}
+
+// ---- value codes of up to 64 tokens, word by word
+// The eight tokens of an aligned run of slots share V^T words.  `lead` lists the runs that the N tokens (slots in LDS,
+// negative: none) touch: the first slot of the run and, a byte per position, which token holds it (0xFF: none of these).
+template <int N>
+struct VRuns {
+  long long first[N];
+  unsigned long long map[N];
+  int n;
+};
+template <int N>
+DEVI void v_runs(const long long* slot, VRuns<N>& r) {        // called by one whole wavefront; the caller's barrier follows
+  const int lane = threadIdx.x & 63;
+  const long long s = lane < N ? slot[lane] : -1, run = s & ~7LL;
+  unsigned long long map = ~0ull;
+  bool leads = s >= 0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const long long o = slot[j];
+    if (o < 0 || (o & ~7LL) != run) continue;
+    if (j < lane) leads = false;
+    const int b = 8 * static_cast<int>(o & 7);
+    map = (map & ~(0xFFull << b)) | (static_cast<unsigned long long>(j) << b);
+  }
+  const unsigned long long who = __ballot(leads);
+  if (leads) {
+    const int at = __popcll(who & ((1ull << lane) - 1));
+    r.first[at] = run;
+    r.map[at] = map;
+  }
+  if (lane == 0) r.n = __popcll(who);
+}
+// word j of a run: whole if the tokens at hand hold all eight positions, else merged (other tokens may be stored at the
+// same time).  codes[token * stride + dim]
+template <int QM, int P>
+DEVI void store_v_words(uint8_t* chunk, int c8, int j, const uint8_t* codes, int stride, unsigned long long map) {
+  using L = Lay<QM, P>;
+  uint32_t wd = 0, mask = 0;
+  if constexpr (QM == QM_ASYM2) {
+    const int e = j >> 1, m = j & 1, dd = 64 * m + 16 * (e >> 3) + (e & 7);
+#pragma unroll
+    for (int tk = 0; tk < 8; ++tk) {
+      const int at = static_cast<int>(map >> (8 * tk)) & 0xFF, sh = 8 * (tk >> 1) + 2 * (tk & 1);
+      if (at == 0xFF) continue;
+      const uint8_t* c = codes + at * stride + dd;
+      wd |= (static_cast<uint32_t>(c[0]) | (static_cast<uint32_t>(c[8]) << 4)) << sh;
+      mask |= 0x33u << sh;
+    }
+    uint32_t* wp = reinterpret_cast<uint32_t*>(chunk + L::V_OFF + (e * (P / 8) + c8) * 8 + 4 * m);
+    if (mask == ~0u) *wp = wd;
+    else { atomicAnd(wp, ~mask); atomicOr(wp, wd); }
+  } else {
+    const int e = j >> 2, sub = j & 3, dd = 64 * (sub >> 1) + 16 * (e >> 3) + 8 * (sub & 1) + (e & 7);
+#pragma unroll
+    for (int tk = 0; tk < 8; ++tk) {
+      const int at = static_cast<int>(map >> (8 * tk)) & 0xFF;
+      if (at == 0xFF) continue;
+      uint32_t m, b;
+      place4<QM>(codes[at * stride + dd], (tk & 1) != 0, tk >> 1, m, b);
+      wd |= b;
+      mask |= m;
+    }
+    uint32_t* wp = reinterpret_cast<uint32_t*>(chunk + L::V_OFF + (e * (P / 8) + c8) * 16 + 4 * sub);
+    if (mask == ~0u) *wp = wd;
+    else { atomicAnd(wp, ~mask); atomicOr(wp, wd); }
+  }
+}
+
 }  // namespace fr
