@@ -68,11 +68,9 @@ DEVI void butterflies(float (&x)[4], int l32) {
   }
 #pragma unroll
   for (int lm = 1; lm < N / 4; lm <<= 1) {
+    const uint32_t flip = (l32 & lm) ? 0x80000000u : 0u;        // upper lane: other - own, as other + (-own)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float o = hx(x[i], lm);
-      x[i] = (l32 & lm) ? (o - x[i]) : (x[i] + o);
-    }
+    for (int i = 0; i < 4; ++i) x[i] = hx(x[i], lm) + __uint_as_float(__float_as_uint(x[i]) ^ flip);
   }
 }
 template <int N>
@@ -107,15 +105,37 @@ DEVI float gmin8(float a) {
 }
 
 // ---------------------------------------------------------------------------------------------- quantisers
+// n_i = rint of the IEEE quotients y_i / s, where |y_i| <= lim.  The quotient itself is formed only where it matters: q = y r
+// with r the hardware reciprocal (1 ulp) lies within 2^-22 lim r of y / s, and rounding y / s to FP32 first moves it by less
+// than that, so rint(q) is the answer unless some q lies within 2^-21 lim r of a half (then, for huge steps and for anything
+// that is not finite: the division).  5 instructions a quotient instead of 11; writers spent a third of their vector
+// instructions on it.
+template <int N>
+DEVI void rint_quotients(const float (&y)[N], float s, float lim, float (&n)[N]) {
+  const float r = __builtin_amdgcn_rcpf(s);
+  float worst = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float q = y[i] * r;
+    n[i] = rintf(q);
+    worst = fmaxf(worst, fabsf(q - n[i]));
+  }
+  if (!(worst < 0.5f - lim * r * 4.76837158203125e-07f && s < 1e30f)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) n[i] = rintf(y[i] / s);
+  }
+}
 // symmetric INT4: s = fp16(amax * fp32(1/7)), q = clamp(rne(y / s), -7, 7), 0 where s == 0
 DEVI uint32_t quant_sym4(const float (&y)[4], float (&q)[4], float (&deq)[4]) {
   float am = fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3])));
   am = gmax8(am);
   const uint32_t w = f16_bits_rn(am * (1.0f / 7.0f));
   const float s = f16_value(w);
+  float n[4];
+  rint_quotients(y, s != 0.f ? s : 1.f, s != 0.f ? am : 0.f, n);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float v = s != 0.f ? rintf(y[i] / s) : 0.f;
+    float v = s != 0.f ? n[i] : 0.f;
     v = fminf(fmaxf(v, -7.f), 7.f);
     q[i] = v;
     deq[i] = v * s;
@@ -129,32 +149,36 @@ DEVI uint32_t scale_word(float s, uint32_t z) {  // FP16 pattern nearest to RN16
   const int x = min(max(h - static_cast<int>(z) + (1 << (NB - 1)), 0) & ~M, 0x7C00 - (1 << NB));
   return static_cast<uint32_t>(x) + z;
 }
+// step, zero point and codes of the range [mn, mx]: s = max((mx - mn) / (2^NB - 1), 1e-12), z = rne(-mn / s),
+// code = clamp(rne(y / s) + z)
 template <int NB>
-DEVI void asym_params(float mn, float mx, float& s, float& z) {
+DEVI void asym_codes(const float (&y)[4], float mn, float mx, float lim, float& s, float& z, float (&c)[4]) {
   constexpr float inv = 1.0f / static_cast<float>((1 << NB) - 1);
   s = fmaxf((mx - mn) * inv, 1e-12f);
-  z = rintf(-mn / s);
-}
-template <int NB>
-DEVI float asym_code(float y, float s, float z) {
-  return fminf(fmaxf(rintf(y / s) + z, 0.f), static_cast<float>((1 << NB) - 1));
+  const float v[5] = {y[0], y[1], y[2], y[3], -mn};
+  float n[5];
+  rint_quotients(v, s, lim, n);
+  z = n[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c[i] = fminf(fmaxf(n[i] + z, 0.f), static_cast<float>((1 << NB) - 1));
 }
 // asymmetric INT4 / INT2.  q, word: the stored form (range widened to include 0, zero point in the NB low bits of
-// the word).  deq (optional): the error form (FP32 step, unbounded zero point) the selection errors are measured on.
+// the word).  deq (optional): the error form (FP32 step, unbounded zero point) the selection errors are measured on; where
+// every range at hand includes 0 the two have the same codes.
 template <int NB, bool WANT_DEQ>
 DEVI uint32_t quant_asym(const float (&y)[4], float (&q)[4], float (&deq)[4]) {
   float mn = fminf(fminf(y[0], y[1]), fminf(y[2], y[3])), mx = fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3]));
   mn = gmin8(mn);
   mx = gmax8(mx);
+  const float lim = fmaxf(fabsf(mn), fabsf(mx));
   float s, z;
   if (WANT_DEQ) {
-    asym_params<NB>(mn, mx, s, z);
+    asym_codes<NB>(y, mn, mx, lim, s, z, q);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) deq[i] = (asym_code<NB>(y[i], s, z) - z) * s;
+    for (int i = 0; i < 4; ++i) deq[i] = (q[i] - z) * s;
+    if (__all(mn <= 0.f && mx >= 0.f)) return scale_word<NB>(s, static_cast<uint32_t>(z));
   }
-  asym_params<NB>(fminf(mn, 0.f), fmaxf(mx, 0.f), s, z);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) q[i] = asym_code<NB>(y[i], s, z);
+  asym_codes<NB>(y, fminf(mn, 0.f), fmaxf(mx, 0.f), lim, s, z, q);
   return scale_word<NB>(s, static_cast<uint32_t>(z));
 }
 template <int QM, bool WANT_DEQ>

@@ -36,6 +36,23 @@ DEVI int kv_code(float x, float mn, float s) {
   q = fminf(fmaxf(q, 0.f), 3.f);
   return static_cast<int>(rintf(q));
 }
+// the codes of four numbers of one (mn, s).  The IEEE quotient is formed only where it matters: the difference times the
+// hardware reciprocal (1 ulp) is off by less than 2^-20 inside the clamp, so its rounding is the answer unless it lies that
+// close to a half (or the step is near the ends of FP32's range, or not a number).
+DEVI void kv_codes(const float (&x)[4], float mn, float s, int (&code)[4]) {
+  const float d = s == 0.f ? 1.f : s, r = __builtin_amdgcn_rcpf(d);
+  float worst = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float q = fminf(fmaxf((x[i] - mn) * r, 0.f), 3.f), n = rintf(q);
+    worst = fmaxf(worst, fabsf(q - n));
+    code[i] = static_cast<int>(n);
+  }
+  if (!(worst < 0.5f - 9.5367431640625e-07f && d > 1e-30f && d < 1e30f)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) code[i] = kv_code(x[i], mn, s);
+  }
+}
 DEVI float kv_rec(int code, float mn, float s) { return static_cast<float>(code) * s + mn; }
 
 }  // namespace frkv

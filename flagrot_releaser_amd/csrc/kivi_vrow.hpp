@@ -22,7 +22,7 @@ enum Basis { AS_STORED = 0, BLOCK32 = 1, WHOLE = 2 };
 template <int NH>
 struct Trial {
   float step[NH], floor[NH];        // of this lane's sub-vector in each half (the 8 lanes of a sub-vector hold the same)
-  int level[NH][4];
+  uint32_t levels[NH];              // the lane's four 2-bit levels, a byte
   float miss[NH][4];                // reconstruction - row, original basis
 };
 
@@ -65,10 +65,13 @@ DEVI void trial_in_basis(const float (&x)[NH][4], int l32, Trial<NH>& t) {
     float st = kv_scale(lo, hi);
     kv_params<F8>(lo, st);
     t.step[s] = st; t.floor[s] = lo;
+    int level[4];
+    kv_codes(y[s], lo, st, level);
+    t.levels[s] = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      t.level[s][i] = kv_code(y[s][i], lo, st);
-      y[s][i] = kv_rec(t.level[s][i], lo, st);
+      t.levels[s] |= static_cast<uint32_t>(level[i] & 3) << (2 * i);
+      y[s][i] = kv_rec(level[i], lo, st);
     }
   }
   rebase<NH, B>(y, l32);
@@ -167,20 +170,19 @@ DEVI Picks pick_matrix(const Trial<NH> (&t)[3], const float* __restrict__ Mh, fl
 // ---- what the row stores for half s once the picks are made
 template <int NH> DEVI int basis_of(const Picks& p, int s) { return p.whole ? WHOLE : ((p.block32 >> s) & 1u) ? BLOCK32 : AS_STORED; }
 
-template <int NH> DEVI uint32_t chosen_byte(const Trial<NH> (&t)[3], int b, int s) {      // the lane's four 2-bit levels
-  uint32_t byte = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int lv = b == AS_STORED ? t[0].level[s][i] : b == BLOCK32 ? t[1].level[s][i] : t[2].level[s][i];
-    byte |= static_cast<uint32_t>(lv & 3) << (2 * i);
-  }
-  return byte;
+// (masks: a choice between members of an array would put all of it into scratch memory)
+DEVI uint32_t of_basis(int b, uint32_t as_stored, uint32_t block32, uint32_t whole) {
+  const uint32_t r = 0u - static_cast<uint32_t>(b == BLOCK32), w = 0u - static_cast<uint32_t>(b == WHOLE);
+  return (as_stored & ~(r | w)) | (block32 & r) | (whole & w);
+}
+template <int NH> DEVI uint32_t chosen_byte(const Trial<NH> (&t)[3], int b, int s) {
+  return of_basis(b, t[0].levels[s], t[1].levels[s], t[2].levels[s]);
 }
 // the stored (step, floor) word of a sub-vector: FP16 pair with the H32 flag in the step's sign bit, or the E4M3 byte
 // pair with the flag in bit 7 of the step byte
 template <int NH, bool F8> DEVI uint32_t chosen_meta(const Trial<NH> (&t)[3], int b, int s) {
-  const float st = b == AS_STORED ? t[0].step[s] : b == BLOCK32 ? t[1].step[s] : t[2].step[s];
-  const float lo = b == AS_STORED ? t[0].floor[s] : b == BLOCK32 ? t[1].floor[s] : t[2].floor[s];
+  const float st = __uint_as_float(of_basis(b, __float_as_uint(t[0].step[s]), __float_as_uint(t[1].step[s]), __float_as_uint(t[2].step[s])));
+  const float lo = __uint_as_float(of_basis(b, __float_as_uint(t[0].floor[s]), __float_as_uint(t[1].floor[s]), __float_as_uint(t[2].floor[s])));
   if (F8) return e4m3_bits(st) | (b == BLOCK32 ? 0x80u : 0u) | (e4m3_bits(lo) << 8);
   return (f16_bits_rn(st) & 0x7FFFu) | (b == BLOCK32 ? 0x8000u : 0u) | (f16_bits_rn(lo) << 16);
 }

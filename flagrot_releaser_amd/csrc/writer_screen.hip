@@ -20,8 +20,8 @@
 // A step takes 16 tokens: candidates in registers (a token on D / 4 lanes, two tokens each), the three error vectors of
 // every token as columns of two BF16 matrices in LDS; the base candidate's column of the head form is put together by
 // address, block by block.
-// Bound by the candidates: 12 IEEE divisions and 4 transforms a row; the matrix pipe takes 1280 cycles a step and
-// wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 131 us (before: the forms in FP32 on the matrix
+// Bound by the candidates: three quantisations and five transforms a row, some 800 vector instructions per pair of tokens;
+// the matrix pipe takes 1280 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 108 us (before: the forms in FP32 on the matrix
 // pipe, C read from L2 at every step); 2000 tokens x 4 heads of 256 on 2-bit pages 241 -> 55 us (before: exact only).
 #include <cstdlib>
 
