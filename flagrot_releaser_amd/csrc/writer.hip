@@ -24,12 +24,18 @@ DEVI void wave_lds_sync() {  // LDS hand-over between lanes of one wavefront
 }
 
 // ------------------------------------------------------------------------------------------------ static writer
+// Workgroup = eight consecutive tokens of one head row (K or V), one per half wave.  Value codes of eight consecutive slots
+// go through LDS and are stored word by word: whole where the slots are one aligned run, merged (one and / or pair a word)
+// where they are the end of one run and the beginning of the next (a chunk that does not begin on a multiple of eight) or
+// anything else in which two neighbours share words; scattered slots (a decode step) field by field.  A decode step is bound
+// by its launch (3 us).  One unaligned chunk of 1024 / 8192 tokens x 8 + 8 rows, 4-bit pages: 31 / 202 -> 7.7 / 36 us
+// (before: a merge per field), 2-bit pages 109 / 725 -> 6.6 / 30 us.
 template <int QM, int P>
 __global__ void __launch_bounds__(256) k_static_write(const StaticWriteParams p) {
   using L = Lay<QM, P>;
-  // workgroup = eight consecutive tokens of one head row (K or V), one per half wave
   __shared__ long long vslot[8];
   __shared__ __align__(16) uint8_t vcodes[8][128];
+  __shared__ VRuns<8> runs;
   const int l32 = threadIdx.x & 31, hw = threadIdx.x >> 5;
   const int H2 = 2 * p.Hkv;
   const int hr = static_cast<int>(blockIdx.x % H2);
@@ -70,21 +76,39 @@ __global__ void __launch_bounds__(256) k_static_write(const StaticWriteParams p)
     store_row<QM, P>(chunk, pos, false, code, word, l32, false);
     return;
   }
-  // value rows: an aligned run of 8 slots of one page gets its V^T words assembled in LDS and stored whole
   if (live) store_v_word<QM, P>(chunk, pos, word, l32, false);
   if (l32 == 0) vslot[hw] = slot;
   *reinterpret_cast<uint32_t*>(&vcodes[hw][4 * l32]) = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
   __syncthreads();
   const long long s0 = vslot[0];
-  bool run = s0 >= 0 && (s0 & 7) == 0;
+  bool run = s0 >= 0, share = false;
 #pragma unroll
-  for (int i = 1; i < 8; ++i) run = run && vslot[i] == s0 + i;
-  if (run) {
-    constexpr int NWORD = QM == QM_ASYM2 ? 64 : 128;
-    if (threadIdx.x < NWORD)
-      store_v_run_word<QM, P>(p.pool + ((s0 / P) * p.Hkv + head) * L::CHUNK, static_cast<int>(s0 % P) >> 3, threadIdx.x, vcodes);
-  } else if (live) {
-    store_v_codes<QM, P>(chunk, pos, code, l32);
+  for (int i = 1; i < 8; ++i) {
+    run = run && vslot[i] == s0 + i;
+    share = share || (vslot[i] >= 0 && ((vslot[i] ^ vslot[i - 1]) & ~7LL) == 0);
+  }
+  constexpr int NWORD = QM == QM_ASYM2 ? 64 : 128;
+  const int off = static_cast<int>(s0 & 7), j = threadIdx.x % NWORD, r = threadIdx.x / NWORD;
+  if (!run) {
+    if (!share) {
+      if (live) store_v_codes<QM, P>(chunk, pos, code, l32);
+      return;
+    }
+    if (threadIdx.x < 64) v_runs<8>(vslot, runs);
+    __syncthreads();
+    const int n = runs.n;
+    for (int i = r; i < n; i += 256 / NWORD)
+      store_v_words<QM, P>(p.pool + ((runs.first[i] / P) * p.Hkv + head) * L::CHUNK, static_cast<int>(runs.first[i] % P) >> 3, j,
+                           &vcodes[0][0], 128, runs.map[i]);
+  } else if (off == 0) {
+    if (r == 0)
+      store_v_run_word<QM, P>(p.pool + ((s0 / P) * p.Hkv + head) * L::CHUNK, static_cast<int>(s0 % P) >> 3, j, vcodes);
+  } else if (r < 2) {                    // position b of the runs: token b - off of the first, b + 8 - off of the second
+    const long long first = s0 - off + 8 * r;
+    unsigned long long map = r == 0 ? 0x0706050403020100ull << (8 * off) : 0x0706050403020100ull >> (8 * (8 - off));
+    map |= r == 0 ? ~0ull >> (8 * (8 - off)) : ~0ull << (8 * off);
+    store_v_words<QM, P>(p.pool + ((first / P) * p.Hkv + head) * L::CHUNK, static_cast<int>(first % P) >> 3, j, &vcodes[0][0], 128,
+                         map);
   }
 }
 
