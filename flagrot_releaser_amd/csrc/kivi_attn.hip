@@ -1,5 +1,5 @@
 // extern "C" surface of libflagrot_kivi.so (declared in include/flagrot_kivi.h) and the split merge of the decode
-// attention.  The value writer, the dequantiser and the LSE merge are in kivi_write.hip, the key group encoder in
+// attention.  The value writer and the LSE merge are in kivi_write.hip, the dequantiser in kivi_read.hip, the key group encoder in
 // kivi_kenc.hip, the decode splits in kivi_decode.hip, the rest of head dim 256 in kivi_wide.hip.
 // Semantics follow integrations/vllm_flagrot/csrc/kivi.cu:1908-1931 (k_merge) and :1933-2342 (C ABI).
 #include <cstdio>
@@ -88,11 +88,8 @@ int kv_dequant(const void* pool, const void* bt, int g0, int g1, int nvalid, int
                int f8, void* stream) {
   if (g1 <= g0) return 0;
   if (D != 128 && D != 256) return bad("kv_dequant: head dim 128 or 256");
-  if (D == 256)
-    return launched(dequant256_launch(static_cast<const uint8_t*>(pool), static_cast<const int*>(bt), g0, g1, nvalid, Hkv, fp32,
-                                      ok, ov, f8 & 1, static_cast<hipStream_t>(stream)), "kv_dequant");
-  return launched(dequant_launch(static_cast<const uint8_t*>(pool), static_cast<const int*>(bt), g0, g1, nvalid, Hkv, fp32, ok,
-                                 ov, f8 & 1, static_cast<hipStream_t>(stream)), "kv_dequant");
+  return launched(dequant_launch(D, static_cast<const uint8_t*>(pool), static_cast<const int*>(bt), g0, g1, nvalid, Hkv, fp32,
+                                 ok, ov, f8 & 1, static_cast<hipStream_t>(stream)), "kv_dequant");
 }
 
 int kv_lse_merge(const void* oa, const void* la, long long la_hs, const void* ob, const void* lb, long long lb_hs,

@@ -138,11 +138,6 @@ DEVI void lds_put(float* row, int l32, const float (&x)[2][4]) {
 }
 
 // ------------------------------------------------------------------------------------------------ dequantiser
-template <typename OT> DEVI OT cvt_out2(float v);
-template <> DEVI float cvt_out2<float>(float v) { return v; }
-template <> DEVI uint16_t cvt_out2<uint16_t>(float v) { return static_cast<uint16_t>(bf16_rn(v)); }
-
-// key flags of a group from its first page: bits 0..7 = sub-vector j is H32, bit 8 = whole head
 template <bool F8> DEVI uint32_t key_flags(const uint8_t* chA) {
   uint32_t f = 0;
   if (F8) {
@@ -152,86 +147,6 @@ template <bool F8> DEVI uint32_t key_flags(const uint8_t* chA) {
     for (int j = 0; j < 9; ++j) f |= ((m0[j] >> 15) & 1u) << j;
   }
   return f;
-}
-
-template <typename OT, bool F8>
-__global__ void __launch_bounds__(256) k_dequant256(const uint8_t* __restrict__ pool, const int* __restrict__ bt, int g0,
-                                                    int Hkv, int nvalid, OT* __restrict__ ok, OT* __restrict__ ov) {
-  const int gi = blockIdx.x, h = blockIdx.y, hw = threadIdx.x >> 5, l32 = threadIdx.x & 31;
-  const int g = g0 + gi;
-  const uint8_t* chA = pool + (static_cast<long long>(bt[2 * g]) * Hkv + h) * CHUNK2<F8>;
-  const uint8_t* chB = pool + (static_cast<long long>(bt[2 * g + 1]) * Hkv + h) * CHUNK2<F8>;
-  const uint32_t kfl = key_flags<F8>(chA);
-  // this lane's key channels 128 s + 4 l32 + i: cell 16 s + (l32 >> 1) (page s), slots 4 (l32 & 1) + i
-  float ks[2][4], kmn[2][4];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const uint8_t* km = (s ? chB : chA) + KM2 + (l32 >> 1) * CELL<F8> + 4 * (l32 & 1) * (F8 ? 2 : 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { bool fl; meta_read<F8>(km + i * (F8 ? 2 : 4), ks[s][i], kmn[s][i], fl); }
-  }
-  const int j = l32 >> 3;
-  for (int t = hw; t < 32; t += 8) {
-    const long long o = static_cast<long long>(gi) * 32 + t;
-    const uint8_t* ch = t < 16 ? chA : chB;
-    const int cell = t & 15;
-    {
-      float x[2][4];
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const uint32_t w = reinterpret_cast<const uint32_t*>(ch + cell * 64)[8 * s + (l32 >> 2)];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int ci = (4 * l32 + i) & 15;
-          x[s][i] = static_cast<float>((w >> (2 * (ci >> 1) + 16 * (ci & 1))) & 3u) * ks[s][i] + kmn[s][i];
-        }
-      }
-      if ((kfl >> 8) & 1u) h256(x, l32);
-      else if (kfl & 0xFFu) {
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          float y[4] = {x[s][0], x[s][1], x[s][2], x[s][3]};
-          fwht<32>(y, l32);
-          if ((kfl >> (4 * s + j)) & 1u) { x[s][0] = y[0]; x[s][1] = y[1]; x[s][2] = y[2]; x[s][3] = y[3]; }
-        }
-      }
-      if (o < nvalid)
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) ok[(o * Hkv + h) * D2 + 128 * s + 4 * l32 + i] = cvt_out2<OT>(x[s][i]);
-    }
-    {
-      const bool f = value_whole<F8>(ch, cell);
-      float x[2][4];
-      uint32_t l = 0;
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        float vs, vmn;
-        bool fl;
-        meta_read<F8>(ch + VM2<F8> + cell * CELL<F8> + (4 * s + j) * (F8 ? 2 : 4), vs, vmn, fl);
-        l |= (fl ? 1u : 0u) << s;
-        const uint32_t byte = ch[VC2<F8> + cell * 64 + 32 * s + l32];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[s][i] = static_cast<float>((byte >> (2 * i)) & 3u) * vs + vmn;
-      }
-      // (the butterflies exchange across the half wave: every lane runs them, the flag only selects the result)
-      if (f) h256(x, l32);
-      else {
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          float y[4] = {x[s][0], x[s][1], x[s][2], x[s][3]};
-          fwht<32>(y, l32);
-          if ((l >> s) & 1u) { x[s][0] = y[0]; x[s][1] = y[1]; x[s][2] = y[2]; x[s][3] = y[3]; }
-        }
-      }
-      if (o < nvalid)
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) ov[(o * Hkv + h) * D2 + 128 * s + 4 * l32 + i] = cvt_out2<OT>(x[s][i]);
-    }
-  }
 }
 
 // ------------------------------------------------------------------------------------------------ decode attention
@@ -450,19 +365,6 @@ int v_write256_launch(const void* kv, long long kv_rs, int n, int Hkv, const lon
                          : (f8 ? k_v_write256<true, false> : k_v_write256<false, false>);
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((items + 7) / 8)), dim3(256), 0, st, static_cast<const uint16_t*>(kv),
                      kv_rs, n, Hkv, slots, co, M, pool, ident, vfix);
-  return hipPeekAtLastError() == hipSuccess ? 0 : 1;
-}
-
-int dequant256_launch(const uint8_t* pool, const int* bt, int g0, int g1, int nvalid, int Hkv, int fp32, void* ok, void* ov,
-                      int f8, hipStream_t st) {
-  dim3 grid(g1 - g0, Hkv);
-  if (fp32) {
-    const auto kern = f8 ? k_dequant256<float, true> : k_dequant256<float, false>;
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, pool, bt, g0, Hkv, nvalid, static_cast<float*>(ok), static_cast<float*>(ov));
-  } else {
-    const auto kern = f8 ? k_dequant256<uint16_t, true> : k_dequant256<uint16_t, false>;
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, pool, bt, g0, Hkv, nvalid, static_cast<uint16_t*>(ok), static_cast<uint16_t*>(ov));
-  }
   return hipPeekAtLastError() == hipSuccess ? 0 : 1;
 }
 

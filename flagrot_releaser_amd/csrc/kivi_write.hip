@@ -1,5 +1,5 @@
-// KIVI-style FlagRot INT2 pages for gfx950: per-token value writer, page dequantiser and the bf16 LSE merge (the key
-// group encoder is in kivi_kenc.hip).  Compiled with -ffp-contract=off: the quantiser (scale, codes,
+// KIVI-style FlagRot INT2 pages for gfx950: per-token value writer and the bf16 LSE merge (the key group
+// encoder is in kivi_kenc.hip, the dequantiser in kivi_read.hip).  Compiled with -ffp-contract=off: the quantiser (scale, codes,
 // reconstruction) rounds every operation on its own, as the reference's (integrations/vllm_flagrot/csrc/kivi.cu:94-125).
 //
 // Page chunk per (16-token page, KV head), D = 128: KC @0 [16][32] key codes (32-bit words of 16 channels, channel i at
@@ -82,108 +82,6 @@ __global__ void __launch_bounds__(256) k_v_write(const uint16_t* __restrict__ kv
   }
 }
 
-// ------------------------------------------------------------------------------------------------ dequantiser
-template <typename OT> DEVI OT cvt_out(float v);
-template <> DEVI float cvt_out<float>(float v) { return v; }
-template <> DEVI uint16_t cvt_out<uint16_t>(float v) { return static_cast<uint16_t>(bf16_rn(v)); }
-
-template <typename OT, bool F8>
-__global__ void __launch_bounds__(256) k_dequant(const uint8_t* __restrict__ pool, const int* __restrict__ bt, int g0,
-                                                 int Hkv, int nvalid, OT* __restrict__ ok, OT* __restrict__ ov) {
-  const int gi = blockIdx.x, h = blockIdx.y, hw = threadIdx.x >> 5, l32 = threadIdx.x & 31;
-  const int g = g0 + gi;
-  const uint8_t* chA = pool + (static_cast<long long>(bt[2 * g]) * Hkv + h) * CHUNK<F8>;
-  const uint8_t* chB = pool + (static_cast<long long>(bt[2 * g + 1]) * Hkv + h) * CHUNK<F8>;
-  uint32_t lm = 0;
-  bool kF;
-  float ks[4], kmn[4];
-  // this lane's channels [4 l32, 4 l32 + 4) = key cell l32
-  if (F8) {
-    for (int j = 0; j < 4; ++j) lm |= static_cast<uint32_t>(chA[512 + 8 * j] >> 7) << j;
-    kF = chA[512 + 8 * 4] >> 7;
-    const uint8_t* km = (l32 < 16 ? chA : chB) + 512 + (l32 & 15) * 8;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { ks[i] = e4m3_value(km[2 * i] & 0x7Fu); kmn[i] = e4m3_value(km[2 * i + 1]); }
-  } else {
-    const uint32_t* m0 = reinterpret_cast<const uint32_t*>(chA + 512);
-    for (int j = 0; j < 4; ++j) lm |= ((m0[j] >> 15) & 1u) << j;
-    kF = (m0[4] >> 15) & 1u;                                    // cell 1, slot 0
-    const uint32_t* km = reinterpret_cast<const uint32_t*>((l32 < 16 ? chA : chB) + 512 + (l32 & 15) * 16);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { ks[i] = f16_value(km[i] & 0x7FFFu); kmn[i] = f16_value(km[i] >> 16); }
-  }
-  const int j = l32 >> 3;
-  for (int t = hw; t < 32; t += 8) {
-    const long long o = static_cast<long long>(gi) * 32 + t;
-    const uint8_t* ch = t < 16 ? chA : chB;
-    const int cell = t & 15;
-    // keys
-    {
-      const uint32_t w = reinterpret_cast<const uint32_t*>(ch + cell * 32)[l32 >> 2];
-      float x[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int ci = (4 * l32 + i) & 15;
-        x[i] = static_cast<float>((w >> (2 * (ci >> 1) + 16 * (ci & 1))) & 3u) * ks[i] + kmn[i];
-      }
-      if (kF) fwht<128>(x, l32);
-      else if (lm) {
-        float y[4] = {x[0], x[1], x[2], x[3]};
-        fwht<32>(y, l32);
-        if ((lm >> j) & 1u) { x[0] = y[0]; x[1] = y[1]; x[2] = y[2]; x[3] = y[3]; }
-      }
-      if (o < nvalid)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ok[(o * Hkv + h) * 128 + 4 * l32 + i] = cvt_out<OT>(x[i]);
-    }
-    // values
-    {
-      uint32_t l = 0;
-      bool f;
-      float vs, vmn;
-      if (F8) {
-        const uint8_t* vm = ch + VM_AT<true> + cell * 8;
-        for (int jj = 0; jj < 4; ++jj) l |= static_cast<uint32_t>(vm[2 * jj] >> 7) << jj;
-        f = ch[512 + cell * 8 + 6] >> 7;
-        vs = e4m3_value(vm[2 * j] & 0x7Fu); vmn = e4m3_value(vm[2 * j + 1]);
-      } else {
-        const uint32_t* vm = reinterpret_cast<const uint32_t*>(ch + VM_AT<false> + cell * 16);
-        for (int jj = 0; jj < 4; ++jj) l |= ((vm[jj] >> 15) & 1u) << jj;
-        f = ch[1536 + cell] != 0;
-        vs = f16_value(vm[j] & 0x7FFFu); vmn = f16_value(vm[j] >> 16);
-      }
-      const uint32_t byte = ch[VC_AT<F8> + cell * 32 + l32];
-      float x[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = static_cast<float>((byte >> (2 * i)) & 3u) * vs + vmn;
-      // The two tokens of a wavefront may differ in their flags: the stages H32 and H128 share (distance 1 .. 16 channels
-      // first, in H128's own order) run once for both, H128 adds its two stages across the sub-vectors.
-      if (f || l) {
-        float y[4] = {x[0], x[1], x[2], x[3]};
-        butterflies<32>(y, l32);
-        if (f) {
-#pragma unroll
-          for (int lm = 8; lm <= 16; lm <<= 1) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float o2 = hx(y[i], lm);
-              y[i] = (l32 & lm) ? (o2 - y[i]) : (y[i] + o2);
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) x[i] = y[i] * kC128;
-        } else if ((l >> j) & 1u) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) x[i] = y[i] * kC32;
-        }
-      }
-      if (o < nvalid)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ov[(o * Hkv + h) * 128 + 4 * l32 + i] = cvt_out<OT>(x[i]);
-    }
-  }
-}
-
 // ------------------------------------------------------------------------------------------------ LSE merge
 __global__ void k_lse_merge(const uint16_t* __restrict__ oa, const float* __restrict__ la, long long la_hs,
                             const uint16_t* __restrict__ ob, const float* __restrict__ lb, long long lb_hs,
@@ -213,19 +111,6 @@ int v_write_launch(const void* kv, long long kv_rs, int n, int Hkv, const long l
   const auto kern = wmat ? (f8 ? k_v_write<true, true> : k_v_write<false, true>) : (f8 ? k_v_write<true, false> : k_v_write<false, false>);
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((items + 7) / 8)), dim3(256), 0, st,
                      static_cast<const uint16_t*>(kv), kv_rs, n, Hkv, slots, co, M, pool, ident, vfix);
-  return hipPeekAtLastError() == hipSuccess ? 0 : 1;
-}
-
-int dequant_launch(const uint8_t* pool, const int* bt, int g0, int g1, int nvalid, int Hkv, int fp32, void* ok, void* ov,
-                   int f8, hipStream_t st) {
-  dim3 grid(g1 - g0, Hkv);
-  if (fp32) {
-    const auto kern = f8 ? k_dequant<float, true> : k_dequant<float, false>;
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, pool, bt, g0, Hkv, nvalid, static_cast<float*>(ok), static_cast<float*>(ov));
-  } else {
-    const auto kern = f8 ? k_dequant<uint16_t, true> : k_dequant<uint16_t, false>;
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, pool, bt, g0, Hkv, nvalid, static_cast<uint16_t*>(ok), static_cast<uint16_t*>(ov));
-  }
   return hipPeekAtLastError() == hipSuccess ? 0 : 1;
 }
 
