@@ -178,6 +178,11 @@ int fr_v2_attn(int fmt, const void* q, long long q_bs, const uint8_t* pool, cons
     return fail(-3, "fr_v2_attn: the head dim 256 kernels need opart and mlpart");
   p.wg_waves = big ? decode_waves(1 << 30) : 4;
   p.dyn = (can_draw && (!big || env_waves > 4)) ? 1 : 0;
+  // Head dim 256: the page loop needs more than 168 registers, so two wavefronts run per SIMD -- one workgroup of eight per
+  // CU, or two of four.  Launches that leave every CU at most one workgroup take the larger one where it has a quad for
+  // each wavefront (us, four against eight: 176 workgroups of 768 tokens 28.7 / 24.1, 32 of 512 20.5 / 18.0; 64 of 256
+  // tokens 15.5 / 16.0; 480 of 1664 tokens 68 / 72).
+  if (variant & HD256) p.wg_waves = pairs * nparts <= cus && chunk >= 512 ? 8 : 4;
   if (variant & HD256) return launched(decode_wide_launch(fmt, p, static_cast<hipStream_t>(stream)), "fr_v2_attn (head dim 256)");
   return launched(decode_launch(fmt, p, static_cast<hipStream_t>(stream)), "fr_v2_attn");
 }

@@ -7,7 +7,7 @@
 //            made once per workgroup; the tokens' whole-head flags sit in half 0's value scale words;
 //   softmax  once per quad;
 //   values   per half: p * V-scale strips of that half's four groups, then its value products into its own accumulators.
-// One workgroup of 4 wavefronts per (KV head x q tile of 4 heads, split, sequence), wavefront = head in the prologue;
+// One workgroup of 4 or 8 wavefronts per (KV head x q tile of 4 heads, split, sequence), wavefront = head in the prologue;
 // the wavefronts draw quads of 64 tokens from a counter in LDS.  Partials go out in the format of k_wide_parts
 // (decode_wide.hip: o [4][256] relative to the part's maxima, (maximum, sum) per head), whose merge kernel serves
 // both; the BF16 sink / window rows are one more split of this grid (plain fp32, a wavefront per row).
@@ -19,9 +19,7 @@ namespace fr {
 using namespace dec;
 namespace {
 
-constexpr int NWW = 4;
-
-template <int QM> struct WideMma {
+template <int QM, int NWW> struct WideMma {
   static constexpr int STRIP_BYTES = Strip<QM>::BYTES;
   alignas(16) uint4 qhi[2][4][64];                   // [half][group][lane of the matrix instruction]: as Smem::qhi
   alignas(16) uint4 qlo[2][4][64];
@@ -44,9 +42,10 @@ template <int QM> struct HalfView {
 
 // The 128-d prologue per half (decode_tiles.hpp q_prologue): wavefront = head, half wave 0 writes the rows of variants
 // 0 (identity, or the static kmask rotation) and 1 (H32), half wave 1 those of variant 2 (H256) and the idle row 3.
-template <int QM, bool K2>
-DEVI void q_prologue_wide(WideMma<QM>& S, const DecodeParams& p, int b, int kvh, int tile) {
+template <int QM, bool K2, int NWW>
+DEVI void q_prologue_wide(WideMma<QM, NWW>& S, const DecodeParams& p, int b, int kvh, int tile) {
   const int w = threadIdx.x >> 6, half = (threadIdx.x >> 5) & 1, l32 = threadIdx.x & 31;
+  if (w >= 4) return;
   const int hq = tile * 4 + w;
   float x[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   if (hq < p.gqa) {
@@ -120,8 +119,8 @@ DEVI void q_prologue_wide(WideMma<QM>& S, const DecodeParams& p, int b, int kvh,
 // lanes own 4 dims (lanes 0..31 half 0, 32..63 half 1), eight rows in flight; the wavefronts are merged through LDS and
 // the partial leaves in the body splits' format.  Static formats merge in the stored basis: the rows' share is rotated
 // on the vmask groups (H32 inside the eight lanes of a group).
-template <int QM, bool K2>
-DEVI void tail_split_wide(WideMma<QM>& S, const DecodeParams& p, int b, int kvh, int tile, float* __restrict__ op,
+template <int QM, bool K2, int NWW>
+DEVI void tail_split_wide(WideMma<QM, NWW>& S, const DecodeParams& p, int b, int kvh, int tile, float* __restrict__ op,
                           float* __restrict__ mlp) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = p.tail_len != nullptr ? p.tail_len[b] : 0;
@@ -144,7 +143,7 @@ DEVI void tail_split_wide(WideMma<QM>& S, const DecodeParams& p, int b, int kvh,
     }
     m[h] = -INFINITY; l[h] = 0.f;
   }
-  for (int tb = wave; tb < n; tb += 4 * 8) {
+  for (int tb = wave; wave < 4 && tb < n; tb += 4 * 8) {      // (four wavefronts share the rows, also of a larger workgroup)
     uint2 kr[8], vr[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -174,20 +173,21 @@ DEVI void tail_split_wide(WideMma<QM>& S, const DecodeParams& p, int b, int kvh,
   float Mwg[4];
   workgroup_max<NWW>(S, lane, Mwg);
   // [wave][head][256] fp32 = 16 KB in place of the operand tables (24 KB, contiguous), which this split never builds
-  static_assert(sizeof(S.qhi) + sizeof(S.qlo) >= NWW * 4 * 256 * 4 && offsetof(WideMma<QM>, qlo) == sizeof(S.qhi), "merge buffer");
+  using SM = WideMma<QM, NWW>;
+  static_assert(sizeof(S.qhi) + sizeof(S.qlo) >= 4 * 4 * 256 * 4 && offsetof(SM, qlo) == sizeof(S.qhi), "merge buffer");
   float* buf = reinterpret_cast<float*>(&S.qhi[0][0][0]);
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
     const float f = m[h] == -INFINITY ? 0.f : fexp2(m[h] - Mwg[h]);
     if (lane == 0) S.l[wave][h] = f * l[h];
-    *reinterpret_cast<float4*>(buf + (wave * 4 + h) * 256 + 4 * lane) = make_float4(f * o[h][0], f * o[h][1], f * o[h][2], f * o[h][3]);
+    if (wave < 4) *reinterpret_cast<float4*>(buf + (wave * 4 + h) * 256 + 4 * lane) = make_float4(f * o[h][0], f * o[h][1], f * o[h][2], f * o[h][3]);
   }
   __syncthreads();
-  {   // wavefront = head: sum over the wavefronts, rotate (static formats), store
+  if (wave < 4) {   // wavefront = head: sum over the wavefronts, rotate (static formats), store
     const int h = wave;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int w = 0; w < NWW; ++w) {
+    for (int w = 0; w < 4; ++w) {
       const float4 v = *reinterpret_cast<const float4*>(buf + (w * 4 + h) * 256 + 4 * lane);
       a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
     }
@@ -204,11 +204,11 @@ DEVI void tail_split_wide(WideMma<QM>& S, const DecodeParams& p, int b, int kvh,
   }
 }
 
-template <int QM, bool K2, int P>
+template <int QM, bool K2, int P, int NWW>
 __global__ void __launch_bounds__(64 * NWW, 2) k_wide_parts_mma(const DecodeParams p, int ntile, int nparts) {
   using L = Lay<QM, P>;
   constexpr int QB = QBLK<QM>, PPQ = 16 * QB / P;
-  __shared__ WideMma<QM> S;
+  __shared__ WideMma<QM, NWW> S;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // Workgroups go to the 8 XCDs round robin in dispatch order, and each XCD has its own L2.  The q tiles of one (KV
   // head, split, sequence) read the same pages: they are made neighbours ON ONE XCD (dispatch positions 8 apart), so
@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(64 * NWW, 2) k_wide_parts_mma(const DecodePara
   float* const op = p.opart + part_id * 4 * 256;
   float* const mlp = p.mlpart + part_id * 8;
   if (p.tail != nullptr && split == p.nsplit) {
-    tail_split_wide<QM, K2>(S, p, b, kvh, tile, op, mlp);
+    tail_split_wide<QM, K2, NWW>(S, p, b, kvh, tile, op, mlp);
     return;
   }
   const int len = p.seq_lens[b];
@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(64 * NWW, 2) k_wide_parts_mma(const DecodePara
   // the pad entry of every strip row group: what the value phase reads for the columns of foreign groups
   for (int i = threadIdx.x; i < NWW * Strip<QM>::ROWS; i += 64 * NWW)
     (reinterpret_cast<uint4*>(S.work + (i / Strip<QM>::ROWS) * Strip<QM>::BYTES) + (i % Strip<QM>::ROWS) * PB_RSTRIDE)[16] = make_uint4(0u, 0u, 0u, 0u);
-  q_prologue_wide<QM, K2>(S, p, b, kvh, tile);
+  q_prologue_wide<QM, K2, NWW>(S, p, b, kvh, tile);
   __syncthreads();
   const HalfView<QM> H0{S.qhi[0], S.qlo[0], S.qz[0], S.work}, H1{S.qhi[1], S.qlo[1], S.qz[1], S.work};
 
@@ -403,7 +403,7 @@ __global__ void __launch_bounds__(64 * NWW, 2) k_wide_parts_mma(const DecodePara
       }
     }
     __syncthreads();
-    {   // thread = (head `wave`, 2 dims of the half)
+    if (wave < 4) {   // thread = (head `wave`, 2 dims of the half)
       float2 acc = make_float2(0.f, 0.f);
 #pragma unroll
       for (int w = 0; w < NWW; ++w) {
@@ -414,19 +414,28 @@ __global__ void __launch_bounds__(64 * NWW, 2) k_wide_parts_mma(const DecodePara
     }
     __syncthreads();
   }
-  if (lane == 0) {
+  if (lane == 0 && wave < 4) {
     mlp[2 * wave] = pick4(Mwg[0], Mwg[1], Mwg[2], Mwg[3], wave);
-    mlp[2 * wave + 1] = (S.l[0][wave] + S.l[1][wave]) + (S.l[2][wave] + S.l[3][wave]);
+    float l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NWW; w += 4) l += (S.l[w][wave] + S.l[w + 1][wave]) + (S.l[w + 2][wave] + S.l[w + 3][wave]);
+    mlp[2 * wave + 1] = l;
   }
+}
+
+template <int QM, bool K2, int NWW>
+int wide_mma_nw(const DecodeParams& p, int ntile, int nparts, hipStream_t st) {
+  const dim3 grid(p.Hkv * ntile, nparts, p.B);
+  if (p.page == 16) hipLaunchKernelGGL((k_wide_parts_mma<QM, K2, 16, NWW>), grid, dim3(64 * NWW), 0, st, p, ntile, nparts);
+  else if (p.page == 32) hipLaunchKernelGGL((k_wide_parts_mma<QM, K2, 32, NWW>), grid, dim3(64 * NWW), 0, st, p, ntile, nparts);
+  else return -5;
+  return hipPeekAtLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int QM, bool K2>
 int wide_mma_qm(const DecodeParams& p, int ntile, int nparts, hipStream_t st) {
-  const dim3 grid(p.Hkv * ntile, nparts, p.B);
-  if (p.page == 16) hipLaunchKernelGGL((k_wide_parts_mma<QM, K2, 16>), grid, dim3(64 * NWW), 0, st, p, ntile, nparts);
-  else if (p.page == 32) hipLaunchKernelGGL((k_wide_parts_mma<QM, K2, 32>), grid, dim3(64 * NWW), 0, st, p, ntile, nparts);
-  else return -5;
-  return hipPeekAtLastError() == hipSuccess ? 0 : -1;
+  if (p.wg_waves > 4) return wide_mma_nw<QM, K2, 8>(p, ntile, nparts, st);
+  return wide_mma_nw<QM, K2, 4>(p, ntile, nparts, st);
 }
 
 }  // namespace
