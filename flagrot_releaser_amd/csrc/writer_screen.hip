@@ -21,8 +21,8 @@
 // every token as columns of two BF16 matrices in LDS; the base candidate's column of the head form is put together by
 // address, block by block.
 // Bound by the candidates: three quantisations and five transforms a row, some 800 vector instructions per pair of tokens;
-// the matrix pipe takes 1280 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 108 us (before: the forms in FP32 on the matrix
-// pipe, C read from L2 at every step); 2000 tokens x 4 heads of 256 on 2-bit pages 241 -> 55 us (before: exact only).
+// the matrix pipe takes 1280 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 105 us (before: the forms in FP32 on the matrix
+// pipe, C read from L2 at every step); 2000 tokens x 4 heads of 256 on 2-bit pages 241 -> 53 us (before: exact only).
 #include <cstdlib>
 
 #include "writer_exact.hpp"
@@ -107,14 +107,15 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
     uint32_t nosign = 0x7FFF7FFFu;
     asm volatile("" : "+s"(nosign));            // (the magnitudes of C are not hoisted out of the loop into registers)
     // ---- P1: candidates and value rows of the unit's two tokens
-    long long slot[2];
-#pragma unroll
+    // (a loop, not two copies: with the copies 24 registers spill, 108 -> 105 us; a loop over the candidates too: 112)
+#pragma unroll 1
     for (int u = 0; u < 2; ++u) {
       const int tk = 2 * unit + u, t = tb0 + tk;
-      slot[u] = -1;
-      if (t < t_hi) slot[u] = p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)];
+      long long slot = -1;
+      if (t < t_hi) slot = p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)];
+      if (lu == 0) S.slot[tk] = slot;
       float x[4] = {0.f, 0.f, 0.f, 0.f}, v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (slot[u] >= 0) {
+      if (slot >= 0) {
         const long long at = static_cast<long long>(t) * p.kv_ts + d0;
         load_row(p.kv, at + static_cast<long long>(h) * D, x);
         if (do_v) load_row(p.kv, at + static_cast<long long>(p.Hkv + h) * D, v);
@@ -152,7 +153,6 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
         for (int i = 0; i < 4; ++i) pack |= code_bits(q[i], QM == QM_SYM4) << (8 * i);
         *reinterpret_cast<uint32_t*>(&S.vcode[tk][d0]) = pack;
         if ((lu & 7) == 0) S.word[3][tk][g] = static_cast<uint16_t>(w);
-        if (lu == 0) S.slot[tk] = slot[u];
       }
     }
     __syncthreads();
@@ -242,9 +242,10 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
     }
     __syncthreads();
     // ---- P4: base against whole head; the rows of the decided tokens into their pages
-#pragma unroll
+#pragma unroll 1
     for (int u = 0; u < 2; ++u) {
       const int tk = 2 * unit + u;
+      const long long slot = S.slot[tk];
       float e[2], b[2];
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
@@ -258,14 +259,14 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
 #pragma unroll
       for (int w = 0; w < NB / 4; ++w)
         if (reinterpret_cast<const uint32_t*>(&S.choice[tk][0])[w] & 0x02020202u) dec = 2;
-      if (slot[u] < 0) continue;
+      if (slot < 0) continue;
       if (dec == 2) {
         if (lu == 0) S.fb[atomicAdd(&S.nfb, 1)] = tb0 + tk;
         continue;
       }
       const int c = dec == 1 ? 2 : S.choice[tk][g];
-      uint8_t* chunk = p.pool + ((slot[u] / P) * (p.Hkv * (D / 128)) + h * (D / 128) + half) * L::CHUNK;
-      const int pos = static_cast<int>(slot[u] % P);
+      uint8_t* chunk = p.pool + ((slot / P) * (p.Hkv * (D / 128)) + h * (D / 128) + half) * L::CHUNK;
+      const int pos = static_cast<int>(slot % P);
       const uint32_t pack = S.code[c][tk][lu];
       const uint32_t code[4] = {pack & 0xFFu, (pack >> 8) & 0xFFu, (pack >> 16) & 0xFFu, pack >> 24};
       store_row<QM, P>(chunk, pos, false, code, S.word[c][tk][g] | (c == 1 ? 0x8000u : 0u), l32, false);
