@@ -21,28 +21,14 @@ struct alignas(16) StepSmem {
   float head[2];
 };
 
-// One token whose slot is not negative, to its page.  VCODES: store the value codes too (field by field).  Every thread of
-// the workgroup calls it; the caller puts a barrier between two calls.
-template <int QM, int P, int D, bool VCODES>
-DEVI void k2_exact_token(const K2WriteParams& p, StepSmem<D>& S, int h, int t, long long slot) {
-  using L = Lay<QM, P>;
-  constexpr int NB = D / 32, O = D / 64;           // column blocks = wavefronts; output channels per lane
-  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31;
-  const bool do_k = p.passes & 1, do_v = p.passes & 2;
-  const int half = D == 256 ? lane >> 5 : 0, d0 = 128 * half + 4 * l32;
-  float x[4] = {0.f, 0.f, 0.f, 0.f};
-  if (wv < 4) {
-    load_row(p.kv, static_cast<long long>(t) * p.kv_ts + static_cast<long long>(wv == 3 ? p.Hkv + h : h) * D + d0, x);
-    if (p.kmu != nullptr && wv < 3) {
-      const float4 m = *reinterpret_cast<const float4*>(p.kmu + h * D + d0);
-      x[0] = x[0] - m.x; x[1] = x[1] - m.y; x[2] = x[2] - m.z; x[3] = x[3] - m.w;
-    }
-  }
-  // CT[k][i] = C_q[i][k]: the thread's column of its local block, and its outputs' rows of the wavefront's block
-  const int cand = tid / D, out = tid % D, g = out >> 5;
-  float cl[32], cf[32][O];
-  if (do_k) {
-    const float* CT = p.CT + static_cast<size_t>(h) * D * D;
+// The thread's numbers of C_q^T (CT[k][i] = C_q[i][k]): the column of its local block, its outputs' rows of the wavefront's
+// block.  Loaded once for all tokens of the workgroup.
+template <int D>
+struct CqRegs {
+  float cl[32], cf[32][D / 64];
+  DEVI void load(const float* CT) {
+    constexpr int O = D / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, out = tid % D, g = out >> 5;
     const float* lcol = CT + static_cast<size_t>(32 * g) * D + out;
     const float* frow = CT + static_cast<size_t>(32 * wv) * D + O * lane;
 #pragma unroll
@@ -58,6 +44,28 @@ DEVI void k2_exact_token(const K2WriteParams& p, StepSmem<D>& S, int h, int t, l
       }
     }
   }
+};
+
+// One token whose slot is not negative, to its page.  FRESH: the numbers of C_q^T are asked for here, behind the rows and
+// before the candidates, and the value codes are stored too (field by field).  Every thread of the workgroup calls it; the
+// caller puts a barrier between two calls.
+template <int QM, int P, int D, bool FRESH>
+DEVI void k2_exact_token(const K2WriteParams& p, StepSmem<D>& S, CqRegs<D>& C, int h, int t, long long slot) {
+  using L = Lay<QM, P>;
+  constexpr int NB = D / 32, O = D / 64;           // column blocks = wavefronts; output channels per lane
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31;
+  const bool do_k = p.passes & 1, do_v = p.passes & 2;
+  const int half = D == 256 ? lane >> 5 : 0, d0 = 128 * half + 4 * l32;
+  float x[4] = {0.f, 0.f, 0.f, 0.f};
+  if (wv < 4) {
+    load_row(p.kv, static_cast<long long>(t) * p.kv_ts + static_cast<long long>(wv == 3 ? p.Hkv + h : h) * D + d0, x);
+    if (p.kmu != nullptr && wv < 3) {
+      const float4 m = *reinterpret_cast<const float4*>(p.kmu + h * D + d0);
+      x[0] = x[0] - m.x; x[1] = x[1] - m.y; x[2] = x[2] - m.z; x[3] = x[3] - m.w;
+    }
+  }
+  const int cand = tid / D, out = tid % D, g = out >> 5;
+  if (FRESH && do_k) C.load(p.CT + static_cast<size_t>(h) * D * D);
   __builtin_amdgcn_sched_barrier(0);               // all of them asked for before the candidates are formed
   uint8_t* chunk = p.pool + ((slot / P) * (p.Hkv * (D / 128)) + h * (D / 128) + half) * L::CHUNK;
   const int pos = static_cast<int>(slot % P);
@@ -76,7 +84,7 @@ DEVI void k2_exact_token(const K2WriteParams& p, StepSmem<D>& S, int h, int t, l
       for (int i = 0; i < 4; ++i) e[i] = e[i] - x[i];
       *reinterpret_cast<float4*>(&S.err[wv][d0]) = make_float4(e[0], e[1], e[2], e[3]);
       S.code[wv][lane] = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
-    } else if (VCODES && (D == 256 || lane < 32)) {
+    } else if (FRESH && (D == 256 || lane < 32)) {
       store_v_codes<QM, P>(chunk, pos, code, l32);
     }
   }
@@ -91,7 +99,7 @@ DEVI void k2_exact_token(const K2WriteParams& p, StepSmem<D>& S, int h, int t, l
         const float e[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float pr = cl[4 * k4 + i] * e[i];
+          const float pr = C.cl[4 * k4 + i] * e[i];
           u = 4 * k4 + i == 0 ? pr : u + pr;
         }
       }
@@ -111,7 +119,7 @@ DEVI void k2_exact_token(const K2WriteParams& p, StepSmem<D>& S, int h, int t, l
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int o = 0; o < O; ++o) {
-            const float pb = cf[4 * k4 + i][o] * b[i], pf = cf[4 * k4 + i][o] * f[i];
+            const float pb = C.cf[4 * k4 + i][o] * b[i], pf = C.cf[4 * k4 + i][o] * f[i];
             ub[o] = 4 * k4 + i == 0 ? pb : ub[o] + pb;
             uf[o] = 4 * k4 + i == 0 ? pf : uf[o] + pf;
           }

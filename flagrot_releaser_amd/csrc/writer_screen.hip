@@ -4,14 +4,15 @@
 // every other token is evaluated exactly at the end of its workgroup.
 //
 // Estimate: C and d are split into two BF16 terms each (C = H + L + R, d = h + l + r with |L| <= 2^-8 |C|,
-// |R| <= 2^-16 |C|, the same for d); H h + H l + L h accumulate in FP32, the outer product takes h + l (exact in FP32).
-// A fourth product gives S~ = |h|^T |H| |h|.  With S = |d|^T |C| |d| and u = 2^-24:
-//   left out        L l, R d, H r and r of the outer product: at most 4 x 2^-16 S
-//   rounding        <= 384 products and sums inside the matrix pipe (128-d; each taken as accurate to 2 u, whatever its
-//                   order), a 16-term dot and 8 more sums: 816 u S; 256-d heads: 1600 u S
+// |R| <= 2^-16 |C|, the same for d); L l + H l + L h and then H h accumulate in FP32, the outer product takes h + l (exact
+// in FP32).  A fifth product gives S~ = |h|^T |H| |h|.  With S = |d|^T |C| |d| and u = 2^-24:
+//   left out        R d, H r and r of the outer product: 3 x 2^-16 S (and terms of 2^-24 S)
+//   rounding        of H h: <= 128 (256) products and sums inside the matrix pipe, each taken as accurate to 2 u, whatever
+//                   their order; the small products come first, so theirs are relative to sums of 2^-7 S: 6 (12) u S; a
+//                   16-term dot and 8 more sums: 24 u S
 //   the reference   sums of <= 39 terms, one product, a tree of depth 8: 48 u S
 //   S               <= (1 - 2^-8)^-3 S~ = 1.012 S~
-// together 1.15e-4 S~ (128-d) and 1.63e-4 S~ (256-d).  The screen uses b = kappa S~ + 2^-100 with kappa = 1.3 x that:
+// together 6.69e-5 S~ (128-d) and 8.27e-5 S~ (256-d).  The screen uses b = kappa S~ + 2^-100 with kappa = 1.15 x that:
 // candidate a beats candidate c for certain when e~_a + b_a < e~_c - b_c.  Infinities and NaN leave every comparison
 // undecided.
 //
@@ -21,7 +22,7 @@
 // every token as columns of two BF16 matrices in LDS; the base candidate's column of the head form is put together by
 // address, block by block.
 // Bound by the candidates: three quantisations and five transforms a row, some 800 vector instructions per pair of tokens;
-// the matrix pipe takes 1280 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 105 us (before: the forms in FP32 on the matrix
+// the matrix pipe takes 1600 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 105 us (before: the forms in FP32 on the matrix
 // pipe, C read from L2 at every step); 2000 tokens x 4 heads of 256 on 2-bit pages 241 -> 53 us (before: exact only).
 #include <cstdlib>
 
@@ -165,10 +166,15 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
       for (int i = 0; i < 2; ++i) {
         const uint4 bh = *reinterpret_cast<const uint4*>(&S.hi[l32][32 * wv + 16 * i + 8 * kq]);
         const uint4 bl = *reinterpret_cast<const uint4*>(&S.lo[l32][32 * wv + 16 * i + 8 * kq]);
-        acc = mfma(ah[i], bh, acc);
-        mag = mfma(magnitude(ah[i], nosign), magnitude(bh, nosign), mag);
+        acc = mfma(al[i], bl, acc);
         acc = mfma(ah[i], bl, acc);
         acc = mfma(al[i], bh, acc);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint4 bh = *reinterpret_cast<const uint4*>(&S.hi[l32][32 * wv + 16 * i + 8 * kq]);
+        acc = mfma(ah[i], bh, acc);
+        mag = mfma(magnitude(ah[i], nosign), magnitude(bh, nosign), mag);
       }
       float f = 0.f, s = 0.f;
 #pragma unroll
@@ -199,17 +205,21 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
       const bool whole = l32 >= 16;
       const int c0 = whole ? 2 * SCR_TOK + tok : tok;
 #pragma unroll
-      for (int i = 0; i < KB; i += 2) {
-        const int blk = (wv + i / 2) & (NB - 1);
+      for (int i = 0; i < 2 * KB; i += 2) {         // the three small products of all blocks, then the large one
+        const int blk = (wv + (i % KB) / 2) & (NB - 1);
         const int col = c0 + (!whole && S.choice[tok][blk] == 1 ? SCR_TOK : 0);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const uint4 bh = *reinterpret_cast<const uint4*>(&S.hi[col][32 * blk + 16 * j + 8 * kq]);
-          const uint4 bl = *reinterpret_cast<const uint4*>(&S.lo[col][32 * blk + 16 * j + 8 * kq]);
-          acc = mfma(ah[i + j], bh, acc);
-          mag = mfma(magnitude(ah[i + j], nosign), magnitude(bh, nosign), mag);
-          acc = mfma(ah[i + j], bl, acc);
-          acc = mfma(al[i + j], bh, acc);
+          if (i < KB) {
+            const uint4 bl = *reinterpret_cast<const uint4*>(&S.lo[col][32 * blk + 16 * j + 8 * kq]);
+            acc = mfma(al[i % KB + j], bl, acc);
+            acc = mfma(ah[i % KB + j], bl, acc);
+            acc = mfma(al[i % KB + j], bh, acc);
+          } else {
+            acc = mfma(ah[i % KB + j], bh, acc);
+            mag = mfma(magnitude(ah[i % KB + j], nosign), magnitude(bh, nosign), mag);
+          }
           if (j == 1) __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -285,11 +295,12 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
   // ---- the tokens the screen could not decide
   __syncthreads();
   const int nfb = S.nfb;
+  if (nfb == 0) return;
+  CqRegs<D> C;
+  C.load(p.CT + static_cast<size_t>(h) * D * D);
   for (int i = 0; i < nfb; ++i) {
     const int t = S.fb[i];
-    K2WriteParams q = p;
-    asm volatile("" : "+s"(q.CT));              // (read again for every token: not kept in registers across the loop)
-    k2_exact_token<QM, P, D, false>(q, S.exact, h, t, p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)]);
+    k2_exact_token<QM, P, D, false>(p, S.exact, C, h, t, p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)]);
     __syncthreads();
   }
 }
@@ -307,7 +318,7 @@ int screen(const K2WriteParams& p, float kappa, hipStream_t st) {
 template <int QM>
 int screen_qm(const K2WriteParams& p, bool all_exact, hipStream_t st) {
   static const float scale = getenv("FLAGROT_W3_KAPPA") != nullptr ? static_cast<float>(atof(getenv("FLAGROT_W3_KAPPA"))) : 1.f;
-  const float kappa = all_exact ? 1e30f : scale * (p.hd == 256 ? 2.12e-4f : 1.5e-4f);
+  const float kappa = all_exact ? 1e30f : scale * (p.hd == 256 ? 9.5e-5f : 7.7e-5f);
   if (p.page != 16 && p.page != 32) return -5;
   if (p.hd == 256) return p.page == 16 ? screen<QM, 16, 256>(p, kappa, st) : screen<QM, 32, 256>(p, kappa, st);
   return p.page == 16 ? screen<QM, 16, 128>(p, kappa, st) : screen<QM, 32, 128>(p, kappa, st);

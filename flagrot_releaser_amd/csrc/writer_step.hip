@@ -15,7 +15,8 @@ __global__ void __launch_bounds__(2 * D) k_k2_step(const K2WriteParams p) {
   const int h = blockIdx.x, t = blockIdx.y;
   const long long slot = p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)];
   if (slot < 0) return;                            // the whole workgroup
-  k2_exact_token<QM, P, D, true>(p, S, h, t, slot);
+  CqRegs<D> C;
+  k2_exact_token<QM, P, D, true>(p, S, C, h, t, slot);
 }
 
 template <int QM, int P>
