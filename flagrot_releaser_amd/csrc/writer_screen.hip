@@ -22,8 +22,8 @@
 // every token as columns of two BF16 matrices in LDS; the base candidate's column of the head form is put together by
 // address, block by block.
 // Bound by the candidates: three quantisations and five transforms a row, some 800 vector instructions per pair of tokens;
-// the matrix pipe takes 1600 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 105 us (before: the forms in FP32 on the matrix
-// pipe, C read from L2 at every step); 2000 tokens x 4 heads of 256 on 2-bit pages 241 -> 53 us (before: exact only).
+// the matrix pipe takes 1600 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 91 us (before: the forms in FP32 on the matrix
+// pipe, C read from L2 at every step); 2000 tokens x 4 heads of 256 on 2-bit pages 241 -> 43 us (before: exact only).
 #include <cstdlib>
 
 #include "writer_exact.hpp"
@@ -307,11 +307,14 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
 
 template <int QM, int P, int D>
 int screen(const K2WriteParams& p, float kappa, hipStream_t st) {
-  // tokens per workgroup: all workgroups resident at once (3 per CU at head dim 128, 1 at 256) as far as the list allows
+  // Steps per workgroup: all workgroups resident at once (3 per CU at head dim 128, 1 at 256) as far as the list of undecided
+  // tokens allows; from five steps on, 128-d heads take workgroups of two, which the dispatcher spreads evenly (8 heads of
+  // 128, us for 1 / 2 / 4 / 6 / 8 steps: 8192 tokens 94 / 91 / 101 / 97 / 106, 6000 tokens 70 / 68 / 66 / 79 / 100; 4 heads of
+  // 256, 8192 tokens 187 / 166 / 139 / 188 / 131).
   constexpr long long RESIDENT = D == 128 ? 768 : 256;
-  const long long steps = (p.T + SCR_TOK - 1) / SCR_TOK;
-  const long long per = (steps * p.Hkv + RESIDENT - 1) / RESIDENT;
-  const int tile = SCR_TOK * static_cast<int>(per < SCR_MAXTILE / SCR_TOK ? per : SCR_MAXTILE / SCR_TOK);
+  const long long steps = (p.T + SCR_TOK - 1) / SCR_TOK, fit = (steps * p.Hkv + RESIDENT - 1) / RESIDENT;
+  const long long per = D == 128 && fit > 4 ? 2 : fit < SCR_MAXTILE / SCR_TOK ? fit : SCR_MAXTILE / SCR_TOK;
+  const int tile = SCR_TOK * static_cast<int>(per);
   hipLaunchKernelGGL((k_k2_screen<QM, P, D>), dim3(p.Hkv, (p.T + tile - 1) / tile), dim3(2 * D), 0, st, p, tile, kappa);
   return hipPeekAtLastError() == hipSuccess ? 0 : -1;
 }
