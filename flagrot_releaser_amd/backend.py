@@ -382,7 +382,8 @@ class KiviDecodeLayer:
         dev = pool.device
         self.ring = torch.zeros((planner.spare + 1) * self.geo.slots, 2 * Hkv, D, dtype=torch.bfloat16, device=dev)
         self.ws = kivi_workspace(dev, planner.max_rows, Hkv, G, D, planner.plan)
-        self._rows = None                                  # made by the first prompt, for prompts up to max_len
+        # row of every token of a prompt's key groups, -1 for the sinks (they stay BF16 only)
+        self._rows = self._rows_upto(planner.max_len // GROUP)
 
     def prefill(self, kv, slots, req: int):
         """a fresh prompt of n tokens: values of every token, the whole key groups, sinks and newest W rows in BF16"""
@@ -391,15 +392,13 @@ class KiviDecodeLayer:
         K.ring_rows(kv, self.ring, base=int(req) * self.geo.slots, sink=self.geo.S, window=self.geo.W)
         whole = n // GROUP
         if whole:
-            KIVI.k_encode(kv, self._prompt_rows(whole), slots[:whole * GROUP].view(whole, GROUP).contiguous(), self.qs,
+            rows = self._rows[:whole] if whole <= self._rows.shape[0] else self._rows_upto(whole)
+            KIVI.k_encode(kv, rows, slots[:whole * GROUP].view(whole, GROUP).contiguous(), self.qs,
                           self.lz, self.scale, self.pool, self.Hkv, D, f8=self.f8)
 
-    def _prompt_rows(self, groups: int):
-        """row of every token of the leading groups of a prompt, -1 for the sinks (they stay BF16 only)"""
-        if self._rows is None or self._rows.shape[0] < groups:
-            pos = torch.arange(max(groups, -(-self.planner.max_len // GROUP)) * GROUP, device=self.pool.device)
-            self._rows = pos.masked_fill_(pos < self.geo.S, -1).view(-1, GROUP)
-        return self._rows[:groups]
+    def _rows_upto(self, groups: int):
+        pos = torch.arange(groups * GROUP, device=self.pool.device)
+        return pos.masked_fill_(pos < self.geo.S, -1).view(-1, GROUP)
 
     def prefill_chunk(self, kv, slots, req: int, start: int, table_row):
         """the next n tokens of request `req`'s prompt, positions [start, start + n): values of every token, the key
