@@ -6,9 +6,10 @@
 // PyTorch encoders (kernels/ref.py:22-33,151-182; kernels/codebook_ref.py:119-236; blockflag/formats.py:135-174);
 // this file is compiled with -ffp-contract=off and IEEE division.
 //
-// Mapping: one half wave (32 lanes) owns one 128-d row, 4 consecutive dims per lane.  The selecting writer keeps the
-// head's 64 KB C_q^T in LDS for the whole workgroup and walks its tokens eight rows at a time; the error vectors of
-// the candidates live in a small per-half-wave LDS strip so that the fixed-order matvec reads them as broadcasts.
+// Mapping: one half wave (32 lanes) owns one 128-d row, 4 consecutive dims per lane.  The selecting writer of this file
+// (exact, any number of tokens; decode steps: writer_step.hip, prompts: writer_screen.hip) keeps the head's
+// 64 KB C_q^T in LDS for the whole workgroup and walks its tokens eight rows at a time; the error vectors of the
+// candidates live in a small per-half-wave LDS strip so that the fixed-order matvec reads them as broadcasts.
 #include <cstdlib>
 
 #include "fr_launch.hpp"
@@ -370,7 +371,7 @@ int k2_write_launch(int kind, const K2WriteParams& p, hipStream_t st) {
   const long long pairs = static_cast<long long>(p.T) * p.Hkv;
   // a decode step's worth of tokens: one workgroup per (token, head)
   static const bool no_step = getenv("FLAGROT_WRITER_LL") != nullptr && getenv("FLAGROT_WRITER_LL")[0] == '0';
-  if (!(no_step && p.hd == 128) && pairs <= 1024) return k2_step_launch(kind, p, st);
+  if (!(no_step && p.hd != 256) && pairs <= 1024) return k2_step_launch(kind, p, st);
   // Prompt-sized key passes: choices screened on the matrix pipe (FLAGROT_W3: 0 off for 128-d heads, 2 every token exact).
   // At 1024 pairs the two forms cost the same: 256-d heads 25 us by tokens, 2048 pairs 49 by tokens against 34-40.
   static const int w3mode = getenv("FLAGROT_W3") != nullptr ? atoi(getenv("FLAGROT_W3")) : 1;
@@ -382,7 +383,7 @@ int k2_write_launch(int kind, const K2WriteParams& p, hipStream_t st) {
   }
   return -4;
 }
-int k2_write_lds_bytes(int hd) {      // LDS a selecting-writer workgroup holds (the 256-d kernel: its error strips; C_q^T stays in L2)
+int k2_write_lds_bytes(int hd) {      // what fr_cb_write_smem reports: C_q^T and error strips; 256-d heads: error strips
   return hd == 256 ? static_cast<int>(8 * 2 * 256 * sizeof(float)) : K2_LDS;
 }
 

@@ -22,8 +22,9 @@
 // every token as columns of two BF16 matrices in LDS; the base candidate's column of the head form is put together by
 // address, block by block.
 // Bound by the candidates: three quantisations and five transforms a row, some 800 vector instructions per pair of tokens;
-// the matrix pipe takes 1600 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 171 -> 91 us (before: the forms in FP32 on the matrix
-// pipe, C read from L2 at every step); 2000 tokens x 4 heads of 256 on 2-bit pages 241 -> 43 us (before: exact only).
+// the matrix pipe takes 1600 cycles a step and wavefront.  Prompt of 8192 tokens x 8 heads of 128 on 4-bit pages 159 ->
+// 90 us (before: the forms in FP32 on the matrix pipe, C read from L2 at every step); 2048 tokens x 4 heads of 256 on
+// 2-bit pages 241 -> 44 us (before: exact only).
 #include <cstdlib>
 
 #include "writer_exact.hpp"
