@@ -410,16 +410,16 @@ def ring_rows(kv, ring, kmu=None, dest=None, base=0, sink=0, window=0, start=0):
     the ring row of every token (negative: skip).  Without it the tokens are positions start .. start + T - 1 of the
     request whose ring starts at row `base`: positions below `sink` go to their own slot, the newest `window` of the rest
     to slot sink + (p - sink) % window."""
-    T = kv.shape[0]
+    T, heads, Dh = kv.shape
     if T == 0:
         return
     assert kv.dtype == torch.bfloat16 and ring.dtype == torch.bfloat16 and ring.is_contiguous()
-    rows, width = _loadable(kv), kv.shape[1] * kv.shape[2]
+    rows = _loadable(kv)
     if dest is None:
-        assert (base + sink + window) * width <= ring.numel(), "the request's rows lie outside the ring"
+        assert (base + sink + window) * heads * Dh <= ring.numel(), "the request's rows lie outside the ring"
     else:
-        assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.shape[0] == T
-    NATIVE.run("fr_ring_rows", rows, rows.stride(0), T, kv.shape[1] // 2, kv.shape[2], _centre(kmu, rows), ring, dest,
+        assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.numel() == T
+    NATIVE.run("fr_ring_rows", rows, rows.stride(0), T, heads // 2, Dh, _centre(kmu, rows), ring, dest,
                base, sink, window, start, current_stream())
 
 
