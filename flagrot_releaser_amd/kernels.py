@@ -18,7 +18,7 @@ import os
 
 import torch
 
-from .native import Library, as_arg, current_stream
+from .native import Library, current_stream
 
 ABI = 9
 D, RB, NG = 128, 32, 4
@@ -241,8 +241,8 @@ class _Bound:
     (what a captured graph would replay), so the tensors have to stay alive and in place."""
 
     def __init__(self, entry: str, args: tuple):
-        self.entry, self.args = entry, args
-        self.fn = getattr(NATIVE.dll, entry)
+        self.entry = entry
+        self.fn, self.args = NATIVE.bind(entry, args)
 
     def __call__(self):
         if self.fn(*self.args):
@@ -251,7 +251,7 @@ class _Bound:
 
 def _decode(entry: str, args: tuple, bound: bool):
     if bound:
-        return _Bound(entry, tuple(map(as_arg, args)))
+        return _Bound(entry, args)
     NATIVE.run(entry, *args)
     return None
 

@@ -21,16 +21,17 @@ import torch
 
 from . import build as _build
 
-_CTYPE = {"p": ctypes.c_void_p, "i": ctypes.c_int, "l": ctypes.c_longlong, "f": ctypes.c_float}
+
+class _Pointer:
+    """argument type of the pointers: tensors pass their device address, everything else what c_void_p takes.  Numbers have
+    ctypes' own types: there a tensor of one element is its value and any other tensor an error, never an address."""
+
+    @staticmethod
+    def from_param(a):
+        return ctypes.c_void_p.from_param(a.data_ptr() if isinstance(a, torch.Tensor) else a)
 
 
-def as_arg(a):
-    """what ctypes gets for one Python argument: tensors -> device address, flags -> int, the rest unchanged"""
-    if isinstance(a, torch.Tensor):
-        return a.data_ptr()
-    if isinstance(a, bool):
-        return int(a)
-    return a
+_CTYPE = {"p": _Pointer, "i": ctypes.c_int, "l": ctypes.c_longlong, "f": ctypes.c_float}
 
 
 def current_stream() -> int:
@@ -104,10 +105,23 @@ class Library:
 
     def ask(self, name: str, *args) -> int:
         """an entry point whose int result is an answer (sizes, counts), not a status"""
-        return getattr(self.dll, name)(*map(as_arg, args))
+        return getattr(self.dll, name)(*args)
+
+    def bind(self, name: str, args: tuple):
+        """(entry point, arguments) for calls that are repeated as they are: the tensors' addresses are taken here"""
+        typed = getattr(self.dll, name)
+        fn = self.dll[name]                                       # a handle of its own, without the look at each argument
+        fn.restype = typed.restype
+        fn.argtypes = [ctypes.c_void_p if kind is _Pointer else kind for kind in typed.argtypes]
+        plain = []
+        for kind, a in zip(typed.argtypes, args, strict=True):
+            if isinstance(a, torch.Tensor):
+                a = a.data_ptr() if kind is _Pointer else a.item()
+            plain.append(a)
+        return fn, tuple(plain)
 
     def run(self, name: str, *args) -> None:
         """an entry point whose int result is a status: 0, or an error this raises with the library's message"""
-        status = getattr(self.dll, name)(*map(as_arg, args))
+        status = getattr(self.dll, name)(*args)
         if status:
             raise RuntimeError(f"{name}: launch failed (code {status}, {self.last_error()})")
