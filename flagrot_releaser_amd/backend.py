@@ -19,6 +19,7 @@ The transform-before-write variants of the reference are out of scope here.
 from __future__ import annotations
 
 import math
+import operator
 from dataclasses import dataclass
 
 import numpy as np
@@ -146,6 +147,11 @@ class RingGeometry:
         if p < S:
             return p
         return S + (p - S) % W if W > 0 else -1
+
+    def first_row(self, req, requests: int) -> int:
+        """first row of request row `req` in a flattened ring of `requests` request rows; the rules of an index: negative
+        ones count from the end, IndexError outside"""
+        return range(requests)[operator.index(req)] * self.slots
 
     def paged_tokens(self, L, out=None):
         """tokens of a length-L sequence that decode reads from pages: [S, L - W) with the sinks masked by kv_start,
@@ -340,10 +346,10 @@ class DecodeLayer:
     def prefill_chunk(self, kv, slots, req: int, start: int):
         """the next n tokens of request row `req`'s prompt, positions [start, start + n): every token to its page; the
         sinks among them and the newest W of the prompt so far also to the BF16 row"""
+        base = None if self.ring is None else self.geo.first_row(req, self.planner.spare + 1)
         self.write_pages(kv, slots)
         if self.ring is not None:
-            K.ring_rows(kv, self.ring, kmu=self.kmu, base=int(req) * self.geo.slots, sink=self.geo.S, window=self.geo.W,
-                        start=start)
+            K.ring_rows(kv, self.ring, kmu=self.kmu, base=base, sink=self.geo.S, window=self.geo.W, start=start)
 
     def update(self, kv, sp: StepPlan):
         """cache update of a decode step: the new tokens to their pages and to their BF16 slots"""
@@ -397,8 +403,9 @@ class KiviDecodeLayer:
     def prefill(self, kv, slots, req: int):
         """a fresh prompt of n tokens: values of every token, the whole key groups, sinks and newest W rows in BF16"""
         n = kv.shape[0]
+        base = self.geo.first_row(req, self.planner.spare + 1)
         KIVI.v_write(kv, slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
-        K.ring_rows(kv, self.ring, base=int(req) * self.geo.slots, sink=self.geo.S, window=self.geo.W)
+        K.ring_rows(kv, self.ring, base=base, sink=self.geo.S, window=self.geo.W)
         whole = n // GROUP
         if whole:
             rows = self._rows[:whole] if whole <= self._rows.shape[0] else self._rows_upto(whole)
@@ -413,14 +420,17 @@ class KiviDecodeLayer:
         """the next n tokens of request `req`'s prompt, positions [start, start + n): values of every token, the key
         groups the chunk completes (their earlier positions read from the ring, which therefore takes the chunk's own
         rows only afterwards), then the sinks and the newest W rows of the prompt so far in BF16"""
-        n = kv.shape[0]
+        n, start = kv.shape[0], operator.index(start)
+        if req < 0:                                        # (its groups' sources would not be ring rows)
+            raise IndexError(f"request row {req}")
+        base = self.geo.first_row(req, self.planner.spare + 1)
         KIVI.v_write(kv, slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
         flat = self.ring.view(-1, 2 * self.Hkv, D)
-        groups = chunk_key_groups(self.geo, start, n, req * self.geo.slots, table_row)
+        groups = chunk_key_groups(self.geo, start, n, base, table_row)
         if groups is not None:
             KIVI.k_encode(kv, groups[0], groups[1], self.qs, self.lz, self.scale, self.pool, self.Hkv, D, src2=flat,
                           f8=self.f8)
-        K.ring_rows(kv, self.ring, base=int(req) * self.geo.slots, sink=self.geo.S, window=self.geo.W, start=start)
+        K.ring_rows(kv, self.ring, base=base, sink=self.geo.S, window=self.geo.W, start=start)
 
     def update(self, kv, sp: StepPlan):
         KIVI.v_write(kv, sp.slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)

@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import operator
 import os
 
 import torch
@@ -415,8 +416,9 @@ def ring_rows(kv, ring, kmu=None, dest=None, base=0, sink=0, window=0, start=0):
         return
     assert kv.dtype == torch.bfloat16 and ring.dtype == torch.bfloat16 and ring.is_contiguous()
     rows = _loadable(kv)
+    base, start = operator.index(base), operator.index(start)
     if dest is None:
-        assert (base + sink + window) * heads * Dh <= ring.numel(), "the request's rows lie outside the ring"
+        assert 0 <= base and (base + sink + window) * heads * Dh <= ring.numel(), "the request's rows lie outside the ring"
     else:
         assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.numel() == T
     NATIVE.run("fr_ring_rows", rows, rows.stride(0), T, heads // 2, Dh, _centre(kmu, rows), ring, dest,

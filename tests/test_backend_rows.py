@@ -1,0 +1,75 @@
+"""Where a prompt's BF16 rows go (flagrot_releaser_amd.backend), on the CPU: the arguments that reach fr_ring_rows, with the
+launches themselves replaced."""
+import numpy as np
+import pytest
+import torch
+
+from flagrot_releaser_amd import backend as BK
+from flagrot_releaser_amd import kernels as K
+from flagrot_releaser_amd import kivi as KV
+
+S, W, R, HKV, G = 4, 32, 3, 2, 4                                      # R request rows and the spare one
+SLOTS = S + W
+
+
+@pytest.fixture
+def sent(monkeypatch):
+    """(base, start) of every fr_ring_rows call"""
+    calls = []
+    monkeypatch.setattr(K, "current_stream", lambda: 0)
+    monkeypatch.setattr(KV, "current_stream", lambda: 0)
+    monkeypatch.setattr(KV.NATIVE, "run", lambda name, *args: None)
+
+    def run(name, *args):
+        if name == "fr_ring_rows":
+            base, sink, window, start = args[8:12]
+            assert (sink, window) == (S, W) and type(base) is int and type(start) is int
+            calls.append((base, start))
+    monkeypatch.setattr(K.NATIVE, "run", run)
+    return calls
+
+
+def _layer(kind):
+    planner = BK.StepPlanner(kind, HKV, G, 256, 4, R, S, W, "cpu", plan_fn=lambda B: (1, 256))
+    if kind == "kivi2":
+        pool = torch.zeros(32, HKV, KV.chunk_bytes(128, False), dtype=torch.uint8)
+        return BK.KiviDecodeLayer(HKV, G, pool, planner, torch.zeros(HKV, 8, 128), torch.zeros(HKV, 8), torch.ones(HKV, 128))
+    pool = torch.zeros(32, HKV, K.v2_chunk_bytes(16, 128, kind), dtype=torch.uint8)
+    return BK.DecodeLayer(kind, HKV, G, pool, planner, wmask=torch.zeros(2 * HKV, 4, dtype=torch.uint8))
+
+
+def _chunk(layer, n, req, start):
+    kv, slots = torch.zeros(n, 2 * HKV, 128, dtype=torch.bfloat16), torch.arange(n)
+    extra = (torch.arange(16, dtype=torch.int32),) if isinstance(layer, BK.KiviDecodeLayer) else ()
+    layer.prefill_chunk(kv, slots, req, start, *extra)
+
+
+@pytest.mark.parametrize("kind", ["int4a", "kivi2"])
+@pytest.mark.parametrize("number", [int, np.int64, torch.tensor, lambda x: torch.tensor([x], dtype=torch.int32)])
+def test_positions_and_requests_in_any_integer_form(sent, kind, number):
+    layer = _layer(kind)
+    _chunk(layer, 40, number(2), number(37))
+    layer.prefill(torch.zeros(40, 2 * HKV, 128, dtype=torch.bfloat16), torch.arange(40), number(1))
+    assert sent == [(2 * SLOTS, 37), (SLOTS, 0)]
+
+
+@pytest.mark.parametrize("kind", ["int4a", "kivi2"])
+def test_request_rows_follow_the_rules_of_an_index(sent, kind):
+    layer = _layer(kind)
+    kv, slots = torch.zeros(5, 2 * HKV, 128, dtype=torch.bfloat16), torch.arange(5)
+    layer.prefill(kv, slots, -1)                                       # the spare row
+    layer.prefill(kv, slots, -R - 1)
+    assert sent == [(R * SLOTS, 0), (0, 0)]
+    for outside in (R + 1, -R - 2):
+        with pytest.raises(IndexError):
+            layer.prefill(kv, slots, outside)
+        with pytest.raises(IndexError):
+            _chunk(layer, 5, outside, 0)
+    with pytest.raises(TypeError):
+        layer.prefill(kv, slots, 1.0)
+    if kind == "kivi2":                                                # a chunk of these pages always refused negative rows
+        with pytest.raises(IndexError):
+            _chunk(layer, 5, -1, 0)
+    else:
+        _chunk(layer, 5, -1, 0)
+        assert sent[2:] == [(R * SLOTS, 0)]
