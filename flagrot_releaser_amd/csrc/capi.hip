@@ -199,12 +199,14 @@ int fr_v2_write(int fmt, const void* kv, long long kv_ts, const long long* slots
 }
 
 int fr_ring_rows(const void* kv, long long kv_ts, int T, int Hkv, int Dh, const float* kmu, void* ring, const long long* dest,
-                 long long base, int S, int W, int start, void* stream) {
+                 long long base, int S, int W, int start, void* stream, long long ring_rows) {
   if (T <= 0) return 0;
   if (Dh != 128 && Dh != 256) return fail(-8, "fr_ring_rows: head dim 128 | 256");
   if (S < 0 || W < 0 || start < 0) return fail(-3, "fr_ring_rows: bad ring geometry");
+  if (dest == nullptr && (base < 0 || base + S + W > ring_rows)) return fail(-3, "fr_ring_rows: the request's rows lie outside the ring");
   RingRowsParams p{};
-  p.kv = kv; p.kv_ts = kv_ts; p.width = 2 * Hkv * Dh; p.kmu = kmu; p.ring = ring; p.dest = dest; p.base = base;
+  p.kv = kv; p.kv_ts = kv_ts; p.width = 2 * Hkv * Dh; p.kmu = kmu; p.ring = ring; p.ring_rows = ring_rows; p.dest = dest;
+  p.base = base;
   p.S = S; p.W = W; p.start = start;
   if (dest != nullptr) p.rows = p.sinks = T;
   else {      // positions below S, and the newest W of the rest

@@ -45,7 +45,8 @@ struct RingRowsParams {
   int width;               // elements of a row: 2 * Hkv * head dim
   const float* kmu;        // [width / 2] subtracted from the key half, or null
   void* ring;              // bf16 [*, width]
-  const long long* dest;   // ring row of every token (< 0: skip), or null: the rule below
+  long long ring_rows;     // rows the ring has: no row outside [0, ring_rows) is written
+  const long long* dest;   // ring row of every token, or null: the rule below
   long long base;          // first ring row of the request
   int S, W, start;         // sinks, window, position of token 0
   int rows, sinks, win0;   // rows copied: tokens [0, sinks) and [win0, win0 + rows - sinks)

@@ -27,7 +27,7 @@ __global__ void __launch_bounds__(256) k_ring_rows(const RingRowsParams p) {
     const int pos = p.start + t;
     slot = p.base + (pos < p.S ? pos : p.S + (pos - p.S) % p.W);
   }
-  if (slot < 0) return;
+  if (slot < 0 || slot >= p.ring_rows) return;
   uint2 raw = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p.kv) + static_cast<long long>(t) * p.kv_ts + c);
   if (p.kmu != nullptr && c < p.width / 2) {
     const float4 m = *reinterpret_cast<const float4*>(p.kmu + c);

@@ -38,7 +38,7 @@ NOALLOC_MAX_PARTS = 8192     # FR_NOALLOC_MAX_PARTS of include/flagrot_kernels.h
 NATIVE = Library("kernels", "FLAGROT_LIB", "fr_abi_version", ABI, "fr_last_error", {
     "fr_v2_attn": "i p l p p i p i i i i i f p p i i i i i p p p p l p p p l l p i i",
     "fr_v2_write": "i p l p i i i p i p p i p",
-    "fr_ring_rows": "p l i i i p p p l i i i p",
+    "fr_ring_rows": "p l i i i p p p l i i i p l",
     "fr_v2_occupancy": "i i i i",
     "fr_v2_chunk_bytes": "i i",
     "fr_cb_nsg": "",
@@ -406,23 +406,26 @@ def cb_attn_noalloc(q, pool, block_table, seq_lens, out, nsplit, chunk, qscale, 
 
 
 def ring_rows(kv, ring, kmu=None, dest=None, base=0, sink=0, window=0, start=0):
-    """The BF16 rows a request keeps beside its pages: rows kv bf16 [T, 2 Hkv, Dh] into ring, a contiguous bf16 tensor of
-    rows of 2 Hkv Dh elements; kmu fp32 [Hkv, Dh] is subtracted from the keys (FP32, one rounding).  dest int64 [T] names
-    the ring row of every token (negative: skip).  Without it the tokens are positions start .. start + T - 1 of the
-    request whose ring starts at row `base`: positions below `sink` go to their own slot, the newest `window` of the rest
-    to slot sink + (p - sink) % window."""
+    """The BF16 rows a request keeps beside its pages: rows kv bf16 [T, 2 Hkv, Dh] into ring bf16 [..., 2 Hkv, Dh], contiguous;
+    kmu fp32 [Hkv, Dh] is subtracted from the keys (FP32, one rounding).  dest int64 [T] names the ring row of every token
+    (rows the ring does not have: skip).  Without it the tokens are positions start .. start + T - 1 of the request whose
+    ring starts at row `base`: positions below `sink` go to their own slot, the newest `window` of the rest to slot
+    sink + (p - sink) % window."""
     T, heads, Dh = kv.shape
     if T == 0:
         return
     assert kv.dtype == torch.bfloat16 and ring.dtype == torch.bfloat16 and ring.is_contiguous()
-    rows = _loadable(kv)
-    base, start = operator.index(base), operator.index(start)
+    assert ring.shape[-2:] == (heads, Dh) and heads % 2 == 0 and ring.device == kv.device and ring.data_ptr() % 8 == 0, \
+        "ring: rows of kv's shape, on its device, 8-byte aligned"
+    rows, have = _loadable(kv), ring.numel() // (heads * Dh)
     if dest is None:
-        assert 0 <= base and (base + sink + window) * heads * Dh <= ring.numel(), "the request's rows lie outside the ring"
+        base, start = operator.index(base), operator.index(start)
+        assert 0 <= base and base + sink + window <= have, "the request's rows lie outside the ring"
     else:
-        assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.numel() == T
+        assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.shape == (T,) and dest.device == kv.device, \
+            "dest: int64 [T], contiguous, on the rows' device"
     NATIVE.run("fr_ring_rows", rows, rows.stride(0), T, heads // 2, Dh, _centre(kmu, rows), ring, dest,
-               base, sink, window, start, current_stream())
+               base, sink, window, start, current_stream(), have)
 
 
 def head_fwht(x, flags, scale, out=None):

@@ -50,12 +50,13 @@ int fr_v2_write(int fmt, const void* kv, long long kv_ts, const long long* slots
 
 /* No counterpart in the reference, whose plugin uses torch operations (vllm_flagrot/attention/backend.py:1266-1325).  The
  * BF16 rows a request keeps beside its pages: rows kv bf16 [T, 2*Hkv, Dh] (token stride kv_ts elements, 8-byte aligned)
- * copied into ring bf16 [*, 2*Hkv, Dh], the key half minus kmu fp32 [Hkv, Dh] (or null) rounded to BF16 once.  dest int64
- * [T]: ring row of every token (< 0 skipped).  dest null: the tokens are positions start .. start + T - 1 of a request
- * with S sinks and a window of W in ring rows base ..; position p < S goes to base + p, one of the newest W of the others
- * to base + S + (p - S) % W, the rest is left out. */
+ * copied into ring bf16 [ring_rows, 2*Hkv, Dh], the key half minus kmu fp32 [Hkv, Dh] (or null) rounded to BF16 once.  dest
+ * int64 [T]: ring row of every token (tokens whose row is not in 0 .. ring_rows - 1 are skipped).  dest null: the tokens are
+ * positions start .. start + T - 1 of a request with S sinks and a window of W in ring rows base .. base + S + W - 1 (-3 if
+ * the ring does not have them); position p < S goes to base + p, one of the newest W of the others to
+ * base + S + (p - S) % W, the rest is left out. */
 int fr_ring_rows(const void* kv, long long kv_ts, int T, int Hkv, int Dh, const float* kmu, void* ring, const long long* dest,
-                 long long base, int S, int W, int start, void* stream);
+                 long long base, int S, int W, int start, void* stream, long long ring_rows);
 
 /* flagrot_capi.cu:79-80.  Resident 4-wavefront workgroups per CU (for the host split planner); bytes per (page, head)
  * chunk. */

@@ -73,3 +73,22 @@ def test_request_rows_follow_the_rules_of_an_index(sent, kind):
     else:
         _chunk(layer, 5, -1, 0)
         assert sent[2:] == [(R * SLOTS, 0)]
+
+
+def test_rows_that_do_not_fit_the_ring_are_refused(monkeypatch):
+    monkeypatch.setattr(K, "current_stream", lambda: 0)
+    monkeypatch.setattr(K.NATIVE, "run", lambda name, *args: None)
+    kv, dest = torch.zeros(3, 4, 128, dtype=torch.bfloat16), torch.arange(3)
+    ring = torch.zeros(6, 4, 128, dtype=torch.bfloat16)
+    K.ring_rows(kv, ring, dest=dest)
+    K.ring_rows(kv, ring, base=2, sink=1, window=3)
+    K.ring_rows(kv, ring.view(3, 2, 4, 128), dest=dest)
+    for bad in (dict(ring=torch.zeros(6, 6, 128, dtype=torch.bfloat16)), dict(ring=torch.zeros(6, 2, 256, dtype=torch.bfloat16)),
+                dict(ring=torch.zeros(6, 8, 64, dtype=torch.bfloat16)), dict(ring=ring[:, :2]), dict(ring=ring.float()),
+                dict(ring=ring.to("meta")), dict(ring=torch.zeros(6 * 512 + 1, dtype=torch.bfloat16)[1:].view(6, 4, 128)),
+                dict(dest=dest.int()), dict(dest=dest[:2]), dict(dest=dest.to("meta")), dict(dest=torch.zeros(6, dtype=torch.int64)[::2]),
+                dict(dest=None, base=-1, sink=1, window=3), dict(dest=None, base=3, sink=1, window=3),
+                dict(kv=kv.half()), dict(kv=kv[:, :3], ring=ring[:, :3].contiguous())):
+        args = {**dict(kv=kv, ring=ring, dest=dest), **bad}
+        with pytest.raises(AssertionError):
+            K.ring_rows(args.pop("kv"), args.pop("ring"), **args)

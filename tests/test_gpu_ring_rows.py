@@ -51,3 +51,22 @@ def test_named_rows(dev):
     K.ring_rows(kv.to(dev), ring, kmu=kmu.to(dev), dest=dest.to(dev))
     want = _want(ring0.clone(), kv, kmu, [(t, r) for t, r in enumerate(dest.tolist()) if r >= 0])
     assert torch.equal(ring.cpu(), want)
+
+
+@pytest.mark.parametrize("dim", [128, 256])
+@pytest.mark.parametrize("n", [1, 8, 9, 65])
+def test_named_rows_as_they_are(dev, n, dim):
+    """a decode step without centring; rows that the ring does not have are left out"""
+    from flagrot_releaser_amd import kernels as K
+    g = torch.Generator().manual_seed(n)
+    H, have = 2, 120
+    kv = torch.randn(n, 2 * H, dim, generator=g).bfloat16()
+    dest = torch.randperm(have, generator=g)[:n]
+    if n > 8:
+        dest[0], dest[3], dest[5], dest[8] = have, -1, 1 << 40, -(1 << 62)
+    ring0 = torch.randn(have, 2 * H, dim, generator=g).bfloat16()
+    room = torch.zeros(2 * have, 2 * H, dim, dtype=torch.bfloat16, device=dev)       # rows behind the ring must stay as they are
+    room[:have] = ring0.to(dev)
+    K.ring_rows(kv.to(dev), room[:have], dest=dest.to(dev))
+    want = _want(ring0.clone(), kv, None, [(t, r) for t, r in enumerate(dest.tolist()) if 0 <= r < have])
+    assert torch.equal(room[:have].cpu(), want) and not room[have:].any()
