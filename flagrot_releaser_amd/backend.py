@@ -188,15 +188,6 @@ def chunk_key_groups(geo: RingGeometry, start: int, n: int, ring_row0: int, tabl
     return src.contiguous(), dst.contiguous()
 
 
-def copy_ring_rows(kv, ring, dest, kmu=None):
-    """a decode step's rows to their BF16 slots.  Up to eight rows without centring take torch's copy: such steps wait for
-    the host, which it costs 5.5 us instead of 7.4; larger ones wait for the GPU, where it is the slower one by 1 us."""
-    if kmu is None and kv.shape[0] <= 8:
-        ring.index_copy_(0, dest, kv)
-    else:
-        K.ring_rows(kv, ring, kmu=kmu, dest=dest)
-
-
 @dataclass
 class StepPlan:
     """what one decode step of a batch needs on the device (views of the planner's persistent buffers)"""
@@ -355,7 +346,7 @@ class DecodeLayer:
         """cache update of a decode step: the new tokens to their pages and to their BF16 slots"""
         self.write_pages(kv, sp.slots)
         if self.ring is not None:
-            copy_ring_rows(kv, self.ring.view(-1, 2 * self.Hkv, D), sp.ring_dest, self.kmu)
+            K.ring_rows(kv, self.ring, kmu=self.kmu, dest=sp.ring_dest)
 
     def decode(self, q, sp: StepPlan, out):
         n = q.shape[0]
@@ -434,7 +425,7 @@ class KiviDecodeLayer:
 
     def update(self, kv, sp: StepPlan):
         KIVI.v_write(kv, sp.slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
-        copy_ring_rows(kv, self.ring, sp.ring_dest)
+        K.ring_rows(kv, self.ring, dest=sp.ring_dest)
         KIVI.k_encode(self.ring, sp.group_src, sp.group_dst, self.qs, self.lz, self.scale, self.pool, self.Hkv, D,
                       f8=self.f8)
 

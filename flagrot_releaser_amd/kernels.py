@@ -215,6 +215,8 @@ def _centre(kmu, kv):
 
 def _loadable(kv):
     """the writers read four bf16 at a time: heads and channels of a row must be dense, rows 8-byte aligned"""
+    if kv.is_contiguous() and kv.shape[2] % 4 == 0 and kv.data_ptr() % 8 == 0:
+        return kv
     dense = kv.stride(2) == 1 and kv.stride(1) == kv.shape[2]
     aligned = kv.stride(0) % 4 == 0 and kv.data_ptr() % 8 == 0
     return kv if dense and aligned else kv.contiguous()

@@ -27,8 +27,8 @@ class _Pointer:
     ctypes' own types: there a tensor of one element is its value and any other tensor an error, never an address."""
 
     @staticmethod
-    def from_param(a):
-        return ctypes.c_void_p.from_param(a.data_ptr() if isinstance(a, torch.Tensor) else a)
+    def from_param(a, address=ctypes.c_void_p.from_param, Tensor=torch.Tensor):
+        return address(a.data_ptr() if isinstance(a, Tensor) else a)
 
 
 _CTYPE = {"p": _Pointer, "i": ctypes.c_int, "l": ctypes.c_longlong, "f": ctypes.c_float}
@@ -45,6 +45,7 @@ class Library:
         never rebuilt); table: entry point -> signature string."""
         self.key, self.env, self.version_fn, self.abi, self.error_fn, self.table = key, env, version_fn, abi, error_fn, table
         self._dll = None
+        self._entry = {}                                          # name -> typed entry point, filled with the handle
 
     # -------------------------------------------------------------------------------------------- where, and how fresh
     @property
@@ -93,6 +94,7 @@ class Library:
                 args, _, ret = sig.partition("->")
                 fn.argtypes = [_CTYPE[c] for c in args.split()]
                 fn.restype = ctypes.c_char_p if ret.strip() == "s" else ctypes.c_int
+                self._entry[name] = fn
             self._dll = dll
         return self._dll
 
@@ -122,6 +124,7 @@ class Library:
 
     def run(self, name: str, *args) -> None:
         """an entry point whose int result is a status: 0, or an error this raises with the library's message"""
-        status = getattr(self.dll, name)(*args)
+        fn = self._entry.get(name) or getattr(self.dll, name)
+        status = fn(*args)
         if status:
             raise RuntimeError(f"{name}: launch failed (code {status}, {self.last_error()})")

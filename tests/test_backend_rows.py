@@ -29,8 +29,8 @@ def sent(monkeypatch):
     return calls
 
 
-def _layer(kind):
-    planner = BK.StepPlanner(kind, HKV, G, 256, 4, R, S, W, "cpu", plan_fn=lambda B: (1, 256))
+def _layer(kind, planner=None):
+    planner = planner or BK.StepPlanner(kind, HKV, G, 256, 4, R, S, W, "cpu", plan_fn=lambda B: (1, 256))
     if kind == "kivi2":
         pool = torch.zeros(32, HKV, KV.chunk_bytes(128, False), dtype=torch.uint8)
         return BK.KiviDecodeLayer(HKV, G, pool, planner, torch.zeros(HKV, 8, 128), torch.zeros(HKV, 8), torch.ones(HKV, 128))
@@ -92,3 +92,21 @@ def test_rows_that_do_not_fit_the_ring_are_refused(monkeypatch):
         args = {**dict(kv=kv, ring=ring, dest=dest), **bad}
         with pytest.raises(AssertionError):
             K.ring_rows(args.pop("kv"), args.pop("ring"), **args)
+
+
+@pytest.mark.parametrize("kind", ["int4a", "kivi2"])
+@pytest.mark.parametrize("n", [1, 8, 9])
+def test_steps_of_any_size_copy_their_rows_the_same_way(monkeypatch, kind, n):
+    """one launch with the planner's destinations, whatever the number of rows: one rule for rows outside the ring"""
+    calls = []
+    monkeypatch.setattr(K, "current_stream", lambda: 0)
+    monkeypatch.setattr(KV, "current_stream", lambda: 0)
+    monkeypatch.setattr(KV.NATIVE, "run", lambda name, *args: None)
+    monkeypatch.setattr(K.NATIVE, "run", lambda name, *args: calls.append((name, args)))
+    planner = BK.StepPlanner(kind, HKV, G, 256, 16, 15, S, W, "cpu", plan_fn=lambda B: (1, 256))
+    layer = _layer(kind, planner)
+    sp = planner.prepare(torch.full((n,), 50, dtype=torch.int32), torch.zeros(n, 16, dtype=torch.int32), torch.arange(n),
+                         homes=np.arange(n))
+    layer.update(torch.zeros(n, 2 * HKV, 128, dtype=torch.bfloat16), sp)
+    (args,) = [a for name, a in calls if name == "fr_ring_rows"]
+    assert args[2] == n and args[6] is layer.ring and args[7] is sp.ring_dest and args[13] == 16 * SLOTS
