@@ -481,9 +481,12 @@ __global__ void __launch_bounds__(512, 1) k_mq8(const Params p) {
 // A wavefront folds FOLD_ROWS consecutive query rows of a tile for one KV head, a lane per channel pair.  The items'
 // (maximum, sum) pairs are read one item per lane (64 at a time), so the common maximum, every item's weight
 // 2^(m - M) and the total sum come from three wave reductions instead of two serial passes; the accumulation loop then
-// takes each weight from its lane.  Tiles of a single item, and of up to FOLD_FEW items in launches short enough to be bound
-// by latency, need no lanes for that: the pairs of the wavefront's rows are neighbours in memory and the same for all lanes,
-// so they come by scalar loads, and the outputs of all rows and items are in flight together.
+// takes each weight from its lane.  Tiles of up to FOLD_FEW items need no lanes for that: the pairs of the wavefront's rows
+// are neighbours in memory and the same for all lanes, so they come by scalar loads, and the outputs of all rows and items
+// are in flight together.  Faster at every size (8 KV heads, us by lanes / this way, graph: 14 tiles of 256 rows x 128, 2
+// items 13.2 / 8.7; 64 tiles, 1 item 37.6 / 25.0, 2 items 45.2 / 28.6, 4 items 79 / 53; 128-row tiles x 256: 14 tiles, 2
+// items 11.6 / 7.2; 48 tiles, 4 items 35.1 / 36.7; 128 tiles, 2 items 92 / 62; the same order on partials that come from
+// memory).
 constexpr int FOLD_ROWS = 4, FOLD_FEW = 4;
 
 // W consecutive floats per lane: W = 2 covers a 128-d row with one wavefront, W = 4 a 256-d row
@@ -508,7 +511,7 @@ template <bool FP32_OUT, int W>
 __global__ void __launch_bounds__(256) k_fold_items(const int* __restrict__ tiles, const float* __restrict__ opart,
                                                     const float* __restrict__ ml, int Hkv, int G, int rows,
                                                     void* __restrict__ out, long long out_stride, float* __restrict__ lse,
-                                                    long long lse_stride, int few) {
+                                                    long long lse_stride) {
   const int lane = threadIdx.x & 63, head = blockIdx.y;
   const int* rec = tiles + TILE_INTS * blockIdx.x;
   const int first = rec[6], count = rec[7];
@@ -536,7 +539,7 @@ __global__ void __launch_bounds__(256) k_fold_items(const int* __restrict__ tile
     if (lse != nullptr && lane == 0)
       lse[qhead * lse_stride + rec[1] + token] = top == -INFINITY ? -INFINITY : (top + log2f(total)) * 0.6931471805599453f;
   };
-  if (count <= few && rows % FOLD_ROWS == 0) {                      // (rows past the last used one are read, not stored)
+  if (count <= FOLD_FEW && rows % FOLD_ROWS == 0) {                 // (rows past the last used one are read, not stored)
     if (row0 >= used) return;
     constexpr int DW = 64 * W;
     const long long at = (static_cast<long long>(first) * Hkv + head) * rows + row0;
@@ -862,10 +865,7 @@ int frmq_merge(const int* tiles, int ntiles, const float* opart, const float* ml
   hipStream_t st = static_cast<hipStream_t>(stream);
   const auto kern = Dh == 256 ? (out_fp32 ? k_fold_items<true, 4> : k_fold_items<false, 4>)
                               : (out_fp32 ? k_fold_items<true, 2> : k_fold_items<false, 2>);
-  // (launches of two rounds and more are bound by the bytes, which the lane-wise form streams a little faster: 8192 workgroups
-  // 21.6 against 25 us; 1792 workgroups 12.8 against 8.2)
-  const int few = static_cast<long long>(grid.x) * grid.y * grid.z <= 4096 ? FOLD_FEW : 1;
-  hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, tiles, opart, ml, Hkv, G, rows, out, o_ts, lse, lse_ts, few);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, tiles, opart, ml, Hkv, G, rows, out, o_ts, lse, lse_ts);
   return done(hipPeekAtLastError() == hipSuccess ? 0 : -1, "frmq_merge");
 }
 
