@@ -1,0 +1,74 @@
+"""The screened writer's workgroups of several 16-token steps: buffers in LDS are used again from step to step and the
+undecided tokens of all steps are evaluated at the end.  Whole-pool bytes against small calls, which run one workgroup per
+(token, head) and whose bytes the oracle pins in test_gpu_writers.py; exact ties, holes and odd rows lie in every step."""
+import os
+import subprocess
+import sys
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+# tokens x heads -> steps of a workgroup: 768 resident workgroups at head dim 128 (two steps from five on), 256 at 256 (at
+# most eight)
+SHAPES = [(128, 8, 2001, 2), (128, 8, 4000, 3), (128, 8, 5005, 4), (128, 8, 6203, 2), (256, 4, 2100, 3), (256, 4, 8201, 8)]
+
+
+def steps_of(D, Hkv, T):
+    resident = 768 if D == 128 else 256
+    fit = -(-(-(-T // 16)) * Hkv // resident)
+    return 2 if D == 128 and fit > 4 else min(fit, 8)
+
+
+def check(kind, D, Hkv, T, page, first=5):
+    from flagrot_releaser_amd import kernels as K
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(T + page)
+    kv = torch.randn(T, 2 * Hkv, D, generator=g)
+    kv[:, :Hkv, 5] *= 7
+    kv *= 0.5 + torch.rand(T, 1, 1, generator=g)
+    t = torch.arange(T)
+    kv[t % 13 == 4] = 0.0                                  # every candidate reproduces the row: undecided
+    kv[t % 37 == 9] = kv[9:10].clone()                     # one token repeated
+    kv[t % 29 == 3] = 0.37                                 # constants
+    kv[t % 17 == 6, :, 32:64] = 0.0                        # a tie in one group only
+    kv[t % 41 == 11] *= 1e-4
+    kv[t % 23 == 2, :, 64:96] *= 500.0
+    qs = torch.randn(Hkv, 256, D, generator=g)
+    qs[:, :, :8] *= 4
+    CT = (qs.transpose(1, 2) @ qs / 256).transpose(1, 2).contiguous().to(dev)
+    co = torch.ones(Hkv, D, device=dev)
+    kv = kv.bfloat16().to(dev)
+    slots = first + t
+    slots[t >= T // 2] += 3                                # a second run of slots
+    slots[t % 19 == 8] = -1
+    slots = slots.to(dev)
+    npg = (T + first + 3) // page + 2
+    pool = torch.randint(0, 256, (npg, Hkv, K.v2_chunk_bytes(page, D, kind)), dtype=torch.uint8, generator=g).to(dev)
+    want, got = pool.clone(), pool.clone()
+    small = 1024 // Hkv
+    for a in range(0, T, small):
+        K.cb_write(kv[a:a + small], slots[a:a + small].contiguous(), CT, co, kind, want, page)
+    if D == 128:
+        K.cb_write3(kv, slots, CT, co, None, None, kind, got, page, split=False)
+    else:
+        K.cb_write(kv, slots, CT, co, kind, got, page)
+    assert torch.equal(got, want), (kind, D, T, page, int((got != want).sum()))
+
+
+@pytest.mark.parametrize("kind", ["konly", "konlya", "konlya2"])
+@pytest.mark.parametrize("page", [16, 32])
+@pytest.mark.parametrize("D,Hkv,T,steps", SHAPES)
+def test_steps_write_the_bytes_of_small_calls(dev, kind, D, Hkv, T, steps, page):
+    assert steps_of(D, Hkv, T) == steps
+    check(kind, D, Hkv, T, page)
+
+
+def test_every_token_exact(dev):
+    """FLAGROT_W3=2 (read once per process): every token takes the exact path at the end, full lists of undecided tokens"""
+    code = ("from tests.test_gpu_writer_steps import check\n"
+            "check('konlya', 128, 8, 4000, 16); check('konlya2', 256, 4, 8201, 32)\nprint('same bytes')\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env={**os.environ, "FLAGROT_W3": "2"}, capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0 and "same bytes" in r.stdout, r.stdout + r.stderr
