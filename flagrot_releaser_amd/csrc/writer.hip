@@ -383,9 +383,9 @@ int k2_write_launch(int kind, const K2WriteParams& p, hipStream_t st) {
   }
   return -4;
 }
-int k2_write_lds_bytes(int hd) {      // what fr_cb_write_smem reports: C_q^T and error strips; 256-d heads: error strips
-  return hd == 256 ? static_cast<int>(8 * 2 * 256 * sizeof(float)) : K2_LDS;
-}
+// what fr_cb_write_smem reports, the most LDS a workgroup of fr_cb_write takes: 128-d heads C_q^T and error strips (this
+// file), 256-d heads the screened kernel (the decode step's takes less in both)
+int k2_write_lds_bytes(int hd) { return hd == 256 ? k2_screen_lds_bytes(256) : K2_LDS; }
 
 int head_fwht_launch(const void* x, long long x_ts, void* out, long long o_ts, int T, int H, const uint8_t* flags,
                      float scale, hipStream_t st, int D) {

@@ -47,8 +47,8 @@ DEVI void head_transform(float (&y)[4], int lane) {
 }
 
 // ---- value codes of up to 64 tokens, word by word
-// The eight tokens of an aligned run of slots share V^T words.  `lead` lists the runs that the N tokens (slots in LDS,
-// negative: none) touch: the first slot of the run and, a byte per position, which token holds it (0xFF: none of these).
+// The eight tokens of an aligned run of slots share V^T words.  VRuns: the n runs that the N tokens (slots in LDS, negative:
+// none) touch, of each the first slot and, a byte per position, which token holds it (0xFF: none of these).
 template <int N>
 struct VRuns {
   long long first[N];

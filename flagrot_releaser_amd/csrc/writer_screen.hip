@@ -338,5 +338,6 @@ int k2_screen_launch(int kind, const K2WriteParams& p, bool all_exact, hipStream
   }
   return -4;
 }
+int k2_screen_lds_bytes(int hd) { return static_cast<int>(hd == 256 ? sizeof(ScreenSmem<256>) : sizeof(ScreenSmem<128>)); }
 
 }  // namespace fr

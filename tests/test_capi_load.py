@@ -170,3 +170,13 @@ def test_decode_front_end_rejects_a_pool_of_another_page_size():
         K.v2_attn(q, pool32, bt, lens, out, 1, 64, None, 1.0, fmt="int4a")
     with pytest.raises(AssertionError, match="not pages of 16 tokens"):
         K.cb_attn_noalloc(q, pool32, bt, lens, out, 1, 64, 1.0, "konlya")
+
+
+def test_writer_lds_covers_the_kernels_that_run():
+    """fr_cb_write_smem: at least C_q^T of a 128-d head; at head dim 256 the error vectors of a 16-token step (3 candidates, two
+    BF16 terms) and the candidates' codes"""
+    from flagrot_releaser_amd import kernels
+    smem = kernels.lib().fr_cb_write_smem
+    assert smem(10, 1, 128) >= 128 * 128 * 4
+    assert 16 * 3 * 256 * (2 * 2 + 1) <= smem(10, 1, 256) <= 160 * 1024
+    assert smem(10, 1, 64) == 0
