@@ -225,6 +225,17 @@ class StepPlanner:
         if kind == "kivi2":
             self._group = torch.full((2, max_rows, GROUP), -1, dtype=torch.int64, device=device)
             self._lane = torch.arange(GROUP, dtype=torch.int64, device=device)
+            self._rows = self._rows_upto(max_len // GROUP)
+
+    def _rows_upto(self, groups: int):
+        pos = torch.arange(groups * GROUP, device=self._dest.device)
+        return pos.masked_fill_(pos < self.geo.S, -1).view(-1, GROUP)
+
+    def prompt_groups(self, groups: int):
+        """kivi2: sources of the first `groups` key groups of a prompt, int64 [groups, 32]: the tokens' own rows, -1 for the
+        sinks (they stay BF16 only).  One table for all layers, made with the planner (a first prompt may come under
+        capture or on another stream); prompts past max_len make their own."""
+        return self._rows[:groups] if groups <= self._rows.shape[0] else self._rows_upto(groups)
 
     def plan(self, B: int):
         b = plan_bucket(B)
@@ -388,8 +399,6 @@ class KiviDecodeLayer:
         dev = pool.device
         self.ring = torch.zeros((planner.spare + 1) * self.geo.slots, 2 * Hkv, D, dtype=torch.bfloat16, device=dev)
         self.ws = kivi_workspace(dev, planner.max_rows, Hkv, G, D, planner.plan)
-        # row of every token of a prompt's key groups, -1 for the sinks (they stay BF16 only)
-        self._rows = self._rows_upto(planner.max_len // GROUP)
 
     def prefill(self, kv, slots, req: int):
         """a fresh prompt of n tokens: values of every token, the whole key groups, sinks and newest W rows in BF16"""
@@ -399,13 +408,8 @@ class KiviDecodeLayer:
         K.ring_rows(kv, self.ring, base=base, sink=self.geo.S, window=self.geo.W)
         whole = n // GROUP
         if whole:
-            rows = self._rows[:whole] if whole <= self._rows.shape[0] else self._rows_upto(whole)
-            KIVI.k_encode(kv, rows, slots[:whole * GROUP].view(whole, GROUP).contiguous(), self.qs,
+            KIVI.k_encode(kv, self.planner.prompt_groups(whole), slots[:whole * GROUP].view(whole, GROUP).contiguous(), self.qs,
                           self.lz, self.scale, self.pool, self.Hkv, D, f8=self.f8)
-
-    def _rows_upto(self, groups: int):
-        pos = torch.arange(groups * GROUP, device=self.pool.device)
-        return pos.masked_fill_(pos < self.geo.S, -1).view(-1, GROUP)
 
     def prefill_chunk(self, kv, slots, req: int, start: int, table_row):
         """the next n tokens of request `req`'s prompt, positions [start, start + n): values of every token, the key

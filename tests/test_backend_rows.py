@@ -110,3 +110,21 @@ def test_steps_of_any_size_copy_their_rows_the_same_way(monkeypatch, kind, n):
     layer.update(torch.zeros(n, 2 * HKV, 128, dtype=torch.bfloat16), sp)
     (args,) = [a for name, a in calls if name == "fr_ring_rows"]
     assert args[2] == n and args[6] is layer.ring and args[7] is sp.ring_dest and args[13] == 16 * SLOTS
+
+
+def test_layers_share_the_rows_of_a_prompt_s_key_groups(monkeypatch):
+    """int64 rows 0 .. of every whole group, sinks left out: one table per planner, not one per layer"""
+    sent = []
+    monkeypatch.setattr(K, "current_stream", lambda: 0)
+    monkeypatch.setattr(KV, "current_stream", lambda: 0)
+    monkeypatch.setattr(K.NATIVE, "run", lambda name, *args: None)
+    monkeypatch.setattr(KV.NATIVE, "run", lambda name, *args: sent.append(args[4]) if name == "kv_k_encode" else None)
+    planner = BK.StepPlanner("kivi2", HKV, G, 256, 4, R, S, W, "cpu", plan_fn=lambda B: (1, 256))
+    for n in (70, 256, 300):                                          # past max_len the last two hold what the first do
+        for layer in (_layer("kivi2", planner), _layer("kivi2", planner)):
+            layer.prefill(torch.zeros(n, 2 * HKV, 128, dtype=torch.bfloat16), torch.arange(n), 0)
+        a, b = sent[-2:]
+        want = torch.arange(n // 32 * 32)
+        want[:S] = -1
+        assert torch.equal(a, want.view(-1, 32)) and torch.equal(a, b) and a.dtype == torch.int64 and a.is_contiguous()
+        assert n > 256 or a.data_ptr() == b.data_ptr()
