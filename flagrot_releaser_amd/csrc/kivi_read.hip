@@ -5,8 +5,9 @@
 // A lane owns eight channels of a row (16 bytes of BF16), so a sub-vector lies on four lanes and a rotation exchanges
 // twice between neighbours instead of three times; code x step is exact, so that and the minimum are one instruction.  The
 // KV heads of a group are neighbours in dispatch order: together they write whole tokens (2 KB and more in one piece).
-// Bound by vector issue before (four channels a lane, 2-byte stores, heads outermost).  32640 tokens x 8 heads, 24 MB in and
-// 134 MB out: kernel 41 -> 34 us (4.6 TB/s, what a large copy reaches), the call on cold pages 59 -> 50 us.
+// Bound by vector issue (20.1 M instructions a launch of 32640 tokens x 8 heads: 81 k of a SIMD's 82 k cycles) and as much by
+// its 24 MB in and 134 MB out: kernel 41 -> 34 us (4.6 TB/s, what a large copy reaches), the call on cold pages 59 -> 50 us
+// (before: four channels a lane, 2-byte stores, heads outermost).
 #include "fr_common.hpp"
 #include "kivi_launch.hpp"
 #include "kivi_quant.hpp"

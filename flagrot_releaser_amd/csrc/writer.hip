@@ -373,7 +373,10 @@ int k2_write_launch(int kind, const K2WriteParams& p, hipStream_t st) {
   static const bool no_step = getenv("FLAGROT_WRITER_LL") != nullptr && getenv("FLAGROT_WRITER_LL")[0] == '0';
   if (!(no_step && p.hd != 256) && pairs <= 1024) return k2_step_launch(kind, p, st);
   // Prompt-sized key passes: choices screened on the matrix pipe (FLAGROT_W3: 0 off for 128-d heads, 2 every token exact).
-  // At 1024 pairs the two forms cost the same: 256-d heads 25 us by tokens, 2048 pairs 49 by tokens against 34-40.
+  // us by tokens / screened at 768, 1024, 1280, 1536, 2048 pairs: 4 heads of 256 23 / 31, 28 / 28, 33 / 31, 38 / 28, 49 / 28;
+  // 8 heads of 128 on 4-bit pages 11.0 / 17.3, 13.5 / 17.4, 15.6 / 17.3, 17.2 / 17.3, 20.8 / 17.5, on 2-bit pages 12.0 / 17.7,
+  // 15.3 / 17.7, 16.6 / 20.1, 18.5 / 17.8, 22.9 / 17.9.  So the lines lie at 1024 and near 1500; one rule serves both, which
+  // costs 128-d heads at most 3 us in between.
   static const int w3mode = getenv("FLAGROT_W3") != nullptr ? atoi(getenv("FLAGROT_W3")) : 1;
   if (p.hd == 256 || (w3mode != 0 && p.screen && (p.passes & 1) && pairs > 1024)) return k2_screen_launch(kind, p, w3mode == 2, st);
   switch (kind) {
