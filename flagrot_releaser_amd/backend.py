@@ -324,7 +324,8 @@ class DecodeLayer:
         self.ws = decode_workspace(dev, tile_layout(kind, Hkv, G), planner.max_rows, planner.plan)
 
     def center_rows(self, kv):
-        """what the BF16 slots hold: key rows with the static mean removed (fp32 subtraction, one bf16 rounding)"""
+        """what the BF16 slots hold, in torch operations: key rows with the static mean removed (fp32 subtraction, one bf16
+        rounding).  For programs that fill a ring themselves; the layer's own copies do this in K.ring_rows."""
         if self.kmu is None:
             return kv
         H = self.Hkv
