@@ -65,10 +65,13 @@ def test_steps_write_the_bytes_of_small_calls(dev, kind, D, Hkv, T, steps, page)
     check(kind, D, Hkv, T, page)
 
 
-def test_every_token_exact(dev):
-    """FLAGROT_W3=2 (read once per process): every token takes the exact path at the end, full lists of undecided tokens"""
+@pytest.mark.parametrize("env", [{"FLAGROT_W3": "2"}, {"FLAGROT_W3_KAPPA": "0.1"}], ids=["every token exact", "a tenth of the bound"])
+def test_screen_at_its_ends(dev, env):
+    """FLAGROT_W3=2: every token takes the exact path at the end, full lists of undecided tokens.  FLAGROT_W3_KAPPA=0.1: the
+    estimates decide on a tenth of their proven bound, matrix pipe included, and no choice changes (measured: none down to a
+    hundredth of it on these rows, the first at three thousandths).  Both are read once per process."""
     code = ("from tests.test_gpu_writer_steps import check\n"
             "check('konlya', 128, 8, 4000, 16); check('konlya2', 256, 4, 8201, 32)\nprint('same bytes')\n")
-    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env={**os.environ, "FLAGROT_W3": "2"}, capture_output=True,
-                       text=True, timeout=100)
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env={**os.environ, **env}, capture_output=True, text=True,
+                       timeout=100)
     assert r.returncode == 0 and "same bytes" in r.stdout, r.stdout + r.stderr
