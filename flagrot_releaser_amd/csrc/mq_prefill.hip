@@ -20,6 +20,7 @@
 // :789-823 (q preparation), :1350-1465 (BF16 window gather / sink merge), :1469-1601 (C ABI).
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 
 #include "../../include/flagrot_mq.h"
 #include "fr_common.hpp"
@@ -480,14 +481,19 @@ __global__ void __launch_bounds__(512, 1) k_mq8(const Params p) {
 // ------------------------------------------------------------------------------------------------ items of a tile, folded
 // A wavefront folds FOLD_ROWS consecutive query rows of a tile for one KV head, a lane per channel pair.  The items'
 // (maximum, sum) pairs are read one item per lane (64 at a time), so the common maximum, every item's weight
-// 2^(m - M) and the total sum come from three wave reductions instead of two serial passes; the accumulation loop then
-// takes each weight from its lane.  Tiles of up to FOLD_FEW items need no lanes for that: the pairs of the wavefront's rows
-// are neighbours in memory and the same for all lanes, so they come by scalar loads, and the outputs of all rows and items
-// are in flight together.  Faster at every size (8 KV heads, us by lanes / this way, graph: 14 tiles of 256 rows x 128, 2
-// items 13.2 / 8.7; 64 tiles, 1 item 37.6 / 25.0, 2 items 45.2 / 28.6, 4 items 79 / 53; 128-row tiles x 256: 14 tiles, 2
-// items 11.6 / 7.2; 48 tiles, 4 items 35.1 / 36.7; 128 tiles, 2 items 92 / 62; the same order on partials that come from
-// memory).
-constexpr int FOLD_ROWS = 4, FOLD_FEW = 4;
+// 2^(m - M) and the total sum come from three wave reductions instead of two serial passes; the accumulation takes each
+// weight from its lane and has 16 outputs (rows x items) in flight whatever the weights are -- a load behind a test of its
+// weight is a memory round trip per item and row (8 KV heads of 128 rows, 1 tile of 19 items: 38 us; now 7).  Tiles of up to
+// FOLD_FEW items need no lanes for that: the pairs of the wavefront's rows are neighbours in memory and the same for all
+// lanes, so they come by scalar loads, and the outputs of all rows and items are in flight together.  Faster at every size
+// (8 KV heads, us by lanes / this way, graph: 14 tiles of 256 rows x 128, 2 items 13.2 / 8.7; 64 tiles, 1 item 37.6 / 25.0, 2
+// items 45.2 / 28.6; 128-row tiles x 256: 14 tiles, 2 items 11.6 / 7.2; 128 tiles, 2 items 92 / 62).
+// Launches of fewer than FOLD_SHORT rows leave CUs idle with four rows a wavefront and take one, with four times the items
+// in flight (us by fours / by ones, 8 KV heads x 128: 1024 rows of 1 / 8 / 70 items 3.2 / 2.1, 6.3 / 4.3, 24.5 / 12.2; 4096 rows
+// of 8 / 70 7.5 / 6.4, 37.0 / 32.0; 8192 rows of 1 / 5 / 20 3.9 / 3.9, 8.5 / 9.2, 19.1 / 22.2; x 256: 2048 rows of 8 items 8.3 / 6.4,
+// 6144 14.6 / 13.3, 16384 of 5 22.1 / 24.6).
+constexpr int FOLD_SHORT = 8192;
+constexpr int FOLD_FEW = 4;
 
 // W consecutive floats per lane: W = 2 covers a 128-d row with one wavefront, W = 4 a 256-d row
 template <int W> DEVI void ldw(const float* p, float (&x)[W]) {
@@ -507,11 +513,12 @@ template <int W> DEVI void stw_bf16(uint16_t* p, const float (&x)[W]) {
   else *reinterpret_cast<uint2*>(p) = make_uint2(bf16_rn(x[0]) | (bf16_rn(x[1]) << 16), bf16_rn(x[2]) | (bf16_rn(x[3]) << 16));
 }
 
-template <bool FP32_OUT, int W>
+template <bool FP32_OUT, int W, int FOLD_ROWS>
 __global__ void __launch_bounds__(256) k_fold_items(const int* __restrict__ tiles, const float* __restrict__ opart,
                                                     const float* __restrict__ ml, int Hkv, int G, int rows,
                                                     void* __restrict__ out, long long out_stride, float* __restrict__ lse,
                                                     long long lse_stride) {
+  constexpr int FOLD_STEP = 16 / FOLD_ROWS;                              // items at a time: 16 outputs in flight
   const int lane = threadIdx.x & 63, head = blockIdx.y;
   const int* rec = tiles + TILE_INTS * blockIdx.x;
   const int first = rec[6], count = rec[7];
@@ -575,41 +582,57 @@ __global__ void __launch_bounds__(256) k_fold_items(const int* __restrict__ tile
     }
     return;
   }
+  if (row0 >= used) return;
+  constexpr int DW = 64 * W;                                             // the head dim
+  int row[FOLD_ROWS];                                                    // (rows past the last used one: that one again, not stored)
+  float top[FOLD_ROWS], total[FOLD_ROWS], sum[FOLD_ROWS][W];
+  const long long at = (static_cast<long long>(first) * Hkv + head) * rows;
 #pragma unroll
   for (int i = 0; i < FOLD_ROWS; ++i) {
-    const int row = row0 + i;
-    if (row >= used) break;                                              // wave uniform
-    constexpr int DW = 64 * W;                                           // the head dim
-    const long long at = (static_cast<long long>(first) * Hkv + head) * rows + row;
-    float sum[W];
+    row[i] = min(row0 + i, used - 1);
+    top[i] = -INFINITY; total[i] = 0.f;
 #pragma unroll
-    for (int k = 0; k < W; ++k) sum[k] = 0.f;
-    float top, total;
-    top = -INFINITY; total = 0.f;
-    for (int s0 = 0; s0 < count; s0 += 64)
-      top = fmaxf(top, wave_max64(s0 + lane < count ? ml[2 * (at + (s0 + lane) * per_item)] : -INFINITY));
-    if (top != -INFINITY) {
-      for (int s0 = 0; s0 < count; s0 += 64) {
-        float weight = 0.f, mass = 0.f;
-        if (s0 + lane < count) {
-          const float2 st = *reinterpret_cast<const float2*>(ml + 2 * (at + (s0 + lane) * per_item));
-          weight = st.x == -INFINITY ? 0.f : fexp2(st.x - top);
-          mass = weight * st.y;
-        }
-        total += wave_sum64(mass);
-        const int n = min(64, count - s0);
-        for (int s = 0; s < n; ++s) {
-          const float w = __shfl(weight, s, 64);
-          if (w == 0.f) continue;                                      // an item that saw no key: nothing to read
-          float x[W];
-          ldw<W>(opart + (at + (s0 + s) * per_item) * DW + W * lane, x);
-#pragma unroll
-          for (int k = 0; k < W; ++k) sum[k] += w * x[k];
-        }
-      }
-    }
-    store(row, sum, top, total);
+    for (int k = 0; k < W; ++k) sum[i][k] = 0.f;
   }
+  auto pair = [&](int s, int i) {                                        // item s of the row, nothing past the last item
+    return s < count ? *reinterpret_cast<const float2*>(ml + 2 * (at + s * per_item + row[i])) : make_float2(-INFINITY, 0.f);
+  };
+  for (int s0 = 0; s0 < count; s0 += 64)
+#pragma unroll
+    for (int i = 0; i < FOLD_ROWS; ++i) top[i] = fmaxf(top[i], pair(s0 + lane, i).x);
+#pragma unroll
+  for (int i = 0; i < FOLD_ROWS; ++i) top[i] = wave_max64(top[i]);
+  for (int s0 = 0; s0 < count; s0 += 64) {
+    float weight[FOLD_ROWS];
+#pragma unroll
+    for (int i = 0; i < FOLD_ROWS; ++i) {
+      const float2 st = pair(s0 + lane, i);
+      weight[i] = st.x == -INFINITY ? 0.f : fexp2(st.x - top[i]);
+      total[i] += wave_sum64(weight[i] * st.y);
+    }
+    const int n = min(64, count - s0);
+    for (int g = 0; g < n; g += FOLD_STEP) {
+      float x[FOLD_STEP][FOLD_ROWS][W];
+#pragma unroll
+      for (int j = 0; j < FOLD_STEP; ++j)
+#pragma unroll
+        for (int i = 0; i < FOLD_ROWS; ++i)
+          ldw<W>(opart + (at + (s0 + min(g + j, n - 1)) * per_item + row[i]) * DW + W * lane, x[j][i]);
+#pragma unroll
+      for (int j = 0; j < FOLD_STEP; ++j)
+#pragma unroll
+        for (int i = 0; i < FOLD_ROWS; ++i) {
+          // (weights of lanes past the last item are 0; an item that saw no key stored no outputs)
+          const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight[i]), g + j));
+          if (w == 0.f) continue;
+#pragma unroll
+          for (int k = 0; k < W; ++k) sum[i][k] += w * x[j][i][k];
+        }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < FOLD_ROWS; ++i)
+    if (row0 + i < used) store(row0 + i, sum[i], top[i], total[i]);
 }
 
 // ------------------------------------------------------------------------------------------------ query rows for the kernel
@@ -861,11 +884,16 @@ int frmq_merge(const int* tiles, int ntiles, const float* opart, const float* ml
                long long o_ts, int out_fp32, float* lse, long long lse_ts, int Dh, void* stream) {
   if (ntiles <= 0) return 0;
   if (Dh != D && Dh != 256) return bad(-4, "frmq_merge: head dim 128 or 256");
-  const dim3 grid(ntiles, Hkv, (rows + 4 * FOLD_ROWS - 1) / (4 * FOLD_ROWS));      // four wavefronts x FOLD_ROWS rows per workgroup
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const auto kern = Dh == 256 ? (out_fp32 ? k_fold_items<true, 4> : k_fold_items<false, 4>)
-                              : (out_fp32 ? k_fold_items<true, 2> : k_fold_items<false, 2>);
-  hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, tiles, opart, ml, Hkv, G, rows, out, o_ts, lse, lse_ts);
+  auto go = [&](auto per_wave) {
+    constexpr int R = decltype(per_wave)::value;
+    const auto kern = Dh == 256 ? (out_fp32 ? k_fold_items<true, 4, R> : k_fold_items<false, 4, R>)
+                                : (out_fp32 ? k_fold_items<true, 2, R> : k_fold_items<false, 2, R>);
+    hipLaunchKernelGGL(kern, dim3(ntiles, Hkv, (rows + 4 * R - 1) / (4 * R)), dim3(256), 0, st, tiles, opart, ml, Hkv, G, rows,
+                       out, o_ts, lse, lse_ts);
+  };
+  if (static_cast<long long>(ntiles) * Hkv * rows < FOLD_SHORT) go(std::integral_constant<int, 1>{});
+  else go(std::integral_constant<int, 4>{});
   return done(hipPeekAtLastError() == hipSuccess ? 0 : -1, "frmq_merge");
 }
 

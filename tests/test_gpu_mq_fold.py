@@ -10,10 +10,19 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("Dh,rows,G,N", [(128, 256, 8, 3), (128, 256, 4, 130), (128, 128, 3, 9), (128, 64, 5, 7), (256, 128, 6, 4),
                                          (256, 128, 4, 260)])
 def test_fold_of_items(dev, Dh, rows, G, N, fp32):
+    fold_check(dev, Dh, rows, G, N, fp32, [1 + (5 * i) % 6 for i in range(N)])
+
+
+# below and above 8192 rows in the launch (one or four rows a wavefront); items around a step of 4 or 16 and around 64 lanes
+@pytest.mark.parametrize("Dh,rows,G,N", [(128, 128, 1, 9), (128, 256, 3, 17), (256, 128, 5, 9), (256, 128, 1, 33)])
+def test_fold_of_many_items(dev, Dh, rows, G, N):
+    fold_check(dev, Dh, rows, G, N, True, [(5, 15, 16, 17, 18, 63, 64, 65, 70)[i % 9] for i in range(N)])
+
+
+def fold_check(dev, Dh, rows, G, N, fp32, counts):
     from flagrot_releaser_amd import prefill_mq as MQ
     Hkv, per = 2, rows // G
     g = torch.Generator(device=dev).manual_seed(N)
-    counts = [1 + (5 * i) % 6 for i in range(N)]
     tokens = [per - (i % 3 if i % 2 else 0) for i in range(N)]
     T = torch.zeros(N, 9, dtype=torch.int32)
     T[:, 1] = T[:, 2] = torch.tensor([0] + tokens[:-1]).cumsum(0)
@@ -42,7 +51,7 @@ def test_fold_of_items(dev, Dh, rows, G, N, fp32):
         safe = torch.where(seen, total, torch.ones_like(total))
         mean, size = (w[..., None] * x).sum(0) / safe[..., None], (w[..., None] * x.abs()).sum(0) / safe[..., None]
         mine = got[row0:row0 + tokens[i]].permute(1, 0, 2, 3).reshape(Hkv, used, Dh)
-        # FP32: exponents to 40 x 2^-24, a dozen roundings of 2^-24; BF16: half a unit of the result on top
+        # FP32: exponents to 40 x 2^-24, a dozen roundings of 2^-24 (70 items: their weights fall off, no more of them count); BF16: half a unit of the result on top
         bar = 4e-6 * size + (0 if fp32 else 2.0 ** -8 * mean.abs()) + 1e-30
         assert ((mine - mean).abs() <= bar).all(), (i, counts[i], float(((mine - mean).abs() / bar).max()))
         mine = lse[:, :, row0:row0 + tokens[i]].permute(0, 2, 1).reshape(Hkv, used).double()
