@@ -79,7 +79,7 @@ int kv_attn(const void* q, long long q_rs, const void* pool, const void* bt, lon
   const int rc = attn_splits_launch(G, q, q_rs, pool, bt, bt_rs, cached, kv_start, B, Hkv, NS, chunk, qscale, ring, tail_len,
                                     tail_idx, T, opart, ml, f8 & 1, st);
   if (rc) return launched(rc, "kv_attn");
-  hipLaunchKernelGGL(k_merge_parts<128>, dim3(B, Hkv * G), dim3(128), 0, st, static_cast<const float*>(opart), static_cast<const float*>(ml),
+  hipLaunchKernelGGL(k_merge_parts<128>, dim3(B, Hkv * G), dim3(MERGE_SLICES * 32), 0, st, static_cast<const float*>(opart), static_cast<const float*>(ml),
                      Hkv, G, NS, static_cast<uint16_t*>(out), out_rs);
   return launched(hipPeekAtLastError() == hipSuccess ? 0 : 1, "kv_attn (merge)");
 }

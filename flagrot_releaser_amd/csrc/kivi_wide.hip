@@ -392,7 +392,7 @@ int attn256_launch(int G, const void* q, long long q_rs, const void* pool, const
                                         tail_idx, T, opart, ml, f8, st);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_merge_parts<D2>, dim3(B, Hkv * G), dim3(256), 0, st, static_cast<const float*>(opart), static_cast<const float*>(ml),
+  hipLaunchKernelGGL(k_merge_parts<D2>, dim3(B, Hkv * G), dim3(MERGE_SLICES * 64), 0, st, static_cast<const float*>(opart), static_cast<const float*>(ml),
                      Hkv, G, NS, static_cast<uint16_t*>(out), out_rs);
   return hipPeekAtLastError() == hipSuccess ? 0 : 1;
 }
