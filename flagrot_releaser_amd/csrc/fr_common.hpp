@@ -68,9 +68,11 @@ DEVI void butterflies(float (&x)[4], int l32) {
   }
 #pragma unroll
   for (int lm = 1; lm < N / 4; lm <<= 1) {
-    const uint32_t flip = (l32 & lm) ? 0x80000000u : 0u;        // upper lane: other - own, as other + (-own)
+    // upper lane: other - own, as own x (-1) + other with ONE rounding: the same number, and one instruction beside an
+    // exchange through LDS (distances 4 and 16) instead of a sign flip and an addition
+    const float sign = (l32 & lm) ? -1.f : 1.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = hx(x[i], lm) + __uint_as_float(__float_as_uint(x[i]) ^ flip);
+    for (int i = 0; i < 4; ++i) x[i] = __builtin_fmaf(x[i], sign, hx(x[i], lm));
   }
 }
 template <int N>
