@@ -30,6 +30,7 @@ DEVI float e4m3_value(uint32_t b) {
 template <bool F8> DEVI void kv_params(float& mn, float& s) {         // the (min, scale) the codes are computed from
   if (F8) { mn = e4m3_value(e4m3_bits(mn)); s = e4m3_value(e4m3_bits(s)); }
 }
+constexpr float KV_SURE = 0.5f - 9.5367431640625e-07f;     // distance of an estimated quotient from its rounding (kv_codes)
 DEVI int kv_code(float x, float mn, float s) {
   const float d = s == 0.f ? 1.f : s;
   float q = (x - mn) / d;
@@ -48,7 +49,7 @@ DEVI void kv_codes(const float (&x)[4], float mn, float s, int (&code)[4]) {
     worst = fmaxf(worst, fabsf(q - n));
     code[i] = static_cast<int>(n);
   }
-  if (!(worst < 0.5f - 9.5367431640625e-07f && d > 1e-30f && d < 1e30f)) {
+  if (!(worst < KV_SURE && d > 1e-30f && d < 1e30f)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) code[i] = kv_code(x[i], mn, s);
   }
