@@ -376,8 +376,12 @@ class DecodeLayer:
                       self.kind, **extra)
 
     def step(self, q, kv, sp: StepPlan, out):
-        """what a captured decode step of this layer contains"""
-        self.update(kv, sp)
+        """what a captured decode step of this layer contains: update, in one launch, and decode"""
+        if self.ring is None:
+            self.write_pages(kv, sp.slots)
+        else:
+            K.step_write(kv, sp.slots, self.kind, self.pool, PAGE, self.ring, sp.ring_dest, mask=self.wmask, CT=self.CT,
+                         kmu=self.kmu)
         self.decode(q, sp, out)
 
 
@@ -431,6 +435,9 @@ class KiviDecodeLayer:
     def update(self, kv, sp: StepPlan):
         KIVI.v_write(kv, sp.slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
         K.ring_rows(kv, self.ring, dest=sp.ring_dest)
+        self._encode_completed(sp)
+
+    def _encode_completed(self, sp: StepPlan):
         KIVI.k_encode(self.ring, sp.group_src, sp.group_dst, self.qs, self.lz, self.scale, self.pool, self.Hkv, D,
                       f8=self.f8)
 
@@ -443,5 +450,9 @@ class KiviDecodeLayer:
                   tail_idx=sp.ring_home, T=self.geo.slots, f8=self.f8)
 
     def step(self, q, kv, sp: StepPlan, out):
-        self.update(kv, sp)
+        if kv.shape[0] == sp.slots.shape[0] and kv.stride(0) % 4 == 0 and kv.data_ptr() % 8 == 0:
+            KIVI.step_write(kv, sp.slots, self.co, self.pool, self.ring, sp.ring_dest, f8=self.f8)
+            self._encode_completed(sp)
+        else:                                              # (the one launch reads both halves of a row eight bytes at a time)
+            self.update(kv, sp)
         self.decode(q, sp, out)

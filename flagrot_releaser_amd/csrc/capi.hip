@@ -217,6 +217,30 @@ int fr_ring_rows(const void* kv, long long kv_ts, int T, int Hkv, int Dh, const 
   return launched(ring_rows_launch(p, static_cast<hipStream_t>(stream)), "fr_ring_rows");
 }
 
+int fr_step_write(int fmt, const void* kv, long long kv_ts, const long long* slots, int T, int Hkv, int page,
+                  const uint8_t* mask, const float* CT, uint8_t* pool, const float* kmu, void* ring, const long long* dest,
+                  long long ring_rows, void* stream) {
+  if (T <= 0) return 0;
+  RingRowsParams r{};
+  r.kv = kv; r.kv_ts = kv_ts; r.width = 2 * Hkv * 128; r.kmu = kmu; r.ring = ring; r.ring_rows = ring_rows; r.dest = dest;
+  r.rows = r.sinks = T;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (fmt == FMT_INT4 || fmt == FMT_INT4A || fmt == FMT_INT2A) {
+    StaticWriteParams p{};
+    p.kv = kv; p.kv_ts = kv_ts; p.slots = slots; p.T = T; p.Hkv = Hkv; p.page = page;
+    p.mask = mask; p.kmu = kmu; p.pool = pool; p.ring = r;
+    return launched(static_write_launch(fmt, p, st), "fr_step_write");
+  }
+  const int kind = fmt == FMT_KONLY ? KIND_KONLY : fmt == FMT_KONLYA ? KIND_KONLYA : fmt == FMT_KONLYA2 ? KIND_KONLYA2 : -1;
+  if (kind < 0) return fail(-4, "fr_step_write: fmt must be 4 .. 9");
+  K2WriteParams p{};
+  p.kv = kv; p.kv_ts = kv_ts; p.slots = slots; p.T = T; p.Hkv = Hkv; p.page = page;
+  p.CT = CT; p.kmu = kmu; p.pool = pool; p.passes = 3; p.hd = 128; p.screen = 1;
+  if (k2_is_step(p)) p.ring = r;                          // more tokens than a decode step has: a launch of their own
+  const int rc = k2_write_launch(kind, p, st);
+  return launched(rc != 0 || p.ring.rows != 0 ? rc : ring_rows_launch(r, st), "fr_step_write");
+}
+
 // What the host split planner multiplies by the CU count to get the number of workgroups that run at once.  The answer
 // is 1: the fastest launch shape is ONE large workgroup per CU (decode_launch takes it whenever the plan's workgroups
 // fit the CUs once with >= 1024 tokens each), and a planner that fills "1 x CUs" slots with the longest chunks that

@@ -5,6 +5,19 @@
 
 namespace fr {
 
+struct RingRowsParams {
+  const void* kv;          // bf16 [T, width], token stride kv_ts
+  long long kv_ts;
+  int width;               // elements of a row: 2 * Hkv * head dim
+  const float* kmu;        // [width / 2] subtracted from the key half, or null
+  void* ring;              // bf16 [*, width]
+  long long ring_rows;     // rows the ring has: no row outside [0, ring_rows) is written
+  const long long* dest;   // ring row of every token, or null: the rule below
+  long long base;          // first ring row of the request
+  int S, W, start;         // sinks, window, position of token 0
+  int rows, sinks, win0;   // rows copied: tokens [0, sinks) and [win0, win0 + rows - sinks)
+};
+
 struct StaticWriteParams {
   const void* kv;          // bf16 [T, rows, 128] (rows = 2 * Hkv half-head rows, K rows first), token stride kv_ts
   long long kv_ts;
@@ -14,6 +27,7 @@ struct StaticWriteParams {
   const uint8_t* hfull;    // [2 * Hkv] whole-head +-1 Hadamard / 16 with a bf16 rounding first, or null
   const float* kmu;        // [Hkv, 128] or null
   uint8_t* pool;
+  RingRowsParams ring;     // rows of a decode step that are kept in BF16 too (rows 0: none)
 };
 int static_write_launch(int fmt, const StaticWriteParams& p, hipStream_t st);
 
@@ -29,8 +43,10 @@ struct K2WriteParams {
   int passes;              // bit 0: key rows, bit 1: value rows
   int screen;              // 1: large key passes may run the screened kernel (same bytes; fr_cb_write3)
   int hd;                  // head dim: 0 | 128, or 256 (fr_cb_write only)
+  RingRowsParams ring;     // rows of a decode step that are kept in BF16 too (rows 0: none; k_k2_step only)
 };
 int k2_write_launch(int kind, const K2WriteParams& p, hipStream_t st);
+bool k2_is_step(const K2WriteParams& p);                                   // k2_write_launch takes k2_step_launch
 int k2_write_lds_bytes(int hd);
 int k2_step_launch(int kind, const K2WriteParams& p, hipStream_t st);      // one workgroup per (token, KV head); same bytes
 
@@ -40,18 +56,6 @@ int k2_screen_lds_bytes(int hd);
 int head_fwht_launch(const void* x, long long x_ts, void* out, long long o_ts, int T, int H, const uint8_t* flags,
                      float scale, hipStream_t st, int D);
 
-struct RingRowsParams {
-  const void* kv;          // bf16 [T, width], token stride kv_ts
-  long long kv_ts;
-  int width;               // elements of a row: 2 * Hkv * head dim
-  const float* kmu;        // [width / 2] subtracted from the key half, or null
-  void* ring;              // bf16 [*, width]
-  long long ring_rows;     // rows the ring has: no row outside [0, ring_rows) is written
-  const long long* dest;   // ring row of every token, or null: the rule below
-  long long base;          // first ring row of the request
-  int S, W, start;         // sinks, window, position of token 0
-  int rows, sinks, win0;   // rows copied: tokens [0, sinks) and [win0, win0 + rows - sinks)
-};
 int ring_rows_launch(const RingRowsParams& p, hipStream_t st);
 
 struct DecodeParams {

@@ -47,7 +47,18 @@ int kv_v_write(const void* kv, long long kv_rs, int n, int Hkv, int D, const voi
                                       static_cast<const int*>(vfix), f8 & 1, static_cast<hipStream_t>(stream)), "kv_v_write");
   return launched(v_write_launch(kv, kv_rs, n, Hkv, static_cast<const long long*>(slots), static_cast<const float*>(co),
                                  static_cast<uint8_t*>(pool), static_cast<const float*>(M), ident, static_cast<const int*>(vfix), f8 & 1,
-                                 static_cast<hipStream_t>(stream)), "kv_v_write");
+                                 static_cast<hipStream_t>(stream), fr::RingRowsParams{}), "kv_v_write");
+}
+
+int kv_step_write(const void* kv, long long kv_rs, int n, int Hkv, const void* slots, const void* co, void* pool, int f8,
+                  void* ring, const void* dest, long long ring_rows, void* stream) {
+  if (n <= 0) return 0;
+  fr::RingRowsParams r{};
+  r.kv = kv; r.kv_ts = kv_rs; r.width = 2 * Hkv * 128; r.ring = ring; r.ring_rows = ring_rows;
+  r.dest = static_cast<const long long*>(dest); r.rows = r.sinks = n;
+  return launched(v_write_launch(kv, kv_rs, n, Hkv, static_cast<const long long*>(slots), static_cast<const float*>(co),
+                                 static_cast<uint8_t*>(pool), nullptr, 0, nullptr, f8 & 1, static_cast<hipStream_t>(stream), r),
+                  "kv_step_write");
 }
 
 int kv_k_encode(const void* src, long long src_rs, const void* src2, long long src2_rs, const void* sidx,

@@ -5,10 +5,13 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fr_launch.hpp"
+
 namespace frkv {
 
 int v_write_launch(const void* kv, long long kv_rs, int n, int Hkv, const long long* slots, const float* co, uint8_t* pool,
-                   const float* M, int ident, const int* vfix, int f8, hipStream_t st);
+                   const float* M, int ident, const int* vfix, int f8, hipStream_t st,
+                   const fr::RingRowsParams& ring);
 int k_encode_launch(int D, const void* src, long long src_rs, const void* src2, long long src2_rs, const long long* sidx,
                     const long long* dslot, int N, int Hkv, const float* qs, const float* lz, int NQ, float qsc,
                     uint8_t* pool, int ident, const int* kfix, int f8, hipStream_t st);

@@ -20,6 +20,7 @@
 #include "kivi_launch.hpp"
 #include "kivi_quant.hpp"
 #include "kivi_vrow.hpp"
+#include "ring_rows.hpp"
 
 namespace frkv {
 using namespace fr;
@@ -38,11 +39,16 @@ template <bool F8, bool WMAT>
 __global__ void __launch_bounds__(256) k_v_write(const uint16_t* __restrict__ kv, long long kv_rs, int n, int Hkv,
                                                  const long long* __restrict__ slots, const float* __restrict__ co,
                                                  const float* __restrict__ M, uint8_t* __restrict__ pool, int ident,
-                                                 const int* __restrict__ vfix) {
+                                                 const int* __restrict__ vfix, const RingRowsParams ring) {
   __shared__ float strips[WMAT ? 8 : 1][WMAT ? 3 * 128 : 1];
   const int l32 = threadIdx.x & 31;
+  const long long items = static_cast<long long>(n) * Hkv, groups = (items + 7) / 8;
+  if (blockIdx.x >= groups) {                            // behind the values: the BF16 rows of the tokens
+    ring_quad(ring, (static_cast<long long>(blockIdx.x) - groups) * 256 + threadIdx.x);
+    return;
+  }
   const long long item = static_cast<long long>(blockIdx.x) * 8 + (threadIdx.x >> 5);
-  if (item >= static_cast<long long>(n) * Hkv) return;
+  if (item >= items) return;
   const int t = static_cast<int>(item / Hkv), h = static_cast<int>(item % Hkv);
   const long long slot = slots[t];
   if (slot < 0) return;
@@ -105,12 +111,12 @@ __global__ void k_lse_merge(const uint16_t* __restrict__ oa, const float* __rest
 }  // namespace
 
 int v_write_launch(const void* kv, long long kv_rs, int n, int Hkv, const long long* slots, const float* co, uint8_t* pool,
-                   const float* M, int ident, const int* vfix, int f8, hipStream_t st) {
+                   const float* M, int ident, const int* vfix, int f8, hipStream_t st, const RingRowsParams& ring) {
   const long long items = static_cast<long long>(n) * Hkv;
   const bool wmat = M != nullptr && !ident && vfix == nullptr;
   const auto kern = wmat ? (f8 ? k_v_write<true, true> : k_v_write<false, true>) : (f8 ? k_v_write<true, false> : k_v_write<false, false>);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((items + 7) / 8)), dim3(256), 0, st,
-                     static_cast<const uint16_t*>(kv), kv_rs, n, Hkv, slots, co, M, pool, ident, vfix);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((items + 7) / 8 + (ring_quads(ring) + 255) / 256)), dim3(256), 0, st,
+                     static_cast<const uint16_t*>(kv), kv_rs, n, Hkv, slots, co, M, pool, ident, vfix, ring);
   return hipPeekAtLastError() == hipSuccess ? 0 : 1;
 }
 

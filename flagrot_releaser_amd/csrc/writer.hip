@@ -13,6 +13,7 @@
 #include <cstdlib>
 
 #include "fr_launch.hpp"
+#include "ring_rows.hpp"
 #include "writer_rows.hpp"
 
 namespace fr {
@@ -39,6 +40,11 @@ __global__ void __launch_bounds__(256) k_static_write(const StaticWriteParams p)
   __shared__ VRuns<8> runs;
   const int l32 = threadIdx.x & 31, hw = threadIdx.x >> 5;
   const int H2 = 2 * p.Hkv;
+  const int tiles = (p.T + 7) / 8 * H2;
+  if (static_cast<int>(blockIdx.x) >= tiles) {  // behind the tokens: their BF16 rows
+    ring_quad(p.ring, static_cast<long long>(blockIdx.x - tiles) * 256 + threadIdx.x);
+    return;
+  }
   const int hr = static_cast<int>(blockIdx.x % H2);
   const int t = static_cast<int>(blockIdx.x / H2) * 8 + hw;
   long long slot = -1;
@@ -322,8 +328,8 @@ __global__ void __launch_bounds__(256) k_k2_write(const K2WriteParams p, int tok
 
 template <int QM>
 int static_write_qm(const StaticWriteParams& p, hipStream_t st) {
-  const unsigned grid = static_cast<unsigned>(static_cast<long long>((p.T + 7) / 8) * 2 * p.Hkv);
-  if (grid == 0) return 0;
+  if (p.T <= 0) return 0;
+  const unsigned grid = static_cast<unsigned>(static_cast<long long>((p.T + 7) / 8) * 2 * p.Hkv + (ring_quads(p.ring) + 255) / 256);
   if (p.page == 16) hipLaunchKernelGGL((k_static_write<QM, 16>), dim3(grid), dim3(256), 0, st, p);
   else if (p.page == 32) hipLaunchKernelGGL((k_static_write<QM, 32>), dim3(grid), dim3(256), 0, st, p);
   else return -5;
@@ -366,12 +372,16 @@ int static_write_launch(int fmt, const StaticWriteParams& p, hipStream_t st) {
   return -4;
 }
 
+// a decode step's worth of tokens: one workgroup per (token, head)
+bool k2_is_step(const K2WriteParams& p) {
+  static const bool no_step = getenv("FLAGROT_WRITER_LL") != nullptr && getenv("FLAGROT_WRITER_LL")[0] == '0';
+  return !(no_step && p.hd != 256) && static_cast<long long>(p.T) * p.Hkv <= 1024;
+}
+
 int k2_write_launch(int kind, const K2WriteParams& p, hipStream_t st) {
   if (p.hd == 256 && p.passes != 3) return -8;             // the two-pass forms exist for 128-d heads only
   const long long pairs = static_cast<long long>(p.T) * p.Hkv;
-  // a decode step's worth of tokens: one workgroup per (token, head)
-  static const bool no_step = getenv("FLAGROT_WRITER_LL") != nullptr && getenv("FLAGROT_WRITER_LL")[0] == '0';
-  if (!(no_step && p.hd != 256) && pairs <= 1024) return k2_step_launch(kind, p, st);
+  if (k2_is_step(p)) return k2_step_launch(kind, p, st);
   // Prompt-sized key passes: choices screened on the matrix pipe (FLAGROT_W3: 0 off for 128-d heads, 2 every token exact).
   // us by tokens / screened at 768, 1024, 1280, 1536, 2048 pairs: 4 heads of 256 23 / 31, 28 / 28, 33 / 31, 38 / 28, 49 / 28;
   // 8 heads of 128 on 4-bit pages 11.0 / 17.3, 13.5 / 17.4, 15.6 / 17.3, 17.2 / 17.3, 20.8 / 17.5, on 2-bit pages 12.0 / 17.7,

@@ -4,6 +4,7 @@
 // Bound by latency: launch, one trip to memory and the chains of the exact evaluation.  Call of 32 tokens x 8 heads of
 // 128, 4-bit / 2-bit pages: 11.6 / 13.4 -> 5.7 us (before: four half waves per token, C_q^T staged in LDS, 2-bit value
 // fields that met on one word); 16 tokens x 4 heads of 256: 47 -> 6.8 us (one half wave per token).
+#include "ring_rows.hpp"
 #include "writer_exact.hpp"
 
 namespace fr {
@@ -13,6 +14,10 @@ template <int QM, int P, int D>
 __global__ void __launch_bounds__(2 * D) k_k2_step(const K2WriteParams p) {
   __shared__ StepSmem<D> S;
   const int h = blockIdx.x, t = blockIdx.y;
+  if (t >= p.T) {                                  // behind the tokens: their BF16 rows
+    ring_quad(p.ring, (static_cast<long long>(t - p.T) * p.Hkv + h) * (2 * D) + threadIdx.x);
+    return;
+  }
   const long long slot = p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)];
   if (slot < 0) return;                            // the whole workgroup
   CqRegs<D> C;
@@ -21,7 +26,8 @@ __global__ void __launch_bounds__(2 * D) k_k2_step(const K2WriteParams p) {
 
 template <int QM, int P>
 void step(const K2WriteParams& p, hipStream_t st) {
-  const dim3 grid(p.Hkv, p.T);
+  const long long per_row = static_cast<long long>(p.Hkv) * (p.hd == 256 ? 512 : 256);      // quads of a row of workgroups
+  const dim3 grid(p.Hkv, p.T + static_cast<unsigned>((ring_quads(p.ring) + per_row - 1) / per_row));
   if (p.hd == 256) hipLaunchKernelGGL((k_k2_step<QM, P, 256>), grid, dim3(512), 0, st, p);
   else hipLaunchKernelGGL((k_k2_step<QM, P, 128>), grid, dim3(256), 0, st, p);
 }

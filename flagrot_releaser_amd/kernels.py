@@ -39,6 +39,7 @@ NATIVE = Library("kernels", "FLAGROT_LIB", "fr_abi_version", ABI, "fr_last_error
     "fr_v2_attn": "i p l p p i p i i i i i f p p i i i i i p p p p l p p p l l p i i",
     "fr_v2_write": "i p l p i i i p i p p i p",
     "fr_ring_rows": "p l i i i p p p l i i i p l",
+    "fr_step_write": "i p l p i i i p p p p p p l p",
     "fr_v2_occupancy": "i i i i",
     "fr_v2_chunk_bytes": "i i",
     "fr_cb_nsg": "",
@@ -407,6 +408,30 @@ def cb_attn_noalloc(q, pool, block_table, seq_lens, out, nsplit, chunk, qscale, 
     return _decode("fr_cb_attn_noalloc", args, bound)
 
 
+def ring_of(kv, ring, dest) -> int:
+    """the number of rows of a ring that rows kv may be copied into, at rows dest if given"""
+    T, heads, Dh = kv.shape
+    assert kv.dtype == torch.bfloat16 and ring.dtype == torch.bfloat16 and ring.is_contiguous()
+    assert ring.shape[-2:] == (heads, Dh) and heads % 2 == 0 and ring.device == kv.device and ring.data_ptr() % 8 == 0, \
+        "ring: rows of kv's shape, on its device, 8-byte aligned"
+    assert dest is None or (dest.dtype == torch.int64 and dest.is_contiguous() and dest.shape == (T,)
+                            and dest.device == kv.device), "dest: int64 [T], contiguous, on the rows' device"
+    return ring.numel() // (heads * Dh)
+
+
+def step_write(kv, slots, fmt, pool, page, ring, dest, mask=None, CT=None, kmu=None):
+    """What a decode step stores of its rows, in one launch: v2_write (static formats, with mask) or cb_write (key-only
+    kinds, with CT) and ring_rows with dest.  Head dim 128."""
+    T, heads, Dh = kv.shape
+    if T == 0:
+        return
+    have = ring_of(kv, ring, dest)
+    assert Dh == D and slots.dtype == torch.int64
+    rows = _loadable(kv)
+    NATIVE.run("fr_step_write", V2_FMT[fmt], rows, rows.stride(0), slots.contiguous(), T, heads // 2, page, mask, CT, pool,
+               _centre(kmu, rows), ring, dest, have, current_stream())
+
+
 def ring_rows(kv, ring, kmu=None, dest=None, base=0, sink=0, window=0, start=0):
     """The BF16 rows a request keeps beside its pages: rows kv bf16 [T, 2 Hkv, Dh] into ring bf16 [..., 2 Hkv, Dh], contiguous;
     kmu fp32 [Hkv, Dh] is subtracted from the keys (FP32, one rounding).  dest int64 [T] names the ring row of every token
@@ -416,16 +441,10 @@ def ring_rows(kv, ring, kmu=None, dest=None, base=0, sink=0, window=0, start=0):
     T, heads, Dh = kv.shape
     if T == 0:
         return
-    assert kv.dtype == torch.bfloat16 and ring.dtype == torch.bfloat16 and ring.is_contiguous()
-    assert ring.shape[-2:] == (heads, Dh) and heads % 2 == 0 and ring.device == kv.device and ring.data_ptr() % 8 == 0, \
-        "ring: rows of kv's shape, on its device, 8-byte aligned"
-    rows, have = _loadable(kv), ring.numel() // (heads * Dh)
+    rows, have = _loadable(kv), ring_of(kv, ring, dest)
     if dest is None:
         base, start = operator.index(base), operator.index(start)
         assert 0 <= base and base + sink + window <= have, "the request's rows lie outside the ring"
-    else:
-        assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.shape == (T,) and dest.device == kv.device, \
-            "dest: int64 [T], contiguous, on the rows' device"
     NATIVE.run("fr_ring_rows", rows, rows.stride(0), T, heads // 2, Dh, _centre(kmu, rows), ring, dest,
                base, sink, window, start, current_stream(), have)
 

@@ -58,6 +58,13 @@ int fr_v2_write(int fmt, const void* kv, long long kv_ts, const long long* slots
 int fr_ring_rows(const void* kv, long long kv_ts, int T, int Hkv, int Dh, const float* kmu, void* ring, const long long* dest,
                  long long base, int S, int W, int start, void* stream, long long ring_rows);
 
+/* No counterpart in the reference.  The cache update of a decode step in one launch, head dim 128: the bytes that fr_v2_write
+ * (fmt 4 | 5 | 8, with mask) or fr_cb_write (fmt 6 | 7 | 9, with CT) store for the rows, and the rows that fr_ring_rows with
+ * dest and kmu copies. */
+int fr_step_write(int fmt, const void* kv, long long kv_ts, const long long* slots, int T, int Hkv, int page,
+                  const uint8_t* mask, const float* CT, uint8_t* pool, const float* kmu, void* ring, const long long* dest,
+                  long long ring_rows, void* stream);
+
 /* flagrot_capi.cu:79-80.  Resident 4-wavefront workgroups per CU (for the host split planner); bytes per (page, head)
  * chunk. */
 int fr_v2_occupancy(int fmt, int variant, int stages, int page);

@@ -31,6 +31,12 @@ int kv_chunk_bytes8(int D);
 int kv_v_write(const void* kv, long long kv_rs, int n, int Hkv, int D, const void* slots, const void* co, const void* M,
                void* pool, int ident, const void* vfix, int f8, void* stream);
 
+/* No counterpart in the reference.  What a decode step stores of its rows before its key groups, in one launch, D = 128:
+ * kv_v_write (co, no M / ident / vfix) and the rows bf16 [n, 2*Hkv, 128] (8-byte aligned) copied to rows dest int64 [n] of ring
+ * bf16 [ring_rows, 2*Hkv, 128] (tokens whose row is not in 0 .. ring_rows - 1 are left out of the ring). */
+int kv_step_write(const void* kv, long long kv_rs, int n, int Hkv, const void* slots, const void* co, void* pool, int f8,
+                  void* ring, const void* dest, long long ring_rows, void* stream);
+
 /* kivi.cu:1951-1977.  src / src2 bf16 rows (K row of head h at + h*D); sidx int64 [N, 32]: r >= 0 src row, r <= -2
  * src2 row -r-2, -1 not in the group; dslot int64 [N, 32] page slots (dslot[n][0] < 0: inactive item); qs fp32
  * [Hkv, NQ, D], lz fp32 [Hkv, NQ]; kfix int32 [Hkv] or null. */
