@@ -53,30 +53,33 @@ __global__ void __launch_bounds__(64 * NW, 4) k_decode(const DecodeParams p, int
   using L = Lay<QM, P>;
   __shared__ Smem<QM, NW> S;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int kvh = blockIdx.x / ntile, tile = blockIdx.x % ntile;
   // Workgroups are dispatched in linear order and the CU's arbiter favours the older wavefronts: the splits of one
-  // sequence are spread over the whole dispatch order (split slowest) so that every sequence gets the same mix.
-  int lin = blockIdx.z * gridDim.y + blockIdx.y;
-  if (ntile > 1 && (p.Hkv * static_cast<int>(gridDim.y * gridDim.z)) % 8 == 0) {
-    // Workgroups go to the 8 XCDs round robin in dispatch order and each XCD has its own L2.  The q tiles of one (KV
-    // head, split, sequence) read the same pages: they are made neighbours on ONE XCD (dispatch positions 8 apart), so
-    // that the second reader finds the first one's lines in that L2 -- whoever runs ahead waits for HBM, whoever
-    // follows catches up.
-    const int pos = blockIdx.x + gridDim.x * lin;
-    const int slot = pos >> 3, t3 = (slot / ntile) * 8 + (pos & 7);
-    tile = slot % ntile;
-    kvh = t3 % p.Hkv;
-    lin = t3 / p.Hkv;
+  // sequence are spread over the whole dispatch order (the grid's z, slowest) so that every sequence gets the same mix.
+  int kvh = blockIdx.x, tile = 0, b = blockIdx.y, split = blockIdx.z;
+  if (ntile > 1) {
+    kvh = blockIdx.x / ntile; tile = blockIdx.x % ntile;
+    if ((p.Hkv * static_cast<int>(gridDim.y * gridDim.z)) % 8 == 0) {
+      // Workgroups go to the 8 XCDs round robin in dispatch order and each XCD has its own L2.  The q tiles of one (KV
+      // head, split, sequence) read the same pages: they are made neighbours on ONE XCD (dispatch positions 8 apart), so
+      // that the second reader finds the first one's lines in that L2 -- whoever runs ahead waits for HBM, whoever
+      // follows catches up.
+      const int pos = blockIdx.x + gridDim.x * (blockIdx.z * gridDim.y + blockIdx.y);
+      const int slot = pos >> 3, t3 = (slot / ntile) * 8 + (pos & 7), lin = t3 / p.Hkv;
+      tile = slot % ntile;
+      kvh = t3 % p.Hkv;
+      split = lin / p.B;
+      b = lin % p.B;
+    }
   }
   // Where the body workgroups of a sequence draw from one shared range, the BF16 rows' workgroups (the last split) go
   // first in dispatch order: short ones that start with the launch instead of trailing it, and a body workgroup that
   // starts later for it just draws what is left.  (With fixed ranges per split a late start is a late end: there the
   // body goes first; measured both ways.)
-  const int nsp = static_cast<int>(gridDim.y * gridDim.z) / p.B;
-  int split = lin / p.B;
-  if (p.tail != nullptr && p.dyn != 0) split = split == 0 ? nsp - 1 : split - 1;
-  const int b = lin % p.B;
+  if (p.tail != nullptr && p.dyn != 0) split = split == 0 ? static_cast<int>(gridDim.z) - 1 : split - 1;
   const bool is_tail = p.tail != nullptr && split == p.nsplit;
+  const bool act = wave < 4;      // the 256 threads that own the workgroup's 4 x 128 outputs, and prepare a query head each
+  uint2 qraw = make_uint2(0u, 0u);                // (requested first: the prologue is the first to wait for memory)
+  if (!is_tail && act) qraw = query_row(p, b, kvh, tile * 4 + wave);
   // The block-table entries of the workgroup's page range are requested before the sequence length is known (the
   // length load and these loads are then in flight together: one memory latency less before the first page arrives).
   // If the range is not empty it starts at this token; entries are bounded by the row's length, and whatever lies
@@ -105,7 +108,6 @@ __global__ void __launch_bounds__(64 * NW, 4) k_decode(const DecodeParams p, int
   if (nspec > 0 && lane < PPQ && PPQ * qi0 + lane < p.bt_stride - pg0s) mine4 = btrow[pg0s + PPQ * qi0 + lane];   // (PPQ <= 8)
   const int len = p.seq_lens[b];
   const long long part_id = ((static_cast<long long>(b) * p.Hkv + kvh) * ntile + tile) * nparts + split;
-  const bool act = wave < 4;      // the 256 threads that own the workgroup's 4 x 128 outputs
 
   // the (sequence, KV head, q tile)'s counter slot: merge ticket, and in the dynamic mode the quad draw counter
   // q tiles per counter slot: always 1.  The value is hidden from the compiler on purpose: folded in as a constant it
@@ -168,7 +170,7 @@ __global__ void __launch_bounds__(64 * NW, 4) k_decode(const DecodeParams p, int
       // the pad entry of every strip row group: what the value phase reads for the columns of foreign groups
       for (int i = threadIdx.x; i < NW * Strip<QM>::ROWS; i += 64 * NW)
         (reinterpret_cast<uint4*>(S.pb(i / Strip<QM>::ROWS)) + (i % Strip<QM>::ROWS) * PB_RSTRIDE)[16] = make_uint4(0u, 0u, 0u, 0u);
-      if (act) q_prologue<QM, K2>(S, p, b, kvh, tile);
+      if (act) q_prologue<QM, K2>(S, p, qraw, kvh);
       __syncthreads();
       const int npg = pg1 - pg0;
       const int nquad = (npg + PPQ - 1) / PPQ;
@@ -369,24 +371,16 @@ __global__ void __launch_bounds__(64 * NW, 4) k_decode(const DecodeParams p, int
       po[0] += f * v.x; po[1] += f * v.y;
     }
   }
+  // a value group's 32 outputs of a head (a row of 16 lanes, two each) between the stored basis and the original one
+  auto unrotate = [&](float (&v)[2]) {
+    const bool rotated = p.vmask[kvh * 4 + (lane >> 4)] != 0;
+    float y[2] = {v[0], v[1]};
+    h32_row16(y[0], y[1], lane);
+    v[0] = rotated ? y[0] : v[0];
+    v[1] = rotated ? y[1] : v[1];
+  };
   if (is_tail && p.vmask != nullptr) {  // the merged sum is rotated back once: bring the tail into the stored basis
-    __syncthreads();
-    if (act) { S.o(0, oh)[2 * lane] = po[0]; S.o(0, oh)[2 * lane + 1] = po[1]; }
-    __syncthreads();
-    if (act) {
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int d = 2 * lane + e, g = d >> 5;
-        if (p.vmask[kvh * 4 + g]) {
-          float a = 0.f;
-          for (int k = 0; k < 32; ++k) {
-            const float v = S.o(0, oh)[32 * g + k];
-            a += (__builtin_popcount(d & k & 31) & 1) ? -v : v;
-          }
-          po[e] = a * kC32;
-        }
-      }
-    }
+    unrotate(po);
   }
   if (nparts > 1) {
     // Partials cross workgroups (and XCDs, each with its own L2) through device-scope relaxed atomic stores / loads,
@@ -396,12 +390,8 @@ __global__ void __launch_bounds__(64 * NW, 4) k_decode(const DecodeParams p, int
     // wait), barrier, ticket; the last arriver reads (device-scope loads) after its ticket has returned.
     if (act) {
       float* op = p.opart + part_id * 512 + oh * 128 + 2 * lane;
-      __hip_atomic_store(op, po[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(op + 1, po[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (lane == 0) {
-        __hip_atomic_store(p.mlpart + part_id * 8 + 2 * oh, pm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(p.mlpart + part_id * 8 + 2 * oh + 1, pl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+      store_shared_pair(op, po[0], po[1]);
+      if (lane == 0) store_shared_pair(p.mlpart + part_id * 8 + 2 * oh, pm, pl);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // this wavefront's partial stores have been acknowledged
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -423,39 +413,19 @@ __global__ void __launch_bounds__(64 * NW, 4) k_decode(const DecodeParams p, int
   const int ntt = nparts > 1 ? tpc : 1;
   const int tile0 = nparts > 1 ? (tile / tpc) * tpc : tile;
   for (int tt = tile0; tt < tile0 + ntt; ++tt) {
-    float M = pm, Lsum = pl, o0 = po[0], o1 = po[1];
+    float M[1] = {pm}, Lsum[1] = {pl}, o[1][2] = {{po[0], po[1]}};
     if (nparts > 1 && act) {
       const long long base = ((static_cast<long long>(b) * p.Hkv + kvh) * ntile + tt) * nparts;
-      merge_parts(p.mlpart, p.opart, base, nparts, oh, lane, M, Lsum, o0, o1);
+      merge_parts<1>(p.mlpart, p.opart, base, nparts, oh, lane, M, Lsum, o);
     }
-    const float inv = Lsum > 0.f ? 1.f / Lsum : 0.f;
-    o0 *= inv; o1 *= inv;
-    if (p.vmask != nullptr) {
-      __syncthreads();
-      if (act) { S.o(0, oh)[2 * lane] = o0; S.o(0, oh)[2 * lane + 1] = o1; }
-      __syncthreads();
-      float r[2] = {o0, o1};
-      if (act) {
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int d = 2 * lane + e, g = d >> 5;
-          if (p.vmask[kvh * 4 + g]) {
-            float a = 0.f;
-            for (int k = 0; k < 32; ++k) {
-              const float v = S.o(0, oh)[32 * g + k];
-              a += (__builtin_popcount(d & k & 31) & 1) ? -v : v;
-            }
-            r[e] = a * kC32;
-          }
-        }
-      }
-      o0 = r[0]; o1 = r[1];
-    }
+    const float inv = Lsum[0] > 0.f ? 1.f / Lsum[0] : 0.f;
+    o[0][0] *= inv; o[0][1] *= inv;
+    if (p.vmask != nullptr) unrotate(o[0]);
     const int hq = tt * 4 + oh;
     if (act && hq < p.gqa) {
       uint16_t* orow = static_cast<uint16_t*>(p.out) + static_cast<long long>(b) * p.o_bs +
                        (static_cast<long long>(kvh) * p.gqa + hq) * 128 + 2 * lane;
-      *reinterpret_cast<uint32_t*>(orow) = bf16_rn(o0) | (bf16_rn(o1) << 16);
+      *reinterpret_cast<uint32_t*>(orow) = bf16_rn(o[0][0]) | (bf16_rn(o[0][1]) << 16);
     }
   }
 }
@@ -472,7 +442,7 @@ int launch_qm(const DecodeParams& p, hipStream_t st) {
   const int ntile = (p.gqa + 3) / 4;
   const int nparts = p.nsplit + ((p.tail != nullptr && !p.fuse_tail) ? 1 : 0);
   if (nparts <= 0 || p.B <= 0) return 0;
-  dim3 grid(p.Hkv * ntile, nparts, p.B);
+  dim3 grid(p.Hkv * ntile, p.B, nparts);
   if (p.page == 32) {
     if (p.wg_waves > 4) hipLaunchKernelGGL((k_decode<QM, K2, 32, BIGW<QM>>), grid, dim3(64 * BIGW<QM>), 0, st, p, ntile, nparts);
     else hipLaunchKernelGGL((k_decode<QM, K2, 32, 4>), grid, dim3(256), 0, st, p, ntile, nparts);

@@ -38,30 +38,36 @@ __global__ void __launch_bounds__(64 * NW, (MINW8<QM, K2, P>)) k_decode8(const D
   using L = Lay<QM, P>;
   __shared__ Smem8<QM, NW> S;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int kvh = blockIdx.x / ntile, tile = blockIdx.x % ntile;
   // Workgroups are dispatched in linear order and the CU's arbiter favours the older wavefronts: the splits of one
-  // sequence are spread over the whole dispatch order (split slowest) so that every sequence gets the same mix.
-  int lin = blockIdx.z * gridDim.y + blockIdx.y;
-  if (ntile > 1 && (p.Hkv * static_cast<int>(gridDim.y * gridDim.z)) % 8 == 0) {
-    // Workgroups go to the 8 XCDs round robin in dispatch order and each XCD has its own L2.  The q tiles of one (KV
-    // head, split, sequence) read the same pages: they are made neighbours on ONE XCD (dispatch positions 8 apart), so
-    // that the second reader finds the first one's lines in that L2 -- whoever runs ahead waits for HBM, whoever
-    // follows catches up.
-    const int pos = blockIdx.x + gridDim.x * lin;
-    const int slot = pos >> 3, t3 = (slot / ntile) * 8 + (pos & 7);
-    tile = slot % ntile;
-    kvh = t3 % p.Hkv;
-    lin = t3 / p.Hkv;
+  // sequence are spread over the whole dispatch order (the grid's z, slowest) so that every sequence gets the same mix.
+  int kvh = blockIdx.x, tile = 0, b = blockIdx.y, split = blockIdx.z;
+  if (ntile > 1) {
+    kvh = blockIdx.x / ntile; tile = blockIdx.x % ntile;
+    if ((p.Hkv * static_cast<int>(gridDim.y * gridDim.z)) % 8 == 0) {
+      // Workgroups go to the 8 XCDs round robin in dispatch order and each XCD has its own L2.  The q tiles of one (KV
+      // head, split, sequence) read the same pages: they are made neighbours on ONE XCD (dispatch positions 8 apart), so
+      // that the second reader finds the first one's lines in that L2 -- whoever runs ahead waits for HBM, whoever
+      // follows catches up.
+      const int pos = blockIdx.x + gridDim.x * (blockIdx.z * gridDim.y + blockIdx.y);
+      const int slot = pos >> 3, t3 = (slot / ntile) * 8 + (pos & 7), lin = t3 / p.Hkv;
+      tile = slot % ntile;
+      kvh = t3 % p.Hkv;
+      split = lin / p.B;
+      b = lin % p.B;
+    }
   }
   // Where the body workgroups of a sequence draw from one shared range, the BF16 rows' workgroups (the last split) go
   // first in dispatch order: short ones that start with the launch instead of trailing it, and a body workgroup that
   // starts later for it just draws what is left.  (With fixed ranges per split a late start is a late end: there the
   // body goes first; measured both ways.)
-  const int nsp = static_cast<int>(gridDim.y * gridDim.z) / p.B;
-  int split = lin / p.B;
-  if (p.tail != nullptr && p.dyn != 0) split = split == 0 ? nsp - 1 : split - 1;
-  const int b = lin % p.B;
+  if (p.tail != nullptr && p.dyn != 0) split = split == 0 ? static_cast<int>(gridDim.z) - 1 : split - 1;
   const bool is_tail = p.tail != nullptr && split == p.nsplit;
+  uint2 qraw[Q8_TURNS<NW>];                       // (requested first: the prologue is the first to wait for memory)
+#pragma unroll
+  for (int turn = 0; turn < Q8_TURNS<NW>; ++turn) {
+    qraw[turn] = make_uint2(0u, 0u);
+    if (!is_tail && wave + turn * NW < 8) qraw[turn] = query_row(p, b, kvh, tile * 8 + wave + turn * NW);
+  }
   // The block-table entries of the workgroup's page range are requested before the sequence length is known (the
   // length load and these loads are then in flight together: one memory latency less before the first page arrives).
   // If the range is not empty it starts at this token; entries are bounded by the row's length, and whatever lies
@@ -154,7 +160,7 @@ __global__ void __launch_bounds__(64 * NW, (MINW8<QM, K2, P>)) k_decode8(const D
       constexpr int RSTR = PB8_RSTRIDE;
       for (int i = threadIdx.x; i < NW * Strip8<QM>::ROWS; i += 64 * NW)
         (reinterpret_cast<uint4*>(S.pb(i / Strip8<QM>::ROWS)) + (i % Strip8<QM>::ROWS) * RSTR)[RSTR - 1] = make_uint4(0u, 0u, 0u, 0u);
-      q_prologue8<QM, K2, NW>(S, p, b, kvh, tile);
+      q_prologue8<QM, K2, NW>(S, p, qraw, kvh);
       __syncthreads();
       const int npg = pg1 - pg0;
       const int nquad = (npg + PPQ - 1) / PPQ;
@@ -359,25 +365,13 @@ __global__ void __launch_bounds__(64 * NW, (MINW8<QM, K2, P>)) k_decode8(const D
       }
     }
   }
-  // a value group's 32 outputs of a head rotated back (static formats): through the head's row in LDS
-  auto unrotate = [&](float (&v2)[2]) {
-    __syncthreads();
-    if (act) { S.o(0, oh)[2 * lane] = v2[0]; S.o(0, oh)[2 * lane + 1] = v2[1]; }
-    __syncthreads();
-    if (act) {
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int d = 2 * lane + e, g = d >> 5;
-        if (p.vmask[kvh * 4 + g]) {
-          float a = 0.f;
-          for (int k = 0; k < 32; ++k) {
-            const float v = S.o(0, oh)[32 * g + k];
-            a += (__builtin_popcount(d & k & 31) & 1) ? -v : v;
-          }
-          v2[e] = a * kC32;
-        }
-      }
-    }
+  // a value group's 32 outputs of a head (a row of 16 lanes, two each) between the stored basis and the original one
+  auto unrotate = [&](float (&v)[2]) {
+    const bool rotated = p.vmask[kvh * 4 + (lane >> 4)] != 0;
+    float y[2] = {v[0], v[1]};
+    h32_row16(y[0], y[1], lane);
+    v[0] = rotated ? y[0] : v[0];
+    v[1] = rotated ? y[1] : v[1];
   };
   if (is_tail && p.vmask != nullptr) {  // the merged sum is rotated back once: bring the tail into the stored basis
 #pragma unroll
@@ -394,12 +388,8 @@ __global__ void __launch_bounds__(64 * NW, (MINW8<QM, K2, P>)) k_decode8(const D
       for (int t = 0; t < NT; ++t) {
         const long long part_id = part0 + static_cast<long long>(t) * nparts;
         float* op = p.opart + part_id * 512 + oh * 128 + 2 * lane;
-        __hip_atomic_store(op, po[t][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(op + 1, po[t][1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (lane == 0) {
-          __hip_atomic_store(p.mlpart + part_id * 8 + 2 * oh, pm[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(p.mlpart + part_id * 8 + 2 * oh + 1, pl[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        store_shared_pair(op, po[t][0], po[t][1]);
+        if (lane == 0) store_shared_pair(p.mlpart + part_id * 8 + 2 * oh, pm[t], pl[t]);
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // this wavefront's partial stores have been acknowledged
@@ -418,16 +408,12 @@ __global__ void __launch_bounds__(64 * NW, (MINW8<QM, K2, P>)) k_decode8(const D
   } else if (dyn && threadIdx.x == 0) {
     __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // the only workgroup of the slot
   }
-  // ---- final merge (last arriving workgroup, or the only one), half by half
+  // ---- final merge (last arriving workgroup, or the only one): both halves' partials in flight together
+  if (nparts > 1 && act) merge_parts<NT>(p.mlpart, p.opart, part0 - split, nparts, oh, lane, pm, pl, po);
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    float M = pm[t], Lsum = pl[t], o0 = po[t][0], o1 = po[t][1];
-    if (nparts > 1 && act) {
-      const long long base = part0 - split + static_cast<long long>(t) * nparts;
-      merge_parts(p.mlpart, p.opart, base, nparts, oh, lane, M, Lsum, o0, o1);
-    }
-    const float inv = Lsum > 0.f ? 1.f / Lsum : 0.f;
-    float r[2] = {o0 * inv, o1 * inv};
+    const float inv = pl[t] > 0.f ? 1.f / pl[t] : 0.f;
+    float r[2] = {po[t][0] * inv, po[t][1] * inv};
     if (p.vmask != nullptr) unrotate(r);
     const int hq = (tile * NT + t) * 4 + oh;
     if (act && hq < p.gqa) {
@@ -453,7 +439,7 @@ int launch_qm(const DecodeParams& p, hipStream_t st) {
   const int ntile = (p.gqa + 7) / 8;
   const int nparts = p.nsplit + ((p.tail != nullptr && !p.fuse_tail) ? 1 : 0);
   if (nparts <= 0 || p.B <= 0) return 0;
-  dim3 grid(p.Hkv * ntile, nparts, p.B);
+  dim3 grid(p.Hkv * ntile, p.B, nparts);
   if (p.page == 32) launch_shape<QM, K2, 32>(p, grid, ntile, nparts, st);
   else launch_shape<QM, K2, 16>(p, grid, ntile, nparts, st);
   return hipPeekAtLastError() == hipSuccess ? 0 : -1;

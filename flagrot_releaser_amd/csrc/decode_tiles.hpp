@@ -71,6 +71,13 @@ struct Smem {
 DEVI int kslot(int isB, int i) { return 2 * (2 * (i & 1) + isB) + (i >> 1); }
 DEVI int vslot(int r8) { return 2 * (r8 & 3) + (r8 >> 2); }
 
+// the lane's share (elements 4 (lane & 31) + i) of query head hq of a GQA group
+DEVI uint2 query_row(const DecodeParams& p, int b, int kvh, int hq) {
+  if (hq >= p.gqa) return make_uint2(0u, 0u);
+  return *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p.q) + static_cast<long long>(b) * p.q_bs +
+                                         (static_cast<long long>(kvh) * p.gqa + hq) * 128 + 4 * (threadIdx.x & 31));
+}
+
 // Rotates the q tile three ways and stores it as the A operands of the score products: rows = (head, variant), per
 // 32-group j and k block (= quarter tg of a code row) the eight elements in the order the masked code words give
 // them.  An element is held as an fp16 pair (value + what its rounding left), both times 2^4 and divided by the
@@ -78,17 +85,11 @@ DEVI int vslot(int r8) { return 2 * (r8 & 3) + (r8 >> 2); }
 // groups of the 2-bit words).  The third operand removes the zero points: -(sum of the group's elements as held).
 // Wavefronts 0..3: one head each; half 0 writes the rows of variants 0 (identity, or the static kmask rotation) and
 // 1 (H32), half 1 those of variant 2 (H128) and the idle row 3; rows of variants a format does not use are zero.
+// raw: the lane's four elements (query_row, zero past the group's heads), requested at the start of the kernel.
 template <int QM, bool K2, class SM>
-DEVI void q_prologue(SM& S, const DecodeParams& p, int b, int kvh, int tile) {
+DEVI void q_prologue(SM& S, const DecodeParams& p, uint2 raw, int kvh) {
   const int w = threadIdx.x >> 6, half = (threadIdx.x >> 5) & 1, l32 = threadIdx.x & 31;
-  const int hq = tile * 4 + w;                       // head inside the GQA group
-  float x[4] = {0.f, 0.f, 0.f, 0.f};
-  if (hq < p.gqa) {
-    const uint16_t* qr = static_cast<const uint16_t*>(p.q) + static_cast<long long>(b) * p.q_bs +
-                         (static_cast<long long>(kvh) * p.gqa + hq) * 128 + 4 * l32;
-    const uint2 raw = *reinterpret_cast<const uint2*>(qr);
-    x[0] = bf16_lo(raw.x); x[1] = bf16_hi(raw.x); x[2] = bf16_lo(raw.y); x[3] = bf16_hi(raw.y);
-  }
+  const float x[4] = {bf16_lo(raw.x), bf16_hi(raw.x), bf16_lo(raw.y), bf16_hi(raw.y)};
   const int g = l32 >> 3, isB = (l32 >> 2) & 1, tg = l32 & 3;   // the lane's dims 4 l32 + i: group, word half, quarter
   float y[4] = {x[0], x[1], x[2], x[3]};
   if (half == 0) fwht<32>(y, l32); else fwht<128>(y, l32);
@@ -249,33 +250,47 @@ DEVI void load_v(VRegs<QM>& r, const uint8_t* const (&chunk)[QBLK<QM>], int lane
 // again in place of those past the end, with weight 0); the running maximum moves from batch to batch and what was
 // summed so far is rescaled with it.  One partial per turn of a loop waits a memory latency per turn (32 splits then
 // took 20 of the 28 us of a single-sequence launch), and a pass for the maxima ahead of the sums is one latency more.
+// Pairs of neighbouring floats (channels, maximum and sum) move eight bytes at a time, NT tiles together: their partials
+// follow one another in the workspace.
+DEVI float2 load_shared_pair(const float* q) {       // read through to what all XCDs see
+  const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(q), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return make_float2(__uint_as_float(static_cast<uint32_t>(v)), __uint_as_float(static_cast<uint32_t>(v >> 32)));
+}
+DEVI void store_shared_pair(float* q, float a, float b) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(q),
+                     __float_as_uint(a) | (static_cast<unsigned long long>(__float_as_uint(b)) << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int NT>
 DEVI void merge_parts(const float* mlpart, const float* opart, long long base, int nparts, int oh, int lane,
-                      float& M, float& Lsum, float& o0, float& o1) {
-  constexpr int NB = 8;
-  auto ld = [](const float* q) { return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  M = -INFINITY; Lsum = 0.f; o0 = 0.f; o1 = 0.f;
+                      float (&M)[NT], float (&Lsum)[NT], float (&o)[NT][2]) {
+  constexpr int NB = 8 / NT;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) { M[t] = -INFINITY; Lsum[t] = 0.f; o[t][0] = o[t][1] = 0.f; }
   for (int s0 = 0; s0 < nparts; s0 += NB) {
-    float m[NB], l[NB], a[NB], c[NB];
+    float2 ml[NT][NB], x[NT][NB];
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const long long part = base + min(s0 + k, nparts - 1);
-      m[k] = ld(mlpart + part * 8 + 2 * oh);
-      l[k] = ld(mlpart + part * 8 + 2 * oh + 1);
-      a[k] = ld(opart + part * 512 + oh * 128 + 2 * lane);
-      c[k] = ld(opart + part * 512 + oh * 128 + 2 * lane + 1);
-    }
-    float top = M;
+    for (int k = 0; k < NB; ++k)
 #pragma unroll
-    for (int k = 0; k < NB; ++k) top = fmaxf(top, m[k]);          // (a partial read twice changes no maximum)
-    const float keep = M == -INFINITY ? 0.f : fexp2(M - top);      // nothing summed yet, or top is finite
-    M = top;
-    Lsum *= keep; o0 *= keep; o1 *= keep;
+      for (int t = 0; t < NT; ++t) {
+        const long long part = base + t * nparts + min(s0 + k, nparts - 1);
+        ml[t][k] = load_shared_pair(mlpart + part * 8 + 2 * oh);
+        x[t][k] = load_shared_pair(opart + part * 512 + oh * 128 + 2 * lane);
+      }
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const float f = (s0 + k < nparts && m[k] != -INFINITY) ? fexp2(m[k] - M) : 0.f;
-      Lsum += f * l[k];
-      o0 += f * a[k];
-      o1 += f * c[k];
+    for (int t = 0; t < NT; ++t) {
+      float top = M[t];
+#pragma unroll
+      for (int k = 0; k < NB; ++k) top = fmaxf(top, ml[t][k].x);        // (a partial read twice changes no maximum)
+      const float keep = M[t] == -INFINITY ? 0.f : fexp2(M[t] - top);    // nothing summed yet, or top is finite
+      M[t] = top;
+      Lsum[t] *= keep; o[t][0] *= keep; o[t][1] *= keep;
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const float f = (s0 + k < nparts && ml[t][k].x != -INFINITY) ? fexp2(ml[t][k].x - M[t]) : 0.f;
+        Lsum[t] += f * ml[t][k].y;
+        o[t][0] += f * x[t][k].x;
+        o[t][1] += f * x[t][k].y;
+      }
     }
   }
 }
@@ -751,19 +766,16 @@ struct WaveState8 {          // WaveState for the two halves of the tile
 
 // q_prologue for a tile of 8 heads: head hh (0..7) is prepared by wavefront hh (workgroups of fewer wavefronts take
 // several heads in turn) into the operand tables of half hh >> 2, rows of head hh & 3.
+// raw: the lane's elements of the wavefront's heads (query_row), requested at the start of the kernel.
+template <int NW> constexpr int Q8_TURNS = NW < 8 ? 8 / NW : 1;
 template <int QM, bool K2, int NW, class SM>
-DEVI void q_prologue8(SM& S, const DecodeParams& p, int b, int kvh, int tile) {
+DEVI void q_prologue8(SM& S, const DecodeParams& p, const uint2 (&raw)[Q8_TURNS<NW>], int kvh) {
   const int wv = threadIdx.x >> 6, half = (threadIdx.x >> 5) & 1, l32 = threadIdx.x & 31;
-  for (int hh = wv; hh < 8; hh += NW) {
-  const int th = hh >> 2, w = hh & 3;
-  const int hq = tile * 8 + hh;                      // head inside the GQA group
-  float x[4] = {0.f, 0.f, 0.f, 0.f};
-  if (hq < p.gqa) {
-    const uint16_t* qr = static_cast<const uint16_t*>(p.q) + static_cast<long long>(b) * p.q_bs +
-                         (static_cast<long long>(kvh) * p.gqa + hq) * 128 + 4 * l32;
-    const uint2 raw = *reinterpret_cast<const uint2*>(qr);
-    x[0] = bf16_lo(raw.x); x[1] = bf16_hi(raw.x); x[2] = bf16_lo(raw.y); x[3] = bf16_hi(raw.y);
-  }
+#pragma unroll
+  for (int turn = 0; turn < Q8_TURNS<NW>; ++turn) {
+  const int hh = wv + turn * NW, th = hh >> 2, w = hh & 3;
+  if (hh >= 8) break;
+  const float x[4] = {bf16_lo(raw[turn].x), bf16_hi(raw[turn].x), bf16_lo(raw[turn].y), bf16_hi(raw[turn].y)};
   const int g = l32 >> 3, isB = (l32 >> 2) & 1, tg = l32 & 3;
   float y[4] = {x[0], x[1], x[2], x[3]};
   if (half == 0) fwht<32>(y, l32); else fwht<128>(y, l32);
@@ -1088,7 +1100,8 @@ DEVI void tail_partial(const DecodeParams& p, int b, int kvh, int tile, float* p
   float lp[4];
 #pragma unroll
   for (int h = 0; h < 4; ++h) { m[h] = -INFINITY; lp[h] = 0.f; o[h][0] = o[h][1] = 0.f; }
-  for (int t0 = wave * 16; t0 < n; t0 += NW * 16) {
+  // (from the last wavefront down: where the pages leave wavefronts idle those are the last ones)
+  for (int t0 = (NW - 1 - wave) * 16; t0 < n; t0 += NW * 16) {
     const uint16_t* kr = base + static_cast<long long>(min(t0 + col, n - 1)) * p.tail_ts + kvh * 128 + 8 * kb;
     uint4 kk[4];
 #pragma unroll
