@@ -204,6 +204,10 @@ class StepPlan:
     group_src: torch.Tensor | None = None    # kivi2: [n, 32] int64 flat ring rows of the key group this step completes (-1: sink)
     group_dst: torch.Tensor | None = None    # kivi2: [n, 32] int64 page slots of that group ([:, 0] < 0: none completes)
 
+    def table_of(self, n: int):
+        """the block-table rows of n queries (a view only where there are more)"""
+        return self.block_table if self.block_table.shape[0] == n else self.block_table[:n]
+
 
 class StepPlanner:
     """per-step bookkeeping of a decode batch (one query token per row).  `ring_rows` request rows + one spare row that
@@ -369,10 +373,10 @@ class DecodeLayer:
         if q.stride(1) != D or q.stride(2) != 1:
             q = q.contiguous()
         if self.static:
-            K.v2_attn(q, self.pool, sp.block_table[:n], sp.page_tokens, out, sp.nsplit, sp.chunk, self.ws, self.qscale,
+            K.v2_attn(q, self.pool, sp.table_of(n), sp.page_tokens, out, sp.nsplit, sp.chunk, self.ws, self.qscale,
                       kmask=self.kmask, vmask=self.vmask, rb=32, fmt=self.kind, **extra)
         else:
-            K.cb_attn(q, self.pool, sp.block_table[:n], sp.page_tokens, out, sp.nsplit, sp.chunk, self.ws, self.qscale,
+            K.cb_attn(q, self.pool, sp.table_of(n), sp.page_tokens, out, sp.nsplit, sp.chunk, self.ws, self.qscale,
                       self.kind, **extra)
 
     def step(self, q, kv, sp: StepPlan, out):
@@ -445,7 +449,7 @@ class KiviDecodeLayer:
         n = q.shape[0]
         if q.stride(1) != D or q.stride(2) != 1:
             q = q.contiguous()
-        KIVI.attn(q, self.pool, sp.block_table[:n], sp.page_tokens, out, sp.nsplit, sp.chunk, self.ws,
+        KIVI.attn(q, self.pool, sp.table_of(n), sp.page_tokens, out, sp.nsplit, sp.chunk, self.ws,
                   self.scale * LOG2E, self.geo.S, self.G, ring=self.ring, tail_len=sp.ring_tokens,
                   tail_idx=sp.ring_home, T=self.geo.slots, f8=self.f8)
 
