@@ -97,9 +97,12 @@ class WorkspacePool:
     def flagrot(self, device, layout, rows: int, plan_fn):
         heads, tile, Dh = layout
         key = ("fr", str(device), heads, tile, Dh)
+        need = self.parts_needed(rows, heads, plan_fn)
         ws = self._held.get(key)
-        if ws is None or ws.rows < rows:
-            ws = self._held[key] = K.Workspace(rows, heads, self.parts_needed(rows, heads, plan_fn), device, tile, Dh)
+        if ws is None or ws.rows < rows or ws.parts < need:       # (fewer rows of longer contexts may have more splits)
+            if ws is not None:
+                rows, need = max(rows, ws.rows), max(need, ws.parts)
+            ws = self._held[key] = K.Workspace(rows, heads, need, device, tile, Dh)
         return ws
 
     def kivi(self, device, rows: int, Hkv: int, G: int, Dh: int, plan_fn):

@@ -104,3 +104,12 @@ def test_chunk_key_groups_against_a_position_walk(S, W):
                         assert a - p <= W, "an earlier position must still be in the window"
                         want = -2 - (req * T + S + (p - S) % W)
                     assert int(src[i, j]) == want, (req, a, b, g, j)
+
+
+def test_shared_workspace_grows_for_more_splits():
+    """layers of a second planner with fewer rows but longer contexts (more splits) share the pool: what they get holds both"""
+    pool = BK.WorkspacePool()
+    first = pool.flagrot("cpu", (2, 4, 128), 8, lambda rows: (2, 512))
+    second = pool.flagrot("cpu", (2, 4, 128), 2, lambda rows: (32, 1024))
+    assert second.fits(2, 2, 33) and second.fits(8, 2, 3) and not first.fits(2, 2, 33)
+    assert pool.flagrot("cpu", (2, 4, 128), 8, lambda rows: (2, 512)) is second
