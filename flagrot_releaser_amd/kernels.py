@@ -408,15 +408,19 @@ def cb_attn_noalloc(q, pool, block_table, seq_lens, out, nsplit, chunk, qscale, 
     return _decode("fr_cb_attn_noalloc", args, bound)
 
 
-def ring_of(kv, ring, dest) -> int:
-    """the number of rows of a ring that rows kv may be copied into, at rows dest if given"""
-    T, heads, Dh = kv.shape
+def ring_of(kv, heads, Dh, ring) -> int:
+    """the number of rows of a ring that rows kv [T, heads, Dh] may be copied into"""
     assert kv.dtype == torch.bfloat16 and ring.dtype == torch.bfloat16 and ring.is_contiguous()
     assert ring.shape[-2:] == (heads, Dh) and heads % 2 == 0 and ring.device == kv.device and ring.data_ptr() % 8 == 0, \
         "ring: rows of kv's shape, on its device, 8-byte aligned"
-    assert dest is None or (dest.dtype == torch.int64 and dest.is_contiguous() and dest.shape == (T,)
-                            and dest.device == kv.device), "dest: int64 [T], contiguous, on the rows' device"
     return ring.numel() // (heads * Dh)
+
+
+def ring_rows_named(dest, T, device):
+    """the ring row of every token, checked"""
+    assert dest.dtype == torch.int64 and dest.is_contiguous() and dest.shape == (T,) and dest.device == device, \
+        "dest: int64 [T], contiguous, on the rows' device"
+    return dest
 
 
 def step_write(kv, slots, fmt, pool, page, ring, dest, mask=None, CT=None, kmu=None):
@@ -425,7 +429,7 @@ def step_write(kv, slots, fmt, pool, page, ring, dest, mask=None, CT=None, kmu=N
     T, heads, Dh = kv.shape
     if T == 0:
         return
-    have = ring_of(kv, ring, dest)
+    have, dest = ring_of(kv, heads, Dh, ring), ring_rows_named(dest, T, kv.device)
     assert Dh == D and slots.dtype == torch.int64
     rows = _loadable(kv)
     NATIVE.run("fr_step_write", V2_FMT[fmt], rows, rows.stride(0), slots.contiguous(), T, heads // 2, page, mask, CT, pool,
@@ -441,10 +445,12 @@ def ring_rows(kv, ring, kmu=None, dest=None, base=0, sink=0, window=0, start=0):
     T, heads, Dh = kv.shape
     if T == 0:
         return
-    rows, have = _loadable(kv), ring_of(kv, ring, dest)
+    rows, have = _loadable(kv), ring_of(kv, heads, Dh, ring)
     if dest is None:
         base, start = operator.index(base), operator.index(start)
         assert 0 <= base and base + sink + window <= have, "the request's rows lie outside the ring"
+    else:
+        ring_rows_named(dest, T, kv.device)
     NATIVE.run("fr_ring_rows", rows, rows.stride(0), T, heads // 2, Dh, _centre(kmu, rows), ring, dest,
                base, sink, window, start, current_stream(), have)
 
