@@ -26,6 +26,7 @@
 #include "fr_common.hpp"
 #include "fr_unpack.hpp"
 #include "mq_launch.hpp"
+#include "mq_rows256.hpp"
 #include "mq_tiles.hpp"
 
 namespace frmq {
@@ -43,7 +44,6 @@ __global__ void __launch_bounds__(64 * NW, 2) k_mq(const Params p) {
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int item = blockIdx.x, h = blockIdx.y;
   const Work work(p, item, ROWS);
-  const int G = p.G, Hq = p.Hkv * G;
   const int* bt = work.block_table;
   const int kend = work.key_end, kb0 = work.block0, kb1 = work.block1;
   const Consts cst = make_consts();
@@ -51,21 +51,18 @@ __global__ void __launch_bounds__(64 * NW, 2) k_mq(const Params p) {
   // this lane's query row
   const int r = 32 * wv + l32;
   const bool rvalid = work.has_row(r);
-  const int lim = rvalid ? work.last_key(r / G) : -1;
+  const int lim = rvalid ? work.last_key(work.token_of(r)) : -1;
 
   // page ids of the first blocks (published by the barriers of the q staging below)
   int cb = kb0;
   auto fill_pages = [&]() { fill_page_window<NT>(S.pages, bt, cb, kb1, kend, tid); };
+  QRows<NT, ROWS> rows;
+  rows.request(p, work, h, D, 0, tid);                 // in flight together with the page ids
   fill_pages();
 
   // q fragments: the tile through LDS (natural order), gathered in code-word order
   u32x4 qf[8];
-  for (int row = tid >> 5; row < ROWS; row += NT / 32) {
-    const int t = row / G, lq = tid & 31;
-    u32x2 raw = {0u, 0u};
-    if (work.has_row(row)) raw = gload<u32x2>(p.q + (static_cast<long long>(work.compact_row + t) * Hq + h * G + row % G) * D + 4 * lq);
-    *reinterpret_cast<u32x2*>(lds + row * QROW + 8 * lq) = raw;
-  }
+  rows.store(lds, work, tid);
   __syncthreads();
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
@@ -147,104 +144,6 @@ struct Smem8 {
 };
 static_assert(256 * QROW <= 2 * (KT_BYTES + VT_BYTES), "q staging aliases the tiles");
 
-// Raw page words of a thread's tile entry, one register set for both groups (a set per group would let the compiler
-// reuse the other group's registers for LDS operands and guard them with waits on outstanding fetches):
-//   group A  w[0] = K code words of (token, tg) (INT2: .x .y), w[1].xy = the token's four K scale words,
-//            w[1].z = the token's group-0 V scale word (whole-head flag of key-only pages)
-//   group B  w[0] = V^T entry (e, c8) of a page, w[1], w[2] = V scale words of the entry's run (eight tokens) in its
-//            two groups: t0 t2 | t4 t6 | t1 t3 | t5 t7
-struct Raw8 {
-  u32x4 w[3];
-};
-
-// A wavefront of the group fetches one page of the block (page = its index in the group): the page base is
-// wave-uniform, the lane adds a 32-bit offset.  Lane = (token pos = lane >> 2, quarter tg) for the K words.
-template <int QM, bool K2>
-DEVI void load_k8(Raw8& R, const Params& p, const int* pg, int h, int kb, int kend, int t256) {
-  using F = Fmt<QM>;
-  const uint32_t lane = t256 & 63, pos = lane >> 2, tg = lane & 3u;
-  const int pgi = __builtin_amdgcn_readfirstlane(t256 >> 6);
-  const int j0 = kb * BN + PAGE * pgi;
-  if (j0 + static_cast<int>(pos) < kend) {
-    const int page = __builtin_amdgcn_readfirstlane(pg[pgi]);
-    const uint8_t* ch = p.pool + static_cast<long long>(page) * p.page_stride + static_cast<long long>(h) * F::CHUNK;
-    if constexpr (QM == QM_ASYM2) {
-      const u32x2 c = gload<u32x2>(ch + (32u * (pos ^ ((pos >> 1) & 2u)) + 8u * tg));
-      R.w[0] = u32x4{c.x, c.y, 0u, 0u};
-    } else {
-      R.w[0] = gload<u32x4>(ch + 16u * lane);
-    }
-    const u32x2 ks = gload<u32x2>(ch + (F::KS_OFF + 8u * pos));
-    R.w[1].x = ks.x; R.w[1].y = ks.y;
-    if constexpr (K2) R.w[1].z = gload<uint16_t>(ch + (F::VS_OFF + (8u * (pos >> 3) + static_cast<uint32_t>(vs_slot8(pos))) * 2u));
-  }
-}
-template <int QM>
-DEVI void load_v8(Raw8& R, const Params& p, const int* pg, int h, int kb, int kend, int t256) {
-  using F = Fmt<QM>;
-  const uint32_t lane = t256 & 63, g = lane >> 5, c8 = lane & 1u;      // entry e = lane >> 1: its dims lie in groups g, g + 2
-  const int pgi = __builtin_amdgcn_readfirstlane(t256 >> 6);
-  const int j0 = kb * BN + PAGE * pgi;
-  if (j0 < kend) {
-    const int page = __builtin_amdgcn_readfirstlane(pg[pgi]);
-    const uint8_t* ch = p.pool + static_cast<long long>(page) * p.page_stride + static_cast<long long>(h) * F::CHUNK;
-    if constexpr (QM == QM_ASYM2) {
-      const u32x2 c = gload<u32x2>(ch + (F::V_OFF + 8u * lane));
-      R.w[0] = u32x4{c.x, c.y, 0u, 0u};
-    } else {
-      R.w[0] = gload<u32x4>(ch + (F::V_OFF + 16u * lane));
-    }
-    R.w[1] = gload<u32x4>(ch + (F::VS_OFF + (g * PAGE + 8u * c8) * 2u));
-    R.w[2] = gload<u32x4>(ch + (F::VS_OFF + ((g + 2u) * PAGE + 8u * c8) * 2u));
-  }
-}
-
-// V^T tile entry: the scale / zero point pairs of the entry's run come from the thread's own scale words, in the run
-// order (t0,t4) (t1,t5) (t2,t6) (t3,t7); tokens at or beyond kend get scale 0
-template <int QM>
-DEVI void convert_v8(uint8_t* vt, const Raw8& R, int kb, int kend, const Consts& cst, int t256) {
-  using F = Fmt<QM>;
-  const int pgi = t256 >> 6, e = (t256 & 63) >> 1, c8 = t256 & 1, run = 2 * pgi + c8;
-  const bool have = kb * BN + PAGE * pgi < kend;
-  const bool ragged = kb * BN + BN > kend;                         // uniform: only the last block of an item
-  uint32_t w[4] = {0u, 0u, 0u, 0u};
-  if (have) {
-    if constexpr (QM == QM_ASYM2) {
-      w[0] = R.w[0].x; w[1] = R.w[0].x >> 4; w[2] = R.w[0].y; w[3] = R.w[0].y >> 4;
-    } else {
-      w[0] = R.w[0].x; w[1] = R.w[0].y; w[2] = R.w[0].z; w[3] = R.w[0].w;
-    }
-  }
-  uint32_t sc[2][4], nz[2][4];
-#pragma unroll
-  for (int gg = 0; gg < 2; ++gg) {
-    const u32x4 v = R.w[1 + gg];
-    const uint32_t pr[4] = {__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
-                            __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u)};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      sc[gg][i] = have ? pr[i] & 0x7FFF7FFFu : 0u;
-      nz[gg][i] = (pr[i] & (F::ZM * 0x10001u)) | 0xE400E400u;
-    }
-  }
-  if (ragged) {
-    const int t0 = kb * BN + 8 * run;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t m = (t0 + i < kend ? 0xFFFFu : 0u) | (t0 + i + 4 < kend ? 0xFFFF0000u : 0u);
-      sc[0][i] &= m; sc[1][i] &= m;
-    }
-  }
-#pragma unroll
-  for (int sub = 0; sub < 4; ++sub) {
-    const int d = 64 * (sub >> 1) + 16 * (e >> 3) + 8 * (sub & 1) + (e & 7);   // group d >> 5 = 2 (sub >> 1) + (e >> 4)
-    uint32_t x[4];
-    Unpack<QM>::run(w[sub], nz[sub >> 1], cst, x);
-    *reinterpret_cast<u32x4*>(vt + d * VROW + 16 * run) =
-        u32x4{pk_mul(x[0], sc[sub >> 1][0]), pk_mul(x[1], sc[sub >> 1][1]), pk_mul(x[2], sc[sub >> 1][2]), pk_mul(x[3], sc[sub >> 1][3])};
-  }
-}
-
 // The 256-row kernel keeps a per-row REFERENCE instead of the running maximum: the score accumulators start at
 // -reference (qk8), so that exp2 applies to them as they are; the reference moves (and O, l are rescaled) only when a
 // score exceeds it by more than 2^8, which keeps p <= 256 in fp16.  Any reference gives the same O / l; the partial's
@@ -280,57 +179,6 @@ DEVI void qk8(const uint8_t* kt, const u32x4 (&qf)[8], f32x16 (&sacc)[2], float 
   __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
 }
 
-// lane = row, lanes l and l + 32 hold the two halves of its 64 keys; sacc = score - reference.  full: no key of the
-// block is masked for any row of the wavefront.
-DEVI void softmax8(f32x16 (&sacc)[2], u32x4 (&pb)[4], f32x16 (&o)[4], float& ref, float& lrow, bool full, int kb, int lim,
-                   int kmin, int hh) {
-  if (!full) {
-    const int jb = kb * BN;
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int j = jb + 32 * kt + token_of_acc(i, hh);
-        if (!(j <= lim && j >= kmin)) sacc[kt][i] = -INFINITY;
-      }
-  }
-  float mx = -INFINITY;
-#pragma unroll
-  for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[kt][i]);
-  mx = max_halves(mx);
-  const bool bump = (mx > 8.f || ref == -INFINITY) && mx != -INFINITY;
-  if (__any(bump)) {                                     // rare after the first blocks: move the reference to the row maximum
-    const float delta = bump ? mx : 0.f;
-    const float alpha = ref == -INFINITY ? 0.f : fexp2(-delta);   // no reference yet: O and l are still zero
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sacc[kt][i] -= delta;
-#pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
-    lrow *= alpha;
-    if (bump) ref = (ref == -INFINITY ? 0.f : ref) + delta;
-  }
-  typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-  const h2v ones = {static_cast<_Float16>(1.f), static_cast<_Float16>(1.f)};
-  float s4[4] = {0.f, 0.f, 0.f, 0.f};                   // the sum of what the value product uses
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {      // ks = 2 kt + s
-    const int kt = ks >> 1, s2 = ks & 1;
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = pack_h2_rn(fexp2(sacc[kt][8 * s2 + 2 * j]), fexp2(sacc[kt][8 * s2 + 2 * j + 1]));
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s4[j] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2v, w[j]), ones, s4[j], false);
-    pb[ks] = u32x4{w[0], w[1], w[2], w[3]};
-  }
-  lrow += (s4[0] + s4[1]) + (s4[2] + s4[3]);
-}
-
 template <int QM, bool K2>
 __global__ void __launch_bounds__(512, 1) k_mq8(const Params p) {
   constexpr int NT = 512, ROWS = 256;
@@ -340,26 +188,26 @@ __global__ void __launch_bounds__(512, 1) k_mq8(const Params p) {
   const int grp = __builtin_amdgcn_readfirstlane(wv >> 2);
   const int item = blockIdx.x, h = blockIdx.y;
   const Work work(p, item, ROWS);
-  const int G = p.G, Hq = p.Hkv * G;
   const int* bt = work.block_table;
   const int kend = work.key_end, kb0 = work.block0, kb1 = work.block1;
   const Consts cst = make_consts();
 
   const int r = 32 * wv + l32;
   const bool rvalid = work.has_row(r);
-  const int lim = rvalid ? work.last_key(r / G) : -1;
+  const int lim = rvalid ? work.last_key(work.token_of(r)) : -1;
 
   int cb = kb0;
   auto fill_pages = [&]() { fill_page_window<NT>(S.pages, bt, cb, kb1, kend, tid); };
   fill_pages();
+  QRows<NT, ROWS> rows;
+  rows.request(p, work, h, D, 0, tid);
 
   u32x4 qf[8];
-  for (int row = tid >> 5; row < ROWS; row += NT / 32) {
-    const int t = row / G, lq = tid & 31;
-    u32x2 raw = {0u, 0u};
-    if (work.has_row(row)) raw = gload<u32x2>(p.q + (static_cast<long long>(work.compact_row + t) * Hq + h * G + row % G) * D + 4 * lq);
-    *reinterpret_cast<u32x2*>(lds + row * QROW + 8 * lq) = raw;
-  }
+  __syncthreads();                                     // the page ids
+  Raw8 raw;                                            // fetched at the end of a matrix slot, converted in the next vector slot
+  if (grp == 0) load_k8<QM, K2>(raw, p, S.pages, h, kb0, kend, tid_now() & 255);
+  else load_v8<QM>(raw, p, S.pages, h, kb0, kend, tid_now() & 255);
+  rows.store(lds, work, tid);
   __syncthreads();
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
@@ -389,16 +237,11 @@ __global__ void __launch_bounds__(512, 1) k_mq8(const Params p) {
     for (int i = 0; i < 16; ++i) sacc[t][i] = -INFINITY;
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) pb[ks] = u32x4{0u, 0u, 0u, 0u};
-  Raw8 raw;                                            // fetched at the end of a matrix slot, converted in the next vector slot
   const int nb = kb1 - kb0;                            // blocks of the item
   __syncthreads();                                     // the q staging is no longer read
   for (int i = tid; i < 2 * VT_BYTES / 16; i += NT) reinterpret_cast<u32x4*>(&S.vt[0][0])[i] = u32x4{0u, 0u, 0u, 0u};
-  if (grp == 0) {                                      // K(0) before the first slot
-    load_k8<QM, K2>(raw, p, S.pages, h, kb0, kend, tid_now() & 255);
+  if (grp == 0)                                        // K(0) before the first slot
     convert_k_entry<QM, K2>(S.kt[0], tid_now() & 255, raw.w[0], u32x2{raw.w[1].x, raw.w[1].y}, K2 ? raw.w[1].z : 0u, kb0, kend, cst);
-  } else {
-    load_v8<QM>(raw, p, S.pages, h, kb0, kend, tid_now() & 255);
-  }
   __syncthreads();
 
   auto slot_barrier = [&]() {                          // nothing of a slot may move into the next one

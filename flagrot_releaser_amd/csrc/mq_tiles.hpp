@@ -21,6 +21,20 @@ constexpr int KT_BYTES = BN * KROW, VT_BYTES = D * VROW;
 constexpr int QROW = 264;                    // bytes per staged q row (natural order)
 constexpr int PG_CACHE = 1024;               // page ids kept in LDS (256 blocks of 64 keys)
 
+// Where a tile keeps the 16-byte piece c of K row `row` (16 pieces a row) and the run of eight keys of V^T row d (8 runs a row):
+// padded rows for tiles that are converted where they are read, and the rows side by side with their pieces permuted for
+// the images that travel through memory and are copied to LDS as they are -- 16 rows' pieces c lie in 64 different banks
+// either way.
+struct Padded {
+  static DEVI int k(int row, int c) { return row * KROW + 16 * c; }
+  static DEVI int v(int d, int run) { return d * VROW + 16 * run; }
+};
+struct Image {
+  static constexpr int K_BYTES = BN * 256, V_BYTES = D * 128, BYTES = K_BYTES + V_BYTES;
+  static DEVI int k(int row, int c) { return row * 256 + ((c ^ (row & 15)) << 4); }
+  static DEVI int v(int d, int run) { return d * 128 + ((run ^ ((d >> 1) & 7)) << 4); }
+};
+
 struct Smem {
   alignas(16) uint8_t kt[KT_BYTES];
   alignas(16) uint8_t vt[VT_BYTES];
@@ -66,7 +80,11 @@ struct Work {
     block0 = irec[1];
     block1 = key_end > block0 * BN ? (key_end + BN - 1) / BN : block0;
     rows_used = min(rows / p.G, tokens) * p.G;
+    per_row = (65536u + static_cast<uint32_t>(p.G) - 1u) / static_cast<uint32_t>(p.G);
   }
+  uint32_t per_row;         // ceil(2^16 / G): token of a row without a division
+
+  DEVI int token_of(int row) const { return static_cast<int>((static_cast<uint32_t>(row) * per_row) >> 16); }   // rows, G <= 256: exact
   DEVI bool has_row(int row) const { return row < rows_used; }
   DEVI int last_key(int token) const { return min(key_end - 1, max(first_pos + token - shift, reach)); }
 };
@@ -75,6 +93,35 @@ struct Work {
 template <typename T> DEVI T gload(const void* p) {
   return *reinterpret_cast<const __attribute__((address_space(1))) T*>(reinterpret_cast<uintptr_t>(p));
 }
+// The tile's query rows (row r = token r / G, head r % G; `width` channels a row, 128 of them from channel `first` on) on their
+// way to LDS: a thread's eight bytes of 16 rows, all requested before the first is stored.  (A loop that stores each as it
+// comes waits a memory latency and two integer divisions per row: 16 new tokens of 256-d heads over 1376 cached ones 33.7 us.)
+template <int NT, int ROWS>
+struct QRows {
+  static constexpr int N = ROWS / (NT / 32);
+  u32x2 raw[N];
+  DEVI void request(const Params& p, const Work& work, int h, int width, int first, int tid) {
+    const uint16_t* tile = p.q + (static_cast<long long>(work.compact_row) * p.Hkv + h) * p.G * width + first + 4 * (tid & 31);
+    const int last = work.rows_used - 1;                 // (rows past it: that one again, zeroed)
+    if (last < 0) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) raw[i] = u32x2{0u, 0u};
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int row = min((tid >> 5) + i * (NT / 32), last), t = work.token_of(row);
+      raw[i] = gload<u32x2>(tile + static_cast<long long>(t * p.Hkv * p.G + (row - t * p.G)) * width);
+    }
+  }
+  DEVI void store(uint8_t* lds, const Work& work, int tid) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int row = (tid >> 5) + i * (NT / 32);
+      *reinterpret_cast<u32x2*>(lds + row * QROW + 8 * (tid & 31)) = work.has_row(row) ? raw[i] : u32x2{0u, 0u};
+    }
+  }
+};
 DEVI float fexp2(float x) { return __builtin_amdgcn_exp2f(x); }
 DEVI half8 as_h8(u32x4 v) { return __builtin_bit_cast(half8, v); }
 DEVI uint32_t pack_h2(float a, float b) {
@@ -295,17 +342,17 @@ DEVI void k2_values(const u32x4 kc, const u32x2 sw, bool whole, int tg, const Co
 }
 
 // K tile entry idx = (token tk = idx >> 2 of the block, quarter tg = idx & 3) from the token's raw words
-template <int QM, bool K2>
+template <int QM, bool K2, class At = Padded>
 DEVI void convert_k_entry(uint8_t* kt, int idx, const u32x4 kc, const u32x2 sw, uint32_t vf, int kb, int kend, const Consts& cst) {
   using F = Fmt<QM>;
   {
     const int tk = idx >> 2, tg = idx & 3;
     const int j = kb * BN + tk;
     const int row = 32 * (tk >> 5) + krow_of_token(tk & 31);
-    u32x4* dst = reinterpret_cast<u32x4*>(kt + row * KROW);
+    auto put = [&](int g, const u32x4 v) { *reinterpret_cast<u32x4*>(kt + At::k(row, 4 * g + tg)) = v; };
     if (j >= kend) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) dst[4 * g + tg] = u32x4{0u, 0u, 0u, 0u};
+      for (int g = 0; g < 4; ++g) put(g, u32x4{0u, 0u, 0u, 0u});
       return;
     }
     uint32_t w[4];
@@ -322,7 +369,7 @@ DEVI void convert_k_entry(uint8_t* kt, int idx, const u32x4 kc, const u32x2 sw, 
         const uint32_t nz[4] = {z, z, z, z};
         uint32_t x[4];
         Unpack<QM>::run(w[g], nz, cst, x);
-        dst[4 * g + tg] = u32x4{pk_mul(x[0], sc), pk_mul(x[1], sc), pk_mul(x[2], sc), pk_mul(x[3], sc)};
+        put(g, u32x4{pk_mul(x[0], sc), pk_mul(x[1], sc), pk_mul(x[2], sc), pk_mul(x[3], sc)});
       }
     } else {
       // key-only pages: the token's flags select identity / H32 per group / whole-head H128 (the quad of a token agrees)
@@ -331,7 +378,7 @@ DEVI void convert_k_entry(uint8_t* kt, int idx, const u32x4 kc, const u32x2 sw, 
       bool rot[4];
       k2_values<QM, 128>(kc, sw, ff, tg, cst, v, rot);
 #pragma unroll
-      for (int g = 0; g < 4; ++g) dst[4 * g + tg] = u32x4{v[g][0], v[g][1], v[g][2], v[g][3]};
+      for (int g = 0; g < 4; ++g) put(g, u32x4{v[g][0], v[g][1], v[g][2], v[g][3]});
     }
   }
 }

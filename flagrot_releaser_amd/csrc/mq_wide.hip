@@ -70,17 +70,19 @@ __global__ void __launch_bounds__(256, 2) k_mq256(const Params p) {
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int item = blockIdx.x, h = blockIdx.y, vz = blockIdx.z;
   const Work work(p, item, ROWS);
-  const int G = p.G, Hq = p.Hkv * G;
   const int* bt = work.block_table;
   const int kend = work.key_end, kb0 = work.block0, kb1 = work.block1;
   const Consts cst = make_consts();
 
   const int r = 32 * wv + l32;
   const bool rvalid = work.has_row(r);
-  const int lim = rvalid ? work.last_key(r / G) : -1;
+  const int lim = rvalid ? work.last_key(work.token_of(r)) : -1;
 
   int cb = kb0;
   auto fill_pages = [&]() { fill_page_window<NT>(S.pages, bt, cb, kb1, kend, tid); };
+  QRows<NT, ROWS> rows[2];
+  rows[0].request(p, work, h, DW, 0, tid);             // in flight together with the page ids
+  rows[1].request(p, work, h, DW, 128, tid);
   fill_pages();
 
   // q fragments of both halves: the tile through LDS (natural order), gathered in code-word order
@@ -88,13 +90,7 @@ __global__ void __launch_bounds__(256, 2) k_mq256(const Params p) {
 #pragma unroll
   for (int s2 = 0; s2 < 2; ++s2) {
     if (s2) __syncthreads();
-    for (int row = tid >> 5; row < ROWS; row += NT / 32) {
-      const int t = row / G, lq = tid & 31;
-      u32x2 raw = {0u, 0u};
-      if (work.has_row(row))
-        raw = gload<u32x2>(p.q + (static_cast<long long>(work.compact_row + t) * Hq + h * G + row % G) * DW + 128 * s2 + 4 * lq);
-      *reinterpret_cast<u32x2*>(lds + row * QROW + 8 * lq) = raw;
-    }
+    rows[s2].store(lds, work, tid);
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
