@@ -723,6 +723,22 @@ int frmq_attn(const void* q16, const uint8_t* pool, long long page_stride, const
   return done(rc, "frmq_attn");
 }
 
+int frmq_image_bytes(void) { return image_bytes(); }
+
+int frmq_attn_images(const void* q16, const uint8_t* pool, long long page_stride, const int* bt, long long bt_stride,
+                     const int* tiles, const int* items, int nitems, const int* tile_block, const int* recs, int nblocks, int Hkv,
+                     int G, int shift, int konly, uint8_t* images, int heads, float* opart, float* ml, void* stream, int kmin) {
+  if (nitems <= 0) return 0;
+  if (G < 1 || G > 256) return bad(-3, "frmq_attn_images: G out of range");
+  if (nblocks < 1 || heads < 1) return bad(-3, "frmq_attn_images: at least one block and one head");
+  if (reinterpret_cast<uintptr_t>(images) & 15u) return bad(-3, "frmq_attn_images: images must be 16-byte aligned");
+  Params p{};
+  p.q = static_cast<const uint16_t*>(q16); p.pool = pool; p.page_stride = page_stride; p.bt = bt; p.bt_stride = bt_stride;
+  p.tiles = tiles; p.items = items; p.Hkv = Hkv; p.G = G; p.shift = shift; p.kmin = kmin; p.opart = opart; p.ml = ml;
+  return done(images_attn_launch(p, nitems, konly, tile_block, recs, nblocks, images, heads, static_cast<hipStream_t>(stream)),
+              "frmq_attn_images");
+}
+
 int frmq_merge(const int* tiles, int ntiles, const float* opart, const float* ml, int Hkv, int G, int rows, void* out,
                long long o_ts, int out_fp32, float* lse, long long lse_ts, int Dh, void* stream) {
   if (ntiles <= 0) return 0;

@@ -42,6 +42,8 @@ NATIVE = Library("mq", "FLAGROT_MQ_LIB", "frmq_abi_version", ABI, "frmq_last_err
     "frmq_smem_bytes": "",
     "frmq_prep_q": "p i l p i i i p p f p i p",
     "frmq_attn": "p p l p l p p i i i i i p p i i p i",
+    "frmq_image_bytes": "",
+    "frmq_attn_images": "p p l p l p p i p p i i i i i p i p p p i",
     "frmq_merge": "p i p p i i i p l i p l i p",
     "frmq_win_gather": "p i p p p l p l i p p i p",
     "frmq_bf_merge": "i i i p l p p p p p p p p p i i f p l i p",
@@ -82,7 +84,8 @@ def num_sms(device) -> int:
 @dataclass
 class Plan:
     """One step's work list.  `buf` (int32, on the device) holds, back to back: the tile records [ntiles, 9], the item
-    records [nitems, 4] and the output row of each of the m compact query rows.  A tile record is (block-table row,
+    records [nitems, 4], the output row of each of the m compact query rows and, with nblocks, every tile's first block record
+    [ntiles] and the block records [nblocks, 4] (image_arrays).  A tile record is (block-table row,
     first compact row, first output row, tokens, position of the first token, page keys of the request, first item,
     items, extra visible key or a large negative number); an item record is (tile, first key block, end key block, 0).
     `reqs` keeps the requests in the order their rows were compacted; `rows` is the number of query rows a workgroup of
@@ -96,6 +99,7 @@ class Plan:
     rows: int = 128
     D: int = 128
     kmin: int = 0
+    nblocks: int = 0                # blocks whose tile images key-only pages make first; 0: every tile converts what it reads
 
     def _span(self, start: int, count: int):
         return self.buf[start:start + count]
@@ -111,6 +115,15 @@ class Plan:
     @property
     def idx(self):
         return self._span(self.ntiles * TILE_INTS + self.nitems * ITEM_INTS, self.m)
+
+    @property
+    def tile_block(self):
+        """the first block record of every tile"""
+        return self._span(self.ntiles * TILE_INTS + self.nitems * ITEM_INTS + self.m, self.ntiles)
+
+    @property
+    def block_recs(self):
+        return self._span(self.ntiles * (TILE_INTS + 1) + self.nitems * ITEM_INTS + self.m, self.nblocks * BLOCK_INTS)
 
 
 _W = os.environ.get("FLAGROT_MQ_WAVES")                         # grid target: WAVES x the resident workgroups of the GPU;
@@ -197,6 +210,42 @@ def plan_arrays(reqs, G: int, Hkv: int, shift: int, ncu: int, kernel: int = KERN
     return T, I, out_row.astype(np.int32), rows
 
 
+BLOCK_INTS = 4
+IMAGE = 32768                   # bytes of a block's tile images (one KV head)
+# Key-only pages of heavy calls take the images: their conversion (rotations undone per token and block) is paid once per
+# request instead of once per query tile, for 32 KB written per block and head and two more launches.  us direct / by images,
+# 8 KV heads, 4-bit key-only pages: 4 requests x 16 tiles over 16 k 1345 / 1046 + 72 for the images; 1 x 16 tiles over 8 k
+# (17 k reads of a block by a tile and head, 15 per block) 189 / 164; 4 x 6 over 8 k (25 k, 6) 282 / 260; 4 x 16 over 1 k
+# (12.5 k, 12) 176 / 138; 8 x 4 over 4 k (17 k, 4) 174 / 168; below: 4 x 8 over 1 k (5 k, 7) 69 / 71, 1 x 8 over 2 k (2 k, 7)
+# 42 / 43, 4 x 2 over 1 k (1 k, 2) 27 / 40.  Static pages convert fast enough to lose (1 x 16 over 8 k 155 / 165).
+IMAGE_READS = int(os.environ.get("FLAGROT_MQ_IMAGE_READS", "12000"))            # reads of a block by a tile and KV head
+IMAGE_REUSE = float(os.environ.get("FLAGROT_MQ_IMAGE_REUSE", "4"))              # ... per block
+IMAGE_BYTES = int(os.environ.get("FLAGROT_MQ_IMAGE_BYTES", str(192 << 20)))     # room for images per call: they stay in the caches
+
+
+def image_arrays(T, I):
+    """Which blocks of which requests the tiles read: (first block record of every tile int32 [nt], block records int32
+    [nblocks, 4] = (block-table row, block, page keys of the request, 0)).  Tiles of one request share its blocks."""
+    reach = I[T[:, T_ITEM0] + T[:, T_NITEMS] - 1, I_KB1]                                            # blocks a tile reads
+    reqs, owner = np.unique(T[:, [T_BTROW, T_NKEYS]], axis=0, return_inverse=True)
+    owner = owner.reshape(-1)
+    blocks = np.zeros(len(reqs), dtype=np.int64)
+    np.maximum.at(blocks, owner, reach)
+    first = np.cumsum(blocks) - blocks
+    of = np.repeat(np.arange(len(reqs)), blocks)
+    recs = np.zeros((of.size, BLOCK_INTS), dtype=np.int32)
+    recs[:, 0], recs[:, 1], recs[:, 2] = reqs[of, 0], np.arange(of.size) - first[of], reqs[of, 1]
+    return first[owner].astype(np.int32), recs
+
+
+def image_heads(plan, Hkv: int, ncu: int) -> int:
+    """KV heads per pass over the images: of what IMAGE_BYTES have room for, the number with the fewest rounds of workgroups
+    (one per CU) over all passes, the larger one on ties"""
+    room = min(Hkv, max(1, IMAGE_BYTES // (plan.nblocks * IMAGE)))
+    rounds = lambda n: -(-plan.nitems * n // ncu)                                                    # noqa: E731
+    return min(range(room, 0, -1), key=lambda n: Hkv // n * rounds(n) + (rounds(Hkv % n) if Hkv % n else 0))
+
+
 def build_plan(reqs, G: int, Hkv: int, shift: int, device, sink: int = 0, kernel: int | None = None,
                waves: float | None = None, min_blocks: int | None = None, D: int = D, ext: dict | None = None) -> Plan:
     """plan_arrays for the GPU `device`, uploaded as one int32 tensor.  sink: keys [0, sink) are masked in the kernel
@@ -206,9 +255,15 @@ def build_plan(reqs, G: int, Hkv: int, shift: int, device, sink: int = 0, kernel
     kernel = 3 if D == 256 else kernel or KERNEL or pick_kernel(reqs, G)     # head dim 256: one kernel, 128-row tiles
     T, I, out_row, rows = plan_arrays(reqs, G, Hkv, shift, num_sms(device), kernel, WAVES if waves is None else waves,
                                       MIN_BLOCKS if min_blocks is None else min_blocks, ext)
-    packed = torch.from_numpy(np.concatenate([T.ravel(), I.ravel(), out_row]))
+    parts, nblocks, reads = [T.ravel(), I.ravel(), out_row], 0, int((I[:, I_KB1] - I[:, I_KB0]).sum())
+    if kernel == 4 and reads * Hkv >= IMAGE_READS:
+        tile_block, recs = image_arrays(T, I)
+        if len(recs) * IMAGE <= IMAGE_BYTES and reads >= IMAGE_REUSE * len(recs):
+            parts += [tile_block, recs.ravel()]
+            nblocks = len(recs)
+    packed = torch.from_numpy(np.concatenate(parts))
     return Plan(ntiles=len(T), nitems=len(I), m=len(out_row), buf=packed.to(device), reqs=reqs, kernel=kernel, rows=rows,
-                D=D, kmin=int(sink))
+                D=D, kmin=int(sink), nblocks=nblocks)
 
 
 # ------------------------------------------------------------------------------------------------ launches
@@ -237,7 +292,8 @@ def attn(q16, pool, bt, plan: Plan, G: int, shift: int, konly: bool, int2: bool 
     """The page part of the attention, still split by item: (opart fp32 [items, Hkv, rows, D], unnormalised;
     ml fp32 [items, Hkv, rows, 2] = running maximum in log2 units and sum).  pool uint8 [pages, Hkv, chunk bytes] (at
     head dim 256 a chunk is two 128-d half chunks), bt int32 block table, q16 from prep_q; konly: key-only-rotated page
-    kinds; int2: 2-bit codes (80-byte tokens per 128 dims)."""
+    kinds; int2: 2-bit codes (80-byte tokens per 128 dims).  Plans with block records: up to IMAGE_BYTES of device memory hold
+    the images of their tiles during the call."""
     Hkv, Dh = pool.shape[1], q16.shape[2]
     token_bytes = 80 if int2 else 144
     assert Dh == plan.D, (Dh, plan.D)
@@ -246,6 +302,13 @@ def attn(q16, pool, bt, plan: Plan, G: int, shift: int, konly: bool, int2: bool 
     assert q16.dtype == torch.float16 and q16.is_contiguous() and q16.shape[1] == Hkv * G
     opart = q16.new_empty((plan.nitems, Hkv, plan.rows, Dh), dtype=torch.float32)
     ml = q16.new_empty((plan.nitems, Hkv, plan.rows, 2), dtype=torch.float32)
+    if konly and plan.nblocks:
+        heads = image_heads(plan, Hkv, num_sms(q16.device))
+        images = q16.new_empty(heads * plan.nblocks * IMAGE, dtype=torch.uint8)
+        NATIVE.run("frmq_attn_images", q16, pool, pool.stride(0), bt, bt.stride(0), plan.tiles, plan.items, plan.nitems,
+                   plan.tile_block, plan.block_recs, plan.nblocks, Hkv, G, shift, int(konly) + 2 * int(int2), images, heads,
+                   opart, ml, current_stream(), plan.kmin)
+        return opart, ml
     NATIVE.run("frmq_attn", q16, pool, pool.stride(0), bt, bt.stride(0), plan.tiles, plan.items, plan.nitems, Hkv, G,
                shift, int(konly) + 2 * int(int2), opart, ml, plan.kernel, Dh, current_stream(), plan.kmin)
     return opart, ml

@@ -43,6 +43,16 @@ int frmq_attn(const void* q16, const uint8_t* pool, long long page_stride, const
               const int* tiles, const int* items, int nitems, int Hkv, int G, int shift, int konly, float* opart,
               float* ml, int kernel, int Dh, void* stream, int kmin);
 
+/* No counterpart in the reference.  frmq_attn with kernel 4 at head dim 128 (same arguments, same partials) for plans whose
+ * tiles read the same blocks several times: every block of a request is turned into an image of its fp16 tiles once
+ * (frmq_image_bytes() bytes per block and KV head), `heads` KV heads at a time, and the tiles read the images.  recs int32
+ * [nblocks, 4]: (block-table row, 64-key block, page keys of the request, 0); tile_block int32 [ntiles]: the record of the
+ * tile's block 0 (its blocks follow one another); images: heads * nblocks images, 16-byte aligned, overwritten. */
+int frmq_image_bytes(void);
+int frmq_attn_images(const void* q16, const uint8_t* pool, long long page_stride, const int* bt, long long bt_stride,
+                     const int* tiles, const int* items, int nitems, const int* tile_block, const int* recs, int nblocks, int Hkv,
+                     int G, int shift, int konly, uint8_t* images, int heads, float* opart, float* ml, void* stream, int kmin);
+
 /* mq_prefill.cu:1546-1559.  Combines the items of each tile: out_fp32 = 0: bf16 rows out[(orow0 + t) * o_ts + hq * Dh];
  * 1: fp32 compact rows out[((crow0 + t) * Hq + hq) * Dh]; lse (or null): natural-log sums [Hq][lse_ts], -inf for rows
  * without a visible key. */

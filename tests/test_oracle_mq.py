@@ -194,3 +194,25 @@ def test_bf_merge_is_attention_over_the_union():
             assert np.allclose(out[c][hq], (p @ V[js, hq // G]) / p.sum(), atol=1e-10)
     kw, vw = OM.win_gather(np.array([(2 << 32) | 3, (0 << 32) | 1, (1 << 32) | 0]), sk[0], sk[0][::-1], K, V, Hkv)
     assert np.array_equal(kw[0], K[3]) and np.array_equal(vw[1], V[1]) and np.array_equal(kw[2], K[S - 1])
+
+
+def test_image_arrays_name_every_block_once():
+    from flagrot_releaser_amd import prefill_mq as MQ
+    reqs = [(3, 0, 200, 900, 700), (1, 200, 260, 60, 0), (3, 260, 300, 400, 360)]
+    T, I, _, _ = MQ.plan_arrays(reqs, 4, 2, 0, 256, kernel=4)
+    tile_block, recs = MQ.image_arrays(T, I)
+    assert len({tuple(r) for r in recs.tolist()}) == len(recs) and tile_block.dtype == recs.dtype == np.int32
+    for item in I:
+        t = T[item[0]]
+        for kb in range(item[1], item[2]):                              # every block an item reads is the record it is looked for at
+            assert recs[tile_block[item[0]] + kb].tolist() == [t[0], kb, t[5], 0]
+
+
+def test_image_heads_fit_and_share_the_rounds():
+    from flagrot_releaser_amd import prefill_mq as MQ
+    plan = MQ.Plan(ntiles=0, nitems=64, m=0, buf=None, reqs=[], nblocks=1056)
+    assert MQ.image_heads(plan, 8, 256) == 4                            # five have room, two passes of four have no idle CU
+    plan.nitems, plan.nblocks = 31, 20
+    assert MQ.image_heads(plan, 8, 256) == 8
+    plan.nblocks = MQ.IMAGE_BYTES // MQ.IMAGE
+    assert MQ.image_heads(plan, 8, 256) == 1
