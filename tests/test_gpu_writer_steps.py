@@ -65,6 +65,16 @@ def test_steps_write_the_bytes_of_small_calls(dev, kind, D, Hkv, T, steps, page)
     check(kind, D, Hkv, T, page)
 
 
+# prompts of few pairs: half a step of 8 tokens a workgroup while that makes 256 workgroups at most, a whole step beyond; first
+# and last of the range, rests of one token
+@pytest.mark.parametrize("D,Hkv,T,half", [(128, 8, 129, True), (128, 8, 256, True), (128, 8, 257, False), (128, 1, 1031, True),
+                                          (256, 4, 257, True), (256, 2, 1024, True), (256, 2, 1025, False)])
+@pytest.mark.parametrize("kind,page", [("konly", 32), ("konlya2", 16)])
+def test_half_steps_write_the_bytes_of_small_calls(dev, kind, page, D, Hkv, T, half):
+    assert T * Hkv > 1024 and (-(-T // 8) * Hkv <= 256) == half
+    check(kind, D, Hkv, T, page)
+
+
 @pytest.mark.parametrize("env", [{"FLAGROT_W3": "2"}, {"FLAGROT_W3_KAPPA": "0.1"}], ids=["every token exact", "a tenth of the bound"])
 def test_screen_at_its_ends(dev, env):
     """FLAGROT_W3=2: every token takes the exact path at the end, full lists of undecided tokens.  FLAGROT_W3_KAPPA=0.1: the
