@@ -79,7 +79,7 @@ struct ScreenSmem {
   int fb[SCR_MAXTILE], nfb;
 };
 
-template <int QM, int P, int D>
+template <int QM, int P, int D, int TURNS>
 __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2WriteParams p, int tile, float kappa) {
   using L = Lay<QM, P>;
   constexpr int LU = D / 4, NB = D / 32, KB = D / 16;     // lanes of a token, 32-blocks, K blocks of the matrix product
@@ -110,14 +110,13 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
   for (int tb0 = t_lo; tb0 < t_hi; tb0 += SCR_TOK) {
     uint32_t nosign = 0x7FFF7FFFu;
     asm volatile("" : "+s"(nosign));            // (the magnitudes of C are not hoisted out of the loop into registers)
-    // ---- P1: candidates and value rows of the unit's two tokens, eight apart; a workgroup of eight tokens has one each (and
-    // the second one's columns hold whatever was there: a column is its token's alone)
+    // ---- P1: candidates and value rows of the unit's two tokens; a workgroup of eight tokens has one each (and the other
+    // eight columns hold whatever was there: a column is its token's alone)
     // (a loop, not two copies: with the copies 24 registers spill, 108 -> 105 us; a loop over the candidates too: 112)
-    const int turns = t_hi - tb0 > SCR_TOK / 2 ? 2 : 1;
-    if (turns == 1 && lu == 0) S.slot[unit + SCR_TOK / 2] = -1;
+    if (TURNS == 1 && lu == 0) S.slot[unit + SCR_TOK / 2] = -1;
 #pragma unroll 1
-    for (int u = 0; u < turns; ++u) {
-      const int tk = unit + SCR_TOK / 2 * u, t = tb0 + tk;
+    for (int u = 0; u < TURNS; ++u) {
+      const int tk = TURNS * unit + u, t = tb0 + tk;
       long long slot = -1;
       if (t < t_hi) slot = p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)];
       if (lu == 0) S.slot[tk] = slot;
@@ -259,8 +258,8 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
     __syncthreads();
     // ---- P4: base against whole head; the rows of the decided tokens into their pages
 #pragma unroll 1
-    for (int u = 0; u < turns; ++u) {
-      const int tk = unit + SCR_TOK / 2 * u;
+    for (int u = 0; u < TURNS; ++u) {
+      const int tk = TURNS * unit + u;
       const long long slot = S.slot[tk];
       float e[2], b[2];
 #pragma unroll
@@ -320,12 +319,15 @@ int screen(const K2WriteParams& p, float kappa, hipStream_t st) {
   constexpr long long RESIDENT = D == 128 ? 768 : 256;
   const long long steps = (p.T + SCR_TOK - 1) / SCR_TOK, fit = (steps * p.Hkv + RESIDENT - 1) / RESIDENT;
   const long long per = D == 128 && fit > 4 ? 2 : fit < SCR_MAXTILE / SCR_TOK ? fit : SCR_MAXTILE / SCR_TOK;
+  // (A kernel of its own for the half steps: with the number of turns as a value both lose, 8192 tokens 95.1 -> 99.5 us.)
   // Short prompts, half a step a workgroup where that leaves every CU one at most: the candidates of one token instead of two
   // in a row (us, whole / half steps: 8 heads of 128, 130 tokens 18.2 / 15.6, 260 17.9 / 17.3, 520 19.9 / 21.0; 4 heads of 256,
   // 260 tokens 31.2 / 25.9, 400 31.7 / 25.5, 520 33.6 / 37.6).
   const bool half = static_cast<long long>((p.T + SCR_TOK / 2 - 1) / (SCR_TOK / 2)) * p.Hkv <= 256;
   const int tile = half ? SCR_TOK / 2 : SCR_TOK * static_cast<int>(per);
-  hipLaunchKernelGGL((k_k2_screen<QM, P, D>), dim3(p.Hkv, (p.T + tile - 1) / tile), dim3(2 * D), 0, st, p, tile, kappa);
+  const dim3 grid(p.Hkv, (p.T + tile - 1) / tile);
+  if (half) hipLaunchKernelGGL((k_k2_screen<QM, P, D, 1>), grid, dim3(2 * D), 0, st, p, tile, kappa);
+  else hipLaunchKernelGGL((k_k2_screen<QM, P, D, 2>), grid, dim3(2 * D), 0, st, p, tile, kappa);
   return hipPeekAtLastError() == hipSuccess ? 0 : -1;
 }
 template <int QM>
