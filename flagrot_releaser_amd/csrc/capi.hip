@@ -183,6 +183,13 @@ int fr_v2_attn(int fmt, const void* q, long long q_bs, const uint8_t* pool, cons
   // each wavefront (us, four against eight: 176 workgroups of 768 tokens 28.7 / 24.1, 32 of 512 20.5 / 18.0; 64 of 256
   // tokens 15.5 / 16.0; 480 of 1664 tokens 68 / 72).
   if (variant & HD256) p.wg_waves = pairs * nparts <= cus && chunk >= 512 ? 8 : 4;
+  // ... and where the plan has one and a half workgroups a CU at least, its parts are shared out by the sequences' lengths
+  // (decode_share.hpp).  Decode and merge of uneven lengths down to a quarter, us, fixed ranges / shared out: 512 workgroups
+  // 58.5 / 49.3, 480 41.5 / 38.8, 392 33.7 / 31.3; below, the parts that come on top would sit beside others on their CU and
+  // the merge is 1.4 longer: 352 35.9 / 36.9, 176 20.3 / 20.9.  Even lengths: 512 59.8 / 60.6, 480 44.0 / 44.8.
+  const char* const plain = getenv("FLAGROT_WIDE_PLAIN");      // (the plain kernel has fixed ranges; read at every call)
+  p.share = (variant & HD256) && !force_static && !(plain != nullptr && plain[0] == '1') && B >= 2 && B <= 64 && nsplit >= 2 &&
+            chunk >= 512 && chunk % 64 == 0 && static_cast<long long>(nsplit) * chunk <= (1ll << 24) && 2 * pairs * nsplit >= 3 * cus;
   if (variant & HD256) return launched(decode_wide_launch(fmt, p, static_cast<hipStream_t>(stream)), "fr_v2_attn (head dim 256)");
   return launched(decode_launch(fmt, p, static_cast<hipStream_t>(stream)), "fr_v2_attn");
 }

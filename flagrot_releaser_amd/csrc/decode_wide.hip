@@ -19,6 +19,7 @@
 #include <cstdlib>
 
 #include "fr_common.hpp"
+#include "decode_share.hpp"
 #include "fr_launch.hpp"
 
 namespace fr {
@@ -260,16 +261,26 @@ __global__ void __launch_bounds__(256) k_wide_merge(const DecodeParams p, int nt
   __shared__ float buf[WD];
   const int kvh = blockIdx.x / ntile, tile = blockIdx.x % ntile, b = blockIdx.y, h = blockIdx.z, hq = tile * 4 + h, d = threadIdx.x;
   if (hq >= p.gqa) return;
-  const long long part0 = ((static_cast<long long>(b) * p.Hkv + kvh) * ntile + tile) * nparts;
+  // partials [first, first + n) of `part0` and, with BF16 rows, one more
+  long long part0 = ((static_cast<long long>(b) * p.Hkv + kvh) * ntile + tile) * nparts;
+  int n = nparts, rows_at = -1;
+  if (p.share) {
+    const Shares sh = share_parts(p, threadIdx.x & 63);
+    const long long all = static_cast<long long>(kvh * ntile + tile) * p.B * nparts;
+    part0 = all + __builtin_amdgcn_readlane(sh.first, b);
+    n = __builtin_amdgcn_readlane(sh.n, b);
+    if (p.tail != nullptr) { rows_at = static_cast<int>(all + p.B * p.nsplit + b - part0); ++n; }
+  }
   const float* ml = p.mlpart + part0 * 8 + 2 * h;
   const float* o = p.opart + part0 * 4 * WD + h * WD + d;
   float M = -INFINITY;
 #pragma unroll 8
-  for (int s = 0; s < nparts; ++s) M = fmaxf(M, ml[8 * s]);
+  for (int i = 0; i < n; ++i) M = fmaxf(M, ml[8 * (rows_at >= 0 && i == n - 1 ? rows_at : i)]);
   float acc = 0.f, Lsum = 0.f;
   if (M != -INFINITY) {
 #pragma unroll 8
-    for (int s = 0; s < nparts; ++s) {
+    for (int i = 0; i < n; ++i) {
+      const int s = rows_at >= 0 && i == n - 1 ? rows_at : i;
       const float ms = ml[8 * s], ls = ml[8 * s + 1], os = o[static_cast<long long>(s) * 4 * WD];
       const bool some = ms != -INFINITY;                        // (an empty split stores no outputs)
       const float f = fexp2w(ms - M);

@@ -13,6 +13,7 @@
 // both; the BF16 sink / window rows are one more split of this grid (plain fp32, a wavefront per row).
 #include <cstddef>
 
+#include "decode_share.hpp"
 #include "decode_tiles.hpp"
 
 namespace fr {
@@ -224,15 +225,23 @@ __global__ void __launch_bounds__(64 * NWW, 2) k_wide_parts_mma(const DecodePara
       kvh = t3 % p.Hkv; split = (t3 / p.Hkv) % nparts; b = t3 / (p.Hkv * nparts);
     }
   }
-  const long long part_id = ((static_cast<long long>(b) * p.Hkv + kvh) * ntile + tile) * nparts + split;
+  const bool is_tail = p.tail != nullptr && split == p.nsplit;
+  long long part_id = ((static_cast<long long>(b) * p.Hkv + kvh) * ntile + tile) * nparts + split;
+  int lo = 0, hi = 0;
+  if (p.share) {                                      // (uniform, as all of it: the scalar unit's)
+    const int slot = is_tail ? p.B * p.nsplit + b : b * p.nsplit + split;
+    part_id = static_cast<long long>(kvh * ntile + tile) * p.B * nparts + slot;
+    if (!is_tail && !share_of(p, lane, slot, b, lo, hi)) return;
+  } else if (!is_tail) {
+    const int len = p.seq_lens[b];
+    lo = max(split * p.chunk, min(p.kv_start, len)); hi = min(len, (split + 1) * p.chunk);
+  }
   float* const op = p.opart + part_id * 4 * 256;
   float* const mlp = p.mlpart + part_id * 8;
-  if (p.tail != nullptr && split == p.nsplit) {
+  if (is_tail) {
     tail_split_wide<QM, K2, NWW>(S, p, b, kvh, tile, op, mlp);
     return;
   }
-  const int len = p.seq_lens[b];
-  const int lo = max(split * p.chunk, min(p.kv_start, len)), hi = min(len, (split + 1) * p.chunk);
   if (lo >= hi) {                                     // uniform: nothing of the range is visible
     if (threadIdx.x < 4) { mlp[2 * threadIdx.x] = -INFINITY; mlp[2 * threadIdx.x + 1] = 0.f; }
     return;
