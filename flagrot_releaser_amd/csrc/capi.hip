@@ -228,6 +228,10 @@ int fr_step_write(int fmt, const void* kv, long long kv_ts, const long long* slo
                   const uint8_t* mask, const float* CT, uint8_t* pool, const float* kmu, void* ring, const long long* dest,
                   long long ring_rows, void* stream) {
   if (T <= 0) return 0;
+  // (without named rows ring_quad would take a prompt's rule, whose window is empty here: a division by zero)
+  if (ring == nullptr || dest == nullptr || Hkv < 1) return fail(-3, "fr_step_write: ring, dest and at least one KV head");
+  const int kind = fmt == FMT_KONLY ? KIND_KONLY : fmt == FMT_KONLYA ? KIND_KONLYA : fmt == FMT_KONLYA2 ? KIND_KONLYA2 : -1;
+  if (kind >= 0 && CT == nullptr) return fail(-3, "fr_step_write: key-only formats choose by CT");
   RingRowsParams r{};
   r.kv = kv; r.kv_ts = kv_ts; r.width = 2 * Hkv * 128; r.kmu = kmu; r.ring = ring; r.ring_rows = ring_rows; r.dest = dest;
   r.rows = r.sinks = T;
@@ -238,7 +242,6 @@ int fr_step_write(int fmt, const void* kv, long long kv_ts, const long long* slo
     p.mask = mask; p.kmu = kmu; p.pool = pool; p.ring = r;
     return launched(static_write_launch(fmt, p, st), "fr_step_write");
   }
-  const int kind = fmt == FMT_KONLY ? KIND_KONLY : fmt == FMT_KONLYA ? KIND_KONLYA : fmt == FMT_KONLYA2 ? KIND_KONLYA2 : -1;
   if (kind < 0) return fail(-4, "fr_step_write: fmt must be 4 .. 9");
   K2WriteParams p{};
   p.kv = kv; p.kv_ts = kv_ts; p.slots = slots; p.T = T; p.Hkv = Hkv; p.page = page;

@@ -53,6 +53,8 @@ int kv_v_write(const void* kv, long long kv_rs, int n, int Hkv, int D, const voi
 int kv_step_write(const void* kv, long long kv_rs, int n, int Hkv, const void* slots, const void* co, void* pool, int f8,
                   void* ring, const void* dest, long long ring_rows, void* stream) {
   if (n <= 0) return 0;
+  // (without named rows ring_quad would take a prompt's rule, whose window is empty here: a division by zero)
+  if (ring == nullptr || dest == nullptr || Hkv < 1) return bad("kv_step_write: ring, dest and at least one KV head");
   fr::RingRowsParams r{};
   r.kv = kv; r.kv_ts = kv_rs; r.width = 2 * Hkv * 128; r.ring = ring; r.ring_rows = ring_rows;
   r.dest = static_cast<const long long*>(dest); r.rows = r.sinks = n;

@@ -60,7 +60,7 @@ int fr_ring_rows(const void* kv, long long kv_ts, int T, int Hkv, int Dh, const 
 
 /* No counterpart in the reference.  The cache update of a decode step in one launch, head dim 128: the bytes that fr_v2_write
  * (fmt 4 | 5 | 8, with mask) or fr_cb_write (fmt 6 | 7 | 9, with CT) store for the rows, and the rows that fr_ring_rows with
- * dest and kmu copies. */
+ * dest and kmu copies.  -3 without ring, dest or a head, or without CT for a key-only format. */
 int fr_step_write(int fmt, const void* kv, long long kv_ts, const long long* slots, int T, int Hkv, int page,
                   const uint8_t* mask, const float* CT, uint8_t* pool, const float* kmu, void* ring, const long long* dest,
                   long long ring_rows, void* stream);

@@ -33,7 +33,8 @@ int kv_v_write(const void* kv, long long kv_rs, int n, int Hkv, int D, const voi
 
 /* No counterpart in the reference.  What a decode step stores of its rows before its key groups, in one launch, D = 128:
  * kv_v_write (co, no M / ident / vfix) and the rows bf16 [n, 2*Hkv, 128] (8-byte aligned) copied to rows dest int64 [n] of ring
- * bf16 [ring_rows, 2*Hkv, 128] (tokens whose row is not in 0 .. ring_rows - 1 are left out of the ring). */
+ * bf16 [ring_rows, 2*Hkv, 128] (tokens whose row is not in 0 .. ring_rows - 1 are left out of the ring).
+ * 2 without ring, dest or a head. */
 int kv_step_write(const void* kv, long long kv_rs, int n, int Hkv, const void* slots, const void* co, void* pool, int f8,
                   void* ring, const void* dest, long long ring_rows, void* stream);
 
