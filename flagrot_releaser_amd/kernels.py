@@ -423,16 +423,22 @@ def ring_rows_named(dest, T, device):
     return dest
 
 
+def step_slots(slots, T, device):
+    """the page slot of every token of a step, checked and packed"""
+    assert slots.dtype == torch.int64 and slots.shape == (T,) and slots.device == device, "slots: int64 [T] on the rows' device"
+    return slots.contiguous()
+
+
 def step_write(kv, slots, fmt, pool, page, ring, dest, mask=None, CT=None, kmu=None):
     """What a decode step stores of its rows, in one launch: v2_write (static formats, with mask) or cb_write (key-only
     kinds, with CT) and ring_rows with dest.  Head dim 128."""
     T, heads, Dh = kv.shape
     if T == 0:
         return
-    have, dest = ring_of(kv, heads, Dh, ring), ring_rows_named(dest, T, kv.device)
-    assert Dh == D and slots.dtype == torch.int64
+    have, dest, slots = ring_of(kv, heads, Dh, ring), ring_rows_named(dest, T, kv.device), step_slots(slots, T, kv.device)
+    assert Dh == D and (fmt not in K2 or CT is not None)
     rows = _loadable(kv)
-    NATIVE.run("fr_step_write", V2_FMT[fmt], rows, rows.stride(0), slots.contiguous(), T, heads // 2, page, mask, CT, pool,
+    NATIVE.run("fr_step_write", V2_FMT[fmt], rows, rows.stride(0), slots, T, heads // 2, page, mask, CT, pool,
                _centre(kmu, rows), ring, dest, have, current_stream())
 
 

@@ -40,3 +40,30 @@ def test_step_writers_refuse_a_missing_ring_row_or_calibration():
         a = {**dict(ring=x, dest=x, H=1), **less}
         rc = KV.NATIVE.ask("kv_step_write", x, 256, 1, a["H"], x, x, x, 0, a["ring"], a["dest"], 4, None)
         assert rc == 2 and KV.NATIVE.last_error().startswith("kv_step_write"), (less, rc)
+
+
+def test_step_writers_take_one_slot_for_every_token(monkeypatch):
+    """the number of tokens is the rows': slots that are fewer, of another shape, strided or elsewhere are not read"""
+    from flagrot_releaser_amd import kivi as KV
+    seen = []
+    for lib in (K, KV):
+        monkeypatch.setattr(lib.NATIVE, "run", lambda name, *a: seen.append((name, a)))
+        monkeypatch.setattr(lib, "current_stream", lambda: 0)
+    T, H = 3, 2
+    kv, ring = torch.zeros(T, 2 * H, 128, dtype=torch.bfloat16), torch.zeros(8, 2 * H, 128, dtype=torch.bfloat16)
+    dest, x = torch.arange(T), torch.zeros(4)
+    calls = [lambda s: K.step_write(kv, s, "int4", x, 16, ring, dest, mask=x), lambda s: K.step_write(kv, s, "konly", x, 16, ring, dest, CT=x),
+             lambda s: KV.step_write(kv, s, x, x, ring, dest)]
+    good = torch.arange(T)
+    for call in calls:
+        for bad in (good[:2], torch.arange(T + 1), good.int(), good.view(T, 1), torch.empty(T, dtype=torch.int64, device="meta")):
+            with pytest.raises(AssertionError):
+                call(bad)
+        assert not seen
+        call(good)
+        call(torch.arange(2 * T)[::2])                                 # every second one: a copy goes to the device
+        packed = [next(t for t in a if isinstance(t, torch.Tensor) and t.dtype == torch.int64) for _, a in seen]
+        assert packed[0].tolist() == [0, 1, 2] and packed[1].tolist() == [0, 2, 4] and packed[1].is_contiguous()
+        seen.clear()
+    with pytest.raises(AssertionError):
+        K.step_write(kv, good, "konly", x, 16, ring, dest)             # key-only pages without their calibration
