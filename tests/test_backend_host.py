@@ -113,3 +113,55 @@ def test_shared_workspace_grows_for_more_splits():
     second = pool.flagrot("cpu", (2, 4, 128), 2, lambda rows: (32, 1024))
     assert second.fits(2, 2, 33) and second.fits(8, 2, 3) and not first.fits(2, 2, 33)
     assert pool.flagrot("cpu", (2, 4, 128), 8, lambda rows: (2, 512)) is second
+
+
+def test_a_step_stores_what_update_stores(monkeypatch):
+    """step() is update() and decode(): a subclass that overrides one of them is asked, and both list the same launches; what
+    the one launch cannot read goes through the writer and the row copy"""
+    calls = []
+    note = lambda name: lambda *a, **kw: calls.append(name)                                          # noqa: E731
+    for mod, names in ((BK.K, ("step_write", "ring_rows", "v2_write", "cb_write", "v2_attn", "cb_attn")),
+                       (BK.KIVI, ("step_write", "v_write", "k_encode", "attn"))):
+        for name in names:
+            monkeypatch.setattr(mod, name, note(f"{mod.__name__.split('.')[-1]}.{name}"))
+    monkeypatch.setattr(BK, "decode_plan", lambda *a, **kw: (1, 64))
+    H, G, n = 2, 4, 3
+    table, lengths = torch.arange(n * 4, dtype=torch.int32).view(n, 4), torch.full((n,), 40, dtype=torch.int32)
+    slots = torch.arange(n)
+    q, kv = torch.zeros(n, H * G, 128, dtype=torch.bfloat16), torch.zeros(n, 2 * H, 128, dtype=torch.bfloat16)
+    odd = torch.zeros(n * 2 * H * 128 + 1, dtype=torch.bfloat16)[1:].view(n, 2 * H, 128)             # rows at 2 bytes from 8
+    for kind in ("int4a", "konlya", "kivi2"):
+        for window in (0, 64):
+            if kind == "kivi2" and not window:
+                continue
+            planner = BK.StepPlanner(kind, H, G, 64, n, n, 0, window, "cpu")
+            sp = planner.prepare(lengths, table, slots, homes=np.arange(n))
+            pool = torch.zeros(n * 4, H, BK.KIVI.chunk_bytes(128) if kind == "kivi2" else 2304, dtype=torch.uint8)
+            monkeypatch.setattr(BK, "kivi_workspace", lambda *a: None)
+            monkeypatch.setattr(BK, "decode_workspace", lambda *a: None)
+            if kind == "kivi2":
+                cls, extra = BK.KiviDecodeLayer, (torch.zeros(H, 4, 128), torch.zeros(H, 4), torch.ones(H, 128))
+                make = lambda c: c(H, G, pool, planner, *extra)                                      # noqa: E731
+            else:
+                extra = dict(CT=torch.zeros(H, 128, 128), co=torch.ones(H, 128), wmask=torch.zeros(2 * H, 4, dtype=torch.uint8))
+                cls, make = BK.DecodeLayer, lambda c: c(kind, H, G, pool, planner, **extra)          # noqa: E731
+            layer = make(cls)
+            layer.update(kv, sp)
+            stored = calls.copy()
+            calls.clear()
+            layer.step(q, kv, sp, None)
+            assert calls[:-1] == stored and calls[-1].endswith("attn")
+            assert any(c.endswith("step_write") for c in stored) == bool(window)
+            calls.clear()
+            more = BK.StepPlan(**{**vars(sp), "slots": torch.arange(n + 2)})                         # more slots than rows
+            layer.step(q, kv, more, None)
+            assert not any(c.endswith("step_write") for c in calls)
+            calls.clear()
+            if kind == "kivi2":
+                layer.step(q, odd, sp, None)
+                assert calls[:2] == ["kivi.v_write", "kernels.ring_rows"]
+                calls.clear()
+            sub = make(type("Sub", (cls,), {"update": note("mine")}))
+            sub.step(q, kv, sp, None)
+            assert calls[0] == "mine" and len(calls) == 2
+            calls.clear()
