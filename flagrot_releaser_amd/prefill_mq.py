@@ -246,6 +246,14 @@ def image_heads(plan, Hkv: int, ncu: int) -> int:
     return min(range(room, 0, -1), key=lambda n: Hkv // n * rounds(n) + (rounds(Hkv % n) if Hkv % n else 0))
 
 
+def image_room(size: int, device):
+    """memory for the images of a call, or None where the device has none left (a cache of pages may hold all the rest)"""
+    try:
+        return torch.empty(size, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def build_plan(reqs, G: int, Hkv: int, shift: int, device, sink: int = 0, kernel: int | None = None,
                waves: float | None = None, min_blocks: int | None = None, D: int = D, ext: dict | None = None) -> Plan:
     """plan_arrays for the GPU `device`, uploaded as one int32 tensor.  sink: keys [0, sink) are masked in the kernel
@@ -293,7 +301,8 @@ def attn(q16, pool, bt, plan: Plan, G: int, shift: int, konly: bool, int2: bool 
     ml fp32 [items, Hkv, rows, 2] = running maximum in log2 units and sum).  pool uint8 [pages, Hkv, chunk bytes] (at
     head dim 256 a chunk is two 128-d half chunks), bt int32 block table, q16 from prep_q; konly: key-only-rotated page
     kinds; int2: 2-bit codes (80-byte tokens per 128 dims).  Plans with block records: up to IMAGE_BYTES of device memory hold
-    the images of their tiles during the call."""
+    the images of their tiles during the call (a captured call's belong to its graph's pool); where they cannot be had, every
+    tile converts what it reads."""
     Hkv, Dh = pool.shape[1], q16.shape[2]
     token_bytes = 80 if int2 else 144
     assert Dh == plan.D, (Dh, plan.D)
@@ -302,9 +311,9 @@ def attn(q16, pool, bt, plan: Plan, G: int, shift: int, konly: bool, int2: bool 
     assert q16.dtype == torch.float16 and q16.is_contiguous() and q16.shape[1] == Hkv * G
     opart = q16.new_empty((plan.nitems, Hkv, plan.rows, Dh), dtype=torch.float32)
     ml = q16.new_empty((plan.nitems, Hkv, plan.rows, 2), dtype=torch.float32)
-    if konly and plan.nblocks:
-        heads = image_heads(plan, Hkv, num_sms(q16.device))
-        images = q16.new_empty(heads * plan.nblocks * IMAGE, dtype=torch.uint8)
+    heads = image_heads(plan, Hkv, num_sms(q16.device)) if konly and plan.nblocks else 0
+    images = image_room(heads * plan.nblocks * IMAGE, q16.device) if heads else None
+    if images is not None:
         NATIVE.run("frmq_attn_images", q16, pool, pool.stride(0), bt, bt.stride(0), plan.tiles, plan.items, plan.nitems,
                    plan.tile_block, plan.block_recs, plan.nblocks, Hkv, G, shift, int(konly) + 2 * int(int2), images, heads,
                    opart, ml, current_stream(), plan.kmin)

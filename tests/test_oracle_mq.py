@@ -216,3 +216,31 @@ def test_image_heads_fit_and_share_the_rounds():
     assert MQ.image_heads(plan, 8, 256) == 8
     plan.nblocks = MQ.IMAGE_BYTES // MQ.IMAGE
     assert MQ.image_heads(plan, 8, 256) == 1
+
+
+def test_images_that_cannot_be_had_are_not_needed(monkeypatch):
+    """no memory for the tile images: the call is the kernel's that needs none, with the same plan"""
+    from flagrot_releaser_amd import prefill_mq as MQ
+    import torch
+    calls = []
+
+    def out_of_memory(*a, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no memory")
+        return torch.zeros(*a[-1:], **kw)
+
+    monkeypatch.setattr(MQ.NATIVE, "run", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(MQ, "current_stream", lambda: 0)
+    monkeypatch.setattr(MQ, "num_sms", lambda device: 256)
+    Hkv, G = 2, 4
+    plan = MQ.build_plan([(0, 0, 512, 4096, 3584)], G, Hkv, 0, "cpu", kernel=4)
+    plan.nblocks = plan.nblocks or 64
+    q16, bt = torch.zeros(512, Hkv * G, 128, dtype=torch.float16), torch.zeros(1, 256, dtype=torch.int32)
+    pool = torch.zeros(256, Hkv, 2304, dtype=torch.uint8)
+    op, ml = MQ.attn(q16, pool, bt, plan, G, 0, True)
+    assert calls == ["frmq_attn_images"]
+    for where, name in ((torch, "empty"), (torch.Tensor, "new_empty")):
+        monkeypatch.setattr(where, name, out_of_memory)
+    again = MQ.attn(q16, pool, bt, plan, G, 0, True)
+    assert calls == ["frmq_attn_images", "frmq_attn"]
+    assert again[0].shape == op.shape and again[1].shape == ml.shape
