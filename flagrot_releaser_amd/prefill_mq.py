@@ -227,14 +227,13 @@ def image_arrays(T, I):
     """Which blocks of which requests the tiles read: (first block record of every tile int32 [nt], block records int32
     [nblocks, 4] = (block-table row, block, page keys of the request, 0)).  Tiles of one request share its blocks."""
     reach = I[T[:, T_ITEM0] + T[:, T_NITEMS] - 1, I_KB1]                                            # blocks a tile reads
-    reqs, owner = np.unique(T[:, [T_BTROW, T_NKEYS]], axis=0, return_inverse=True)
-    owner = owner.reshape(-1)
-    blocks = np.zeros(len(reqs), dtype=np.int64)
+    names, owner = np.unique((T[:, T_BTROW].astype(np.int64) << 32) | T[:, T_NKEYS], return_inverse=True)
+    blocks = np.zeros(names.size, dtype=np.int64)
     np.maximum.at(blocks, owner, reach)
     first = np.cumsum(blocks) - blocks
-    of = np.repeat(np.arange(len(reqs)), blocks)
-    recs = np.zeros((of.size, BLOCK_INTS), dtype=np.int32)
-    recs[:, 0], recs[:, 1], recs[:, 2] = reqs[of, 0], np.arange(of.size) - first[of], reqs[of, 1]
+    recs = np.zeros((int(blocks.sum()), BLOCK_INTS), dtype=np.int32)
+    recs[:, 0], recs[:, 2] = np.repeat(names >> 32, blocks), np.repeat(names & 0xFFFFFFFF, blocks)
+    recs[:, 1] = np.arange(len(recs)) - np.repeat(first, blocks)
     return first[owner].astype(np.int32), recs
 
 
@@ -255,16 +254,18 @@ def image_room(size: int, device):
 
 
 def build_plan(reqs, G: int, Hkv: int, shift: int, device, sink: int = 0, kernel: int | None = None,
-               waves: float | None = None, min_blocks: int | None = None, D: int = D, ext: dict | None = None) -> Plan:
+               waves: float | None = None, min_blocks: int | None = None, D: int = D, ext: dict | None = None, konly: bool = True) -> Plan:
     """plan_arrays for the GPU `device`, uploaded as one int32 tensor.  sink: keys [0, sink) are masked in the kernel
-    (the BF16 sink part covers them); kernel None: pick_kernel."""
+    (the BF16 sink part covers them); kernel None: pick_kernel.  konly False: the pages are of a static format, which has no use
+    for the block records of heavy calls (the plan does for either kind with them; 64 tiles over 16 k: 145 us of host time
+    without, 210 with)."""
     assert D in (128, 256), D
     reqs = list(reqs)
     kernel = 3 if D == 256 else kernel or KERNEL or pick_kernel(reqs, G)     # head dim 256: one kernel, 128-row tiles
     T, I, out_row, rows = plan_arrays(reqs, G, Hkv, shift, num_sms(device), kernel, WAVES if waves is None else waves,
                                       MIN_BLOCKS if min_blocks is None else min_blocks, ext)
     parts, nblocks, reads = [T.ravel(), I.ravel(), out_row], 0, int((I[:, I_KB1] - I[:, I_KB0]).sum())
-    if kernel == 4 and reads * Hkv >= IMAGE_READS:
+    if konly and kernel == 4 and reads * Hkv >= IMAGE_READS:
         tile_block, recs = image_arrays(T, I)
         if len(recs) * IMAGE <= IMAGE_BYTES and reads >= IMAGE_REUSE * len(recs):
             parts += [tile_block, recs.ravel()]

@@ -244,3 +244,14 @@ def test_images_that_cannot_be_had_are_not_needed(monkeypatch):
     again = MQ.attn(q16, pool, bt, plan, G, 0, True)
     assert calls == ["frmq_attn_images", "frmq_attn"]
     assert again[0].shape == op.shape and again[1].shape == ml.shape
+
+
+def test_plans_of_static_pages_carry_no_block_records(monkeypatch):
+    from flagrot_releaser_amd import prefill_mq as MQ
+    monkeypatch.setattr(MQ, "num_sms", lambda device: 256)
+    reqs = [(r, 512 * r, 512 * (r + 1), 4096 + 512, 4096) for r in range(4)]
+    heavy = MQ.build_plan(reqs, 8, 8, 0, "cpu")
+    static = MQ.build_plan(reqs, 8, 8, 0, "cpu", konly=False)
+    assert heavy.nblocks == 4 * 72 and static.nblocks == 0
+    assert static.buf.numel() == heavy.buf.numel() - heavy.ntiles - 4 * heavy.nblocks
+    assert (heavy.buf[:static.buf.numel()] == static.buf).all()
