@@ -174,6 +174,9 @@ int fr_v2_attn(int fmt, const void* q, long long q_bs, const uint8_t* pool, cons
   // the split merge goes through the caller's workspace: partials, their (max, sum) pairs and, at head dim 128, the ticket
   if (nparts > 1 && (opart == nullptr || mlpart == nullptr || (!(variant & HD256) && counter == nullptr)))
     return fail(-3, "fr_v2_attn: more than one partial per (sequence, KV head) needs opart, mlpart and counter");
+  // (neighbouring channels, and a maximum and its sum, cross workgroups as one 8-byte access: store_shared_pair)
+  if (nparts > 1 && !(variant & HD256) && ((reinterpret_cast<uintptr_t>(opart) | reinterpret_cast<uintptr_t>(mlpart)) & 7u) != 0)
+    return fail(-3, "fr_v2_attn: opart and mlpart must be 8-byte aligned");
   if ((variant & HD256) && (opart == nullptr || mlpart == nullptr))
     return fail(-3, "fr_v2_attn: the head dim 256 kernels need opart and mlpart");
   p.wg_waves = big ? decode_waves(1 << 30) : 4;

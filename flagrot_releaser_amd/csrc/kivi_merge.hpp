@@ -30,7 +30,7 @@ __global__ void __launch_bounds__(MERGE_SLICES * D / 4) k_merge_parts(const floa
     for (int i = 0; i < 8; ++i) {      // past the last partial: the slice's first one again, skipped below
       const bool in = s0 + i * MERGE_SLICES <= NS;
       const long long at = (p0 + (in ? s0 + i * MERGE_SLICES : s0)) * G + g;
-      st[i] = *reinterpret_cast<const float2*>(ml + at * 2);
+      __builtin_memcpy(&st[i], ml + at * 2, sizeof(float2));       // (ml may start at any float; opart is written 16 bytes at a time)
       x[i] = *reinterpret_cast<const float4*>(opart + at * D + 4 * lane);
       if (!in) st[i].x = -INFINITY;
     }

@@ -28,7 +28,8 @@ int fr_abi_version(void);
  * With a tail at head dim 128, q and tail must be 16-byte aligned and q_bs, tail_bs, tail_ts multiples of 8 elements
  * (the rows are operands of matrix instructions, read 16 bytes at a time; contiguous torch tensors always are): -3 if not.
  * nsplit counts the body splits; with a tail the workspace must hold B*Hkv*ceil(gqa/GT)*(nsplit+1) partials of
- * GT*128 floats (GT = 8 when variant has bits 1024|2048, else 4); counter int32 [B*Hkv*ceil(gqa/GT)] zeroed once by the
+ * GT*128 floats (GT = 8 when variant has bits 1024|2048, else 4), opart and mlpart 8-byte aligned (-3 if not; at head dim 256
+ * opart 16-byte); counter int32 [B*Hkv*ceil(gqa/GT)] zeroed once by the
  * caller (merge tickets and, when the body workgroups of a sequence share its page range, their page draws; the last
  * arriving workgroup leaves the word at 0).  If B*Hkv*ceil(gqa/GT)*nsplit fits the CUs and chunk >= 1024, split s owns
  * tokens [s, s+1)*chunk and one large workgroup per CU runs it; otherwise nsplit only counts the workgroups per

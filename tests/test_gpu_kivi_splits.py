@@ -22,6 +22,7 @@ def test_merge_of_splits(dev, ns, hd):
     q = torch.randn(3, Hkv * G, hd, generator=g).bfloat16().to(dev)
     num = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)                                  # noqa: E731
     ws = KV.Workspace(3 * Hkv * (ns + 1), G, hd, dev)
+    ws.ml = torch.cat([ws.ml, ws.ml[:1]])[1:]                                                       # pairs at 4 bytes from 8
     out = torch.full((3, Hkv * G * hd + 3), 7.0, dtype=torch.bfloat16, device=dev)                  # rows of an odd stride
     KV.attn(q, pool, bt.to(dev), num(lens), out[:, :-3], ns, 32, ws, math.log2(math.e) / math.sqrt(hd), 33, G, ring=ring,
             tail_len=num(tails), tail_idx=num([2, 0, 1]), T=T)

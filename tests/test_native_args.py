@@ -67,3 +67,17 @@ def test_step_writers_take_one_slot_for_every_token(monkeypatch):
         seen.clear()
     with pytest.raises(AssertionError):
         K.step_write(kv, good, "konly", x, 16, ring, dest)             # key-only pages without their calibration
+
+
+def test_partials_that_pairs_cannot_be_stored_to_are_refused():
+    """head dim 128, more than one partial: outputs and (maximum, sum) move eight bytes at a time"""
+    x = torch.zeros(64, dtype=torch.int64)
+    at = x.data_ptr()
+
+    def call(opart, mlpart, nsplit=2, variant=264):
+        return K.NATIVE.ask("fr_v2_attn", 5, at, 512, at, at, 4, at, 1, 1, 16, nsplit, 8192, 1.0, None, None, 32, 0, 0, variant, 4, opart,
+                            mlpart, at, at, 512, None, None, None, 0, 0, None, 4, 0)
+
+    for bad in ((at + 4, at), (at, at + 4), (at + 12, at + 4)):
+        assert call(*bad) == -3 and "8-byte" in K.NATIVE.last_error()
+    assert call(at + 4, at, nsplit=3, variant=264 | K.GEN) == -3
