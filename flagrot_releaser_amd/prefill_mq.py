@@ -218,6 +218,11 @@ IMAGE = 32768                   # bytes of a block's tile images (one KV head)
 # (17 k reads of a block by a tile and head, 15 per block) 189 / 164; 4 x 6 over 8 k (25 k, 6) 282 / 260; 4 x 16 over 1 k
 # (12.5 k, 12) 176 / 138; 8 x 4 over 4 k (17 k, 4) 174 / 168; below: 4 x 8 over 1 k (5 k, 7) 69 / 71, 1 x 8 over 2 k (2 k, 7)
 # 42 / 43, 4 x 2 over 1 k (1 k, 2) 27 / 40.  Static pages convert fast enough to lose (1 x 16 over 8 k 155 / 165).
+# The same line on 2-bit pages and on ranks of 4 and 2 heads (groups of 4 and 8, 150 plans on it: 1.00 to 1.72 times as fast):
+# 2-bit, 8 heads 4 x 16 over 4 k 363 / 302, 1 x 16 over 8 k 168 / 161; 4 heads, 4-bit 2 x 64 over 2 k 389 / 275, 2-bit 2 x 16
+# over 8 k 167 / 156; 2 heads, 4-bit 4 x 8 over 12 k 127 / 119, 2-bit 123 / 118.  Where the images have room for some of the heads
+# only, several passes may need more rounds of workgroups than one launch for all heads: then the launch stays (4 x 8 over 12 k,
+# 32 items x 8 heads in one round, room for 7 heads: 460 / 686, 2-bit 447 / 677).
 IMAGE_READS = int(os.environ.get("FLAGROT_MQ_IMAGE_READS", "12000"))            # reads of a block by a tile and KV head
 IMAGE_REUSE = float(os.environ.get("FLAGROT_MQ_IMAGE_REUSE", "4"))              # ... per block
 IMAGE_BYTES = int(os.environ.get("FLAGROT_MQ_IMAGE_BYTES", str(192 << 20)))     # room for images per call: they stay in the caches
@@ -237,12 +242,21 @@ def image_arrays(T, I):
     return first[owner].astype(np.int32), recs
 
 
-def image_heads(plan, Hkv: int, ncu: int) -> int:
+def image_rounds(nitems: int, Hkv: int, heads: int, ncu: int) -> int:
+    """rounds of workgroups (one per CU) of all passes over the images, `heads` KV heads a pass"""
+    whole, rest = divmod(Hkv, heads)
+    return whole * -(-nitems * heads // ncu) + -(-nitems * rest // ncu)
+
+
+def heads_per_pass(nitems: int, nblocks: int, Hkv: int, ncu: int) -> int:
     """KV heads per pass over the images: of what IMAGE_BYTES have room for, the number with the fewest rounds of workgroups
-    (one per CU) over all passes, the larger one on ties"""
-    room = min(Hkv, max(1, IMAGE_BYTES // (plan.nblocks * IMAGE)))
-    rounds = lambda n: -(-plan.nitems * n // ncu)                                                    # noqa: E731
-    return min(range(room, 0, -1), key=lambda n: Hkv // n * rounds(n) + (rounds(Hkv % n) if Hkv % n else 0))
+    over all passes, the larger one on ties"""
+    room = min(Hkv, max(1, IMAGE_BYTES // (nblocks * IMAGE)))
+    return min(range(room, 0, -1), key=lambda n: image_rounds(nitems, Hkv, n, ncu))
+
+
+def image_heads(plan, Hkv: int, ncu: int) -> int:
+    return heads_per_pass(plan.nitems, plan.nblocks, Hkv, ncu)
 
 
 def image_room(size: int, device):
@@ -267,9 +281,11 @@ def build_plan(reqs, G: int, Hkv: int, shift: int, device, sink: int = 0, kernel
     parts, nblocks, reads = [T.ravel(), I.ravel(), out_row], 0, int((I[:, I_KB1] - I[:, I_KB0]).sum())
     if konly and kernel == 4 and reads * Hkv >= IMAGE_READS:
         tile_block, recs = image_arrays(T, I)
-        if len(recs) * IMAGE <= IMAGE_BYTES and reads >= IMAGE_REUSE * len(recs):
+        n, ncu = len(recs), num_sms(device)
+        if (n * IMAGE <= IMAGE_BYTES and reads >= IMAGE_REUSE * n
+                and image_rounds(len(I), Hkv, heads_per_pass(len(I), n, Hkv, ncu), ncu) <= image_rounds(len(I), Hkv, Hkv, ncu)):
             parts += [tile_block, recs.ravel()]
-            nblocks = len(recs)
+            nblocks = n
     packed = torch.from_numpy(np.concatenate(parts))
     return Plan(ntiles=len(T), nitems=len(I), m=len(out_row), buf=packed.to(device), reqs=reqs, kernel=kernel, rows=rows,
                 D=D, kmin=int(sink), nblocks=nblocks)

@@ -255,3 +255,21 @@ def test_plans_of_static_pages_carry_no_block_records(monkeypatch):
     assert heavy.nblocks == 4 * 72 and static.nblocks == 0
     assert static.buf.numel() == heavy.buf.numel() - heavy.ntiles - 4 * heavy.nblocks
     assert (heavy.buf[:static.buf.numel()] == static.buf).all()
+
+
+def test_images_do_not_cost_rounds(monkeypatch):
+    """where the images have room for some of the heads only, the passes over them must not need more rounds of workgroups than
+    the one launch that needs no images"""
+    from flagrot_releaser_amd import prefill_mq as MQ
+    monkeypatch.setattr(MQ, "num_sms", lambda device: 256)
+
+    def plan(requests, tokens, prefix, G, Hkv):
+        reqs = [(r, tokens * r, tokens * (r + 1), prefix + tokens, prefix) for r in range(requests)]
+        return MQ.build_plan(reqs, G, Hkv, 0, "cpu")
+
+    many = plan(4, 512, 16384, 8, 8)                                    # 64 items: two rounds of 4 heads, as one launch of 8 has
+    assert many.nblocks == 4 * 264 and MQ.image_heads(many, 8, 256) == 4
+    few = plan(4, 512, 12000, 4, 8)                                     # 32 items: all heads in one round, but room for seven
+    assert few.nitems == 32 and few.nblocks == 0
+    assert plan(4, 512, 8000, 4, 8).nblocks == 4 * 133                  # ... for all of them
+    assert plan(4, 512, 12000, 4, 4).nblocks == 4 * 196                 # a rank of four heads
