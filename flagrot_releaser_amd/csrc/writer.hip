@@ -11,6 +11,7 @@
 // 64 KB C_q^T in LDS for the whole workgroup and walks its tokens eight rows at a time; the error vectors of the
 // candidates live in a small per-half-wave LDS strip so that the fixed-order matvec reads them as broadcasts.
 #include <cstdlib>
+#include <type_traits>
 
 #include "fr_launch.hpp"
 #include "ring_rows.hpp"
@@ -32,7 +33,9 @@ DEVI void wave_lds_sync() {  // LDS hand-over between lanes of one wavefront
 // anything else in which two neighbours share words; scattered slots (a decode step) field by field.  A decode step is bound
 // by its launch (3 us).  One unaligned chunk of 1024 / 8192 tokens x 8 + 8 rows, 4-bit pages: 31 / 202 -> 7.7 / 36 us
 // (before: a merge per field), 2-bit pages 109 / 725 -> 6.6 / 30 us.
-template <int QM, int P>
+// RING: workgroups behind the tokens' copy their BF16 rows (a kernel of its own: 4133 tokens on 4-bit pages 14.7 -> 14.6 us
+// without the test).
+template <int QM, int P, bool RING>
 __global__ void __launch_bounds__(256) k_static_write(const StaticWriteParams p) {
   using L = Lay<QM, P>;
   __shared__ long long vslot[8];
@@ -40,10 +43,12 @@ __global__ void __launch_bounds__(256) k_static_write(const StaticWriteParams p)
   __shared__ VRuns<8> runs;
   const int l32 = threadIdx.x & 31, hw = threadIdx.x >> 5;
   const int H2 = 2 * p.Hkv;
-  const int tiles = (p.T + 7) / 8 * H2;
-  if (static_cast<int>(blockIdx.x) >= tiles) {  // behind the tokens: their BF16 rows
-    ring_quad(p.ring, static_cast<long long>(blockIdx.x - tiles) * 256 + threadIdx.x);
-    return;
+  if constexpr (RING) {
+    const int tiles = (p.T + 7) / 8 * H2;
+    if (static_cast<int>(blockIdx.x) >= tiles) {
+      ring_quad(p.ring, static_cast<long long>(blockIdx.x - tiles) * 256 + threadIdx.x);
+      return;
+    }
   }
   const int hr = static_cast<int>(blockIdx.x % H2);
   const int t = static_cast<int>(blockIdx.x / H2) * 8 + hw;
@@ -330,8 +335,13 @@ template <int QM>
 int static_write_qm(const StaticWriteParams& p, hipStream_t st) {
   if (p.T <= 0) return 0;
   const unsigned grid = static_cast<unsigned>(static_cast<long long>((p.T + 7) / 8) * 2 * p.Hkv + (ring_quads(p.ring) + 255) / 256);
-  if (p.page == 16) hipLaunchKernelGGL((k_static_write<QM, 16>), dim3(grid), dim3(256), 0, st, p);
-  else if (p.page == 32) hipLaunchKernelGGL((k_static_write<QM, 32>), dim3(grid), dim3(256), 0, st, p);
+  const auto go = [&](auto page) {
+    constexpr int P = decltype(page)::value;
+    if (p.ring.rows > 0) hipLaunchKernelGGL((k_static_write<QM, P, true>), dim3(grid), dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((k_static_write<QM, P, false>), dim3(grid), dim3(256), 0, st, p);
+  };
+  if (p.page == 16) go(std::integral_constant<int, 16>{});
+  else if (p.page == 32) go(std::integral_constant<int, 32>{});
   else return -5;
   return hipPeekAtLastError() == hipSuccess ? 0 : -1;
 }

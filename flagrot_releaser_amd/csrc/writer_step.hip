@@ -10,13 +10,17 @@
 namespace fr {
 namespace {
 
-template <int QM, int P, int D>
+// RING: workgroups behind the tokens' copy their BF16 rows.  A kernel of its own: the test alone is 1 to 2 % of a call without
+// rows (graph of calls, 100 tokens x 8 heads on 4-bit pages 9.62 -> 9.44 us, 100 x 4 heads of 256 12.35 -> 12.12).
+template <int QM, int P, int D, bool RING>
 __global__ void __launch_bounds__(2 * D) k_k2_step(const K2WriteParams p) {
   __shared__ StepSmem<D> S;
   const int h = blockIdx.x, t = blockIdx.y;
-  if (t >= p.T) {                                  // behind the tokens: their BF16 rows
-    ring_quad(p.ring, (static_cast<long long>(t - p.T) * p.Hkv + h) * (2 * D) + threadIdx.x);
-    return;
+  if constexpr (RING) {
+    if (t >= p.T) {
+      ring_quad(p.ring, (static_cast<long long>(t - p.T) * p.Hkv + h) * (2 * D) + threadIdx.x);
+      return;
+    }
   }
   const long long slot = p.slots[static_cast<long long>(t) * (p.slot_ph ? p.Hkv : 1) + (p.slot_ph ? h : 0)];
   if (slot < 0) return;                            // the whole workgroup
@@ -26,10 +30,11 @@ __global__ void __launch_bounds__(2 * D) k_k2_step(const K2WriteParams p) {
 
 template <int QM, int P>
 void step(const K2WriteParams& p, hipStream_t st) {
-  const long long per_row = static_cast<long long>(p.Hkv) * (p.hd == 256 ? 512 : 256);      // quads of a row of workgroups
+  const long long per_row = static_cast<long long>(p.Hkv) * 256;                            // quads of a row of workgroups
   const dim3 grid(p.Hkv, p.T + static_cast<unsigned>((ring_quads(p.ring) + per_row - 1) / per_row));
-  if (p.hd == 256) hipLaunchKernelGGL((k_k2_step<QM, P, 256>), grid, dim3(512), 0, st, p);
-  else hipLaunchKernelGGL((k_k2_step<QM, P, 128>), grid, dim3(256), 0, st, p);
+  if (p.hd == 256) hipLaunchKernelGGL((k_k2_step<QM, P, 256, false>), grid, dim3(512), 0, st, p);
+  else if (p.ring.rows > 0) hipLaunchKernelGGL((k_k2_step<QM, P, 128, true>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((k_k2_step<QM, P, 128, false>), grid, dim3(256), 0, st, p);
 }
 template <int QM>
 int step_qm(const K2WriteParams& p, hipStream_t st) {
