@@ -27,16 +27,20 @@ int fr_abi_version(void);
  * [rows, W, 2*Hkv, 128] (strides tail_bs / tail_ts elements) + tail_len int32 [B] (+ tail_idx int32 [B]) or null.
  * With a tail at head dim 128, q and tail must be 16-byte aligned and q_bs, tail_bs, tail_ts multiples of 8 elements
  * (the rows are operands of matrix instructions, read 16 bytes at a time; contiguous torch tensors always are): -3 if not.
- * nsplit counts the body splits; with a tail the workspace must hold B*Hkv*ceil(gqa/GT)*(nsplit+1) partials of
- * GT*128 floats (GT = 8 when variant has bits 1024|2048, else 4), opart and mlpart 8-byte aligned (-3 if not; at head dim 256
- * opart 16-byte); counter int32 [B*Hkv*ceil(gqa/GT)] zeroed once by the
- * caller (merge tickets and, when the body workgroups of a sequence share its page range, their page draws; the last
- * arriving workgroup leaves the word at 0).  If B*Hkv*ceil(gqa/GT)*nsplit fits the CUs and chunk >= 1024, split s owns
- * tokens [s, s+1)*chunk and one large workgroup per CU runs it; otherwise nsplit only counts the workgroups per
- * (sequence, KV head, q tile); nsplit*chunk must cover the longest sequence either way.
+ * nsplit counts the body splits; with a tail the workspace must hold B*Hkv*ceil(gqa/GT)*(nsplit+1) partials of GT*128
+ * floats (GT = 8 when variant has bits 1024|2048, else 4), opart and mlpart 8-byte aligned (-3 if not; at head dim 256
+ * opart 16-byte); counter int32 [B*Hkv*ceil(gqa/GT)] zeroed once by the caller (merge tickets and, when the body
+ * workgroups of a sequence share its page range, their page draws; the last arriving workgroup leaves the word at 0).  If
+ * B*Hkv*ceil(gqa/GT)*nsplit fits the CUs and chunk >= 1024, split s owns tokens [s, s+1)*chunk and one large workgroup
+ * per CU runs it; otherwise nsplit only counts the workgroups per (sequence, KV head, q tile); nsplit*chunk must cover
+ * the longest sequence either way.
  * variant bit 4096 (kernels/csrc/attn_decode_v2g.cuh:11-25, 276): head dim 256 -- q, out and tail rows have 256 channels,
  * the pool chunk is two 128-d half chunks per (page, KV head), kmask / vmask are [Hkv, 8], partials are GT*256 floats
- * with GT = 4, split s owns tokens [s, s+1)*chunk and the counter words are not used. */
+ * with GT = 4 and the counter words are not used.  Split s owns tokens [s, s+1)*chunk, except in batches of 2 .. 64
+ * sequences with nsplit >= 2, chunk >= 512 and a multiple of 64, nsplit*chunk <= 2^24 and B*Hkv*ceil(gqa/4)*nsplit >= 1.5
+ * workgroups a CU: there the B*nsplit parts of a (KV head, q tile) are shared out by seq_lens on the device (same
+ * workspace, partials [KV head, q tile][B*nsplit parts, B window-row parts]), seq_lens must not change before the call
+ * has ended, and where a sequence is cut -- so the last bit of its output -- depends on the other lengths of the batch. */
 int fr_v2_attn(int fmt, const void* q, long long q_bs, const uint8_t* pool, const int* block_table, int bt_stride,
                const int* seq_lens, int B, int Hkv, int page, int nsplit, int chunk, float qscale,
                const uint8_t* kmask, const uint8_t* vmask, int rb, int qrot, int vrot, int variant, int stages,
