@@ -348,7 +348,8 @@ def test_head_dim_256_groups(dev, fmt, G, Hkv):
     _head_dim_256(dev, fmt, 16, G, Hkv)
 
 
-def _head_dim_256(dev, fmt, P, G, Hkv, lens=None, seed=None):
+def _head_dim_256(dev, fmt, P, G, Hkv, lens=None, seed=None, kv_start=3, partials=None):
+    """partials(nsplit, chunk, written): which partial slots of a call were written, by its (maximum, sum) pairs"""
     from flagrot_releaser_amd import kernels as K
     Dh = 256
     static = fmt in ("int4", "int4a", "int2a")
@@ -378,7 +379,7 @@ def _head_dim_256(dev, fmt, P, G, Hkv, lens=None, seed=None):
             K.cb_write(kv, sl, CT, co, fmt, pool, P)
     q = (torch.randn(B, HQ, Dh, generator=g) * 0.8).bfloat16()
     scale = 1 / math.sqrt(Dh)
-    W, R, kv_start = 20, B + 1, 3
+    W, R = 20, B + 1
     tail = torch.randn(R, W, 2 * Hkv, Dh, generator=g).bfloat16()
     tail_idx = torch.randperm(R, generator=g)[:B].int()
     tail_len = torch.randint(0, W + 1, (B,), generator=g).int()
@@ -395,6 +396,7 @@ def _head_dim_256(dev, fmt, P, G, Hkv, lens=None, seed=None):
         HV, GT = K.vheads(Hkv, G, Dh, fmt), K.tile_of(K.v2_variant(fmt, G, Dh))
         assert (HV, GT) == (Hkv * ((G + 3) // 4), 4)
         ws = K.Workspace(B, HV, B * HV * (ns + 1), dev, GT, Dh)
+        ws.mlpart.fill_(float("nan"))
         out = torch.full((B, HQ * Dh), float("nan"), dtype=torch.bfloat16, device=dev)
         if static:
             K.v2_attn(q.to(dev), pool, bt.to(dev), seq.to(dev), out, ns, ch, ws, scale * LOG2E, kmask=mask[:Hkv].to(dev),
@@ -410,6 +412,8 @@ def _head_dim_256(dev, fmt, P, G, Hkv, lens=None, seed=None):
         assert strict.max() <= 1.0, (fmt, P, ns, np.unravel_index(np.argmax(strict), strict.shape))
         assert not got[-1].any()
         assert int(ws.counter.abs().sum()) == 0
+        if partials is not None:
+            partials(ns, ch, ~ws.mlpart.view(-1, 8)[:, 0].isnan().cpu())
 
 
 @pytest.mark.parametrize("fmt,P", [("konlya", 16), ("int2a", 32)])
