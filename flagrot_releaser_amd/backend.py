@@ -306,6 +306,11 @@ class StepPlanner:
         sp.group_src, sp.group_dst = self._group[0, :n], self._group[1, :n]
 
 
+def as_defined(layer, cls, *methods) -> bool:
+    """none of these methods of cls is overridden, in a subclass or on the object"""
+    return all(getattr(getattr(layer, m), "__func__", None) is getattr(cls, m) for m in methods)
+
+
 class DecodeLayer:
     """cache state and call sequence of one attention layer over FlagRot pages: pages + BF16 ring, writer then decode."""
 
@@ -362,11 +367,7 @@ class DecodeLayer:
             K.ring_rows(kv, self.ring, kmu=self.kmu, base=base, sink=self.geo.S, window=self.geo.W, start=start)
 
     def update(self, kv, sp: StepPlan):
-        """cache update of a decode step: the new tokens to their pages and to their BF16 slots, in one launch"""
-        if self.ring is not None and sp.slots.shape[0] == kv.shape[0]:
-            K.step_write(kv, sp.slots, self.kind, self.pool, PAGE, self.ring, sp.ring_dest, mask=self.wmask, CT=self.CT,
-                         kmu=self.kmu)
-            return
+        """cache update of a decode step: the new tokens to their pages and to their BF16 slots"""
         self.write_pages(kv, sp.slots)
         if self.ring is not None:
             K.ring_rows(kv, self.ring, kmu=self.kmu, dest=sp.ring_dest)
@@ -387,8 +388,12 @@ class DecodeLayer:
                       self.kind, **extra)
 
     def step(self, q, kv, sp: StepPlan, out):
-        """what a captured decode step of this layer contains"""
-        self.update(kv, sp)
+        """what a captured decode step of this layer contains: update, its two launches as one, and decode"""
+        if self.ring is not None and kv.shape[0] == sp.slots.shape[0] and as_defined(self, DecodeLayer, "update", "write_pages"):
+            K.step_write(kv, sp.slots, self.kind, self.pool, PAGE, self.ring, sp.ring_dest, mask=self.wmask, CT=self.CT,
+                         kmu=self.kmu)
+        else:
+            self.update(kv, sp)
         self.decode(q, sp, out)
 
 
@@ -440,12 +445,12 @@ class KiviDecodeLayer:
         K.ring_rows(kv, self.ring, base=base, sink=self.geo.S, window=self.geo.W, start=start)
 
     def update(self, kv, sp: StepPlan):
-        """cache update of a decode step: values and BF16 rows of the new tokens, in one launch, and the key groups they complete"""
-        if kv.shape[0] == sp.slots.shape[0] and kv.stride(0) % 4 == 0 and kv.data_ptr() % 8 == 0:
-            KIVI.step_write(kv, sp.slots, self.co, self.pool, self.ring, sp.ring_dest, f8=self.f8)
-        else:                                              # (the one launch reads both halves of a row eight bytes at a time)
-            KIVI.v_write(kv, sp.slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
-            K.ring_rows(kv, self.ring, dest=sp.ring_dest)
+        """cache update of a decode step: values and BF16 rows of the new tokens, then the key groups that they complete"""
+        KIVI.v_write(kv, sp.slots, self.co, None, self.pool, self.Hkv, D, f8=self.f8)
+        K.ring_rows(kv, self.ring, dest=sp.ring_dest)
+        self._encode_completed(sp)
+
+    def _encode_completed(self, sp: StepPlan):
         KIVI.k_encode(self.ring, sp.group_src, sp.group_dst, self.qs, self.lz, self.scale, self.pool, self.Hkv, D,
                       f8=self.f8)
 
@@ -458,5 +463,11 @@ class KiviDecodeLayer:
                   tail_idx=sp.ring_home, T=self.geo.slots, f8=self.f8)
 
     def step(self, q, kv, sp: StepPlan, out):
-        self.update(kv, sp)
+        """update, its first two launches as one where that can read the rows (eight bytes at a time), and decode"""
+        if (kv.shape[0] == sp.slots.shape[0] and kv.stride(0) % 4 == 0 and kv.data_ptr() % 8 == 0
+                and as_defined(self, KiviDecodeLayer, "update")):
+            KIVI.step_write(kv, sp.slots, self.co, self.pool, self.ring, sp.ring_dest, f8=self.f8)
+            self._encode_completed(sp)
+        else:
+            self.update(kv, sp)
         self.decode(q, sp, out)

@@ -115,9 +115,9 @@ def test_shared_workspace_grows_for_more_splits():
     assert pool.flagrot("cpu", (2, 4, 128), 8, lambda rows: (2, 512)) is second
 
 
-def test_a_step_stores_what_update_stores(monkeypatch):
-    """step() is update() and decode(): a subclass that overrides one of them is asked, and both list the same launches; what
-    the one launch cannot read goes through the writer and the row copy"""
+def test_a_step_asks_an_update_of_a_subclass(monkeypatch):
+    """step() is update() and decode(), with what update() stores first in one launch where the layer's own methods store it: a
+    method that a subclass or the object overrides is asked, and what the one launch cannot read goes through update()"""
     calls = []
     note = lambda name: lambda *a, **kw: calls.append(name)                                          # noqa: E731
     for mod, names in ((BK.K, ("step_write", "ring_rows", "v2_write", "cb_write", "v2_attn", "cb_attn")),
@@ -147,21 +147,28 @@ def test_a_step_stores_what_update_stores(monkeypatch):
                 cls, make = BK.DecodeLayer, lambda c: c(kind, H, G, pool, planner, **extra)          # noqa: E731
             layer = make(cls)
             layer.update(kv, sp)
-            stored = calls.copy()
+            apart = calls.copy()
+            assert not any(c.endswith("step_write") for c in apart)
             calls.clear()
             layer.step(q, kv, sp, None)
-            assert calls[:-1] == stored and calls[-1].endswith("attn")
-            assert any(c.endswith("step_write") for c in stored) == bool(window)
+            rest = [c for c in apart if c.endswith("k_encode")]
+            one = [("kivi" if kind == "kivi2" else "kernels") + ".step_write"] + rest
+            assert calls[:-1] == (one if window else apart) and calls[-1].endswith("attn")
             calls.clear()
-            more = BK.StepPlan(**{**vars(sp), "slots": torch.arange(n + 2)})                         # more slots than rows
-            layer.step(q, kv, more, None)
-            assert not any(c.endswith("step_write") for c in calls)
+            layer.step(q, kv, BK.StepPlan(**{**vars(sp), "slots": torch.arange(n + 2)}), None)       # more slots than rows
+            assert calls[:-1] == apart
             calls.clear()
             if kind == "kivi2":
                 layer.step(q, odd, sp, None)
-                assert calls[:2] == ["kivi.v_write", "kernels.ring_rows"]
+                assert calls[:-1] == apart
                 calls.clear()
-            sub = make(type("Sub", (cls,), {"update": note("mine")}))
-            sub.step(q, kv, sp, None)
-            assert calls[0] == "mine" and len(calls) == 2
-            calls.clear()
+            for name in ["update", "decode"] + ["write_pages"] * (kind != "kivi2"):
+                sub = make(type("Sub", (cls,), {name: note("mine")}))
+                sub.step(q, kv, sp, None)
+                assert "mine" in calls and any(c.endswith("step_write") for c in calls) == (name == "decode" and bool(window))
+                calls.clear()
+                alone = make(cls)
+                setattr(alone, name, note("mine"))
+                alone.step(q, kv, sp, None)
+                assert "mine" in calls
+                calls.clear()
