@@ -326,7 +326,10 @@ __global__ void __launch_bounds__(512, 1) k_mq8(const Params p) {
 // (maximum, sum) pairs are read one item per lane (64 at a time), so the common maximum, every item's weight
 // 2^(m - M) and the total sum come from three wave reductions instead of two serial passes; the accumulation takes each
 // weight from its lane and has 16 outputs (rows x items) in flight whatever the weights are -- a load behind a test of its
-// weight is a memory round trip per item and row (8 KV heads of 128 rows, 1 tile of 19 items: 38 us; now 7).  Tiles of up to
+// weight is a memory round trip per item and row (8 KV heads of 128 rows, 1 tile of 19 items: 38 us; now 7).  Eight outputs
+// where four rows of 256 channels share a wavefront, and what all lanes hold alike in scalar registers: 52 / 69 registers, as
+// the tiles of few items need, instead of 68 / 108 (wavefronts in flight are what those are bound by; 128 tiles x 256, 1
+// item 34.1 -> 32.7, 16 tiles of 5 18.1 -> 17.5; 64 tiles x 128, 1 item 25.6 -> 25.2).  Tiles of up to
 // FOLD_FEW items need no lanes for that: the pairs of the wavefront's rows are neighbours in memory and the same for all
 // lanes, so they come by scalar loads, and the outputs of all rows and items are in flight together.  Faster at every size
 // (8 KV heads, us by lanes / this way, graph: 14 tiles of 256 rows x 128, 2 items 13.2 / 8.7; 64 tiles, 1 item 37.6 / 25.0, 2
@@ -361,7 +364,7 @@ __global__ void __launch_bounds__(256) k_fold_items(const int* __restrict__ tile
                                                     const float* __restrict__ ml, int Hkv, int G, int rows,
                                                     void* __restrict__ out, long long out_stride, float* __restrict__ lse,
                                                     long long lse_stride) {
-  constexpr int FOLD_STEP = 16 / FOLD_ROWS;                              // items at a time: 16 outputs in flight
+  constexpr int FOLD_STEP = FOLD_ROWS == 1 ? 16 : W == 2 ? 4 : 2;         // items at a time
   const int lane = threadIdx.x & 63, head = blockIdx.y;
   const int* rec = tiles + TILE_INTS * blockIdx.x;
   const int first = rec[6], count = rec[7];
@@ -437,6 +440,7 @@ __global__ void __launch_bounds__(256) k_fold_items(const int* __restrict__ tile
 #pragma unroll
     for (int k = 0; k < W; ++k) sum[i][k] = 0.f;
   }
+  const auto uniform = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
   auto pair = [&](int s, int i) {                                        // item s of the row, nothing past the last item
     return s < count ? *reinterpret_cast<const float2*>(ml + 2 * (at + s * per_item + row[i])) : make_float2(-INFINITY, 0.f);
   };
@@ -444,14 +448,14 @@ __global__ void __launch_bounds__(256) k_fold_items(const int* __restrict__ tile
 #pragma unroll
     for (int i = 0; i < FOLD_ROWS; ++i) top[i] = fmaxf(top[i], pair(s0 + lane, i).x);
 #pragma unroll
-  for (int i = 0; i < FOLD_ROWS; ++i) top[i] = wave_max64(top[i]);
+  for (int i = 0; i < FOLD_ROWS; ++i) top[i] = uniform(wave_max64(top[i]));
   for (int s0 = 0; s0 < count; s0 += 64) {
     float weight[FOLD_ROWS];
 #pragma unroll
     for (int i = 0; i < FOLD_ROWS; ++i) {
       const float2 st = pair(s0 + lane, i);
       weight[i] = st.x == -INFINITY ? 0.f : fexp2(st.x - top[i]);
-      total[i] += wave_sum64(weight[i] * st.y);
+      total[i] = uniform(total[i] + wave_sum64(weight[i] * st.y));
     }
     const int n = min(64, count - s0);
     for (int g = 0; g < n; g += FOLD_STEP) {
