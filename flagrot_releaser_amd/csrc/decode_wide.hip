@@ -255,8 +255,12 @@ __global__ void __launch_bounds__(256) k_wide_parts(const DecodeParams p, int nt
   if (lane == 0) { mlp[2 * wave] = m_run; mlp[2 * wave + 1] = l_run; }
 }
 
-// Split merge: a workgroup per (sequence, q head), thread = channel, the reads of eight splits in flight together: bound by
-// its launch (16 sequences x 24 heads, 4 splits: 8.7 -> 4.0 us; a workgroup per q tile walked heads and splits in turn).
+// Split merge: a workgroup per (sequence, q head), thread = channel, the reads of eight splits in flight together (the first
+// eight outputs before the maxima are known: SHARE waits for the lengths instead, so a merge is as many trips to memory
+// with shared parts as without): bound by its launch (16 sequences x 24 heads, 4 splits: 8.7 -> 4.0 us; a workgroup per q tile
+// walked heads and splits in turn).
+constexpr int AHEAD = 8;
+template <bool SHARE>
 __global__ void __launch_bounds__(256) k_wide_merge(const DecodeParams p, int ntile, int nparts, int rotate_back) {
   __shared__ float buf[WD];
   const int kvh = blockIdx.x / ntile, tile = blockIdx.x % ntile, b = blockIdx.y, h = blockIdx.z, hq = tile * 4 + h, d = threadIdx.x;
@@ -264,28 +268,50 @@ __global__ void __launch_bounds__(256) k_wide_merge(const DecodeParams p, int nt
   // partials [first, first + n) of `part0` and, with BF16 rows, one more
   long long part0 = ((static_cast<long long>(b) * p.Hkv + kvh) * ntile + tile) * nparts;
   int n = nparts, rows_at = -1;
-  if (p.share) {
-    const Shares sh = share_parts(p, threadIdx.x & 63);
+  if constexpr (SHARE) {
+    __shared__ int2 mine;                             // (one wavefront of four: the others' issue slots are the next workgroup's)
+    if (threadIdx.x < 64) {
+      const Shares sh = share_parts(p, threadIdx.x);
+      if (static_cast<int>(threadIdx.x) == b) mine = make_int2(sh.first, sh.n);
+    }
+    __syncthreads();
     const long long all = static_cast<long long>(kvh * ntile + tile) * p.B * nparts;
-    part0 = all + __builtin_amdgcn_readlane(sh.first, b);
-    n = __builtin_amdgcn_readlane(sh.n, b);
+    part0 = all + __builtin_amdgcn_readfirstlane(mine.x);
+    n = __builtin_amdgcn_readfirstlane(mine.y);
     if (p.tail != nullptr) { rows_at = static_cast<int>(all + p.B * p.nsplit + b - part0); ++n; }
   }
   const float* ml = p.mlpart + part0 * 8 + 2 * h;
   const float* o = p.opart + part0 * 4 * WD + h * WD + d;
-  float M = -INFINITY;
+  const auto place = [&](int i) { return SHARE && rows_at >= 0 && i == n - 1 ? rows_at : i; };
+  float M = -INFINITY, acc = 0.f, Lsum = 0.f;
+  const auto add = [&](float ms, float ls, float os) {
+    const bool some = ms != -INFINITY;                          // (an empty split stores no outputs)
+    const float f = fexp2w(ms - M);
+    Lsum += some ? f * ls : 0.f;
+    acc += some ? f * os : 0.f;
+  };
+  if (n > 0) {
+    float ms[AHEAD], ls[AHEAD], os[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      ms[i] = -INFINITY; ls[i] = os[i] = 0.f;
+      if (i < n) {
+        const int s = place(i);
+        os[i] = o[static_cast<long long>(s) * 4 * WD];
+        ms[i] = ml[8 * s];
+        ls[i] = ml[8 * s + 1];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) M = fmaxf(M, ms[i]);
 #pragma unroll 8
-  for (int i = 0; i < n; ++i) M = fmaxf(M, ml[8 * (rows_at >= 0 && i == n - 1 ? rows_at : i)]);
-  float acc = 0.f, Lsum = 0.f;
-  if (M != -INFINITY) {
+    for (int i = AHEAD; i < n; ++i) M = fmaxf(M, ml[8 * place(i)]);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) add(ms[i], ls[i], os[i]);
 #pragma unroll 8
-    for (int i = 0; i < n; ++i) {
-      const int s = rows_at >= 0 && i == n - 1 ? rows_at : i;
-      const float ms = ml[8 * s], ls = ml[8 * s + 1], os = o[static_cast<long long>(s) * 4 * WD];
-      const bool some = ms != -INFINITY;                        // (an empty split stores no outputs)
-      const float f = fexp2w(ms - M);
-      Lsum += some ? f * ls : 0.f;
-      acc += some ? f * os : 0.f;
+    for (int i = AHEAD; i < n; ++i) {
+      const int s = place(i);
+      add(ml[8 * s], ml[8 * s + 1], o[static_cast<long long>(s) * 4 * WD]);
     }
   }
   float v = Lsum > 0.f ? acc / Lsum : 0.f;
@@ -319,7 +345,7 @@ int wide_qm(const DecodeParams& p, hipStream_t st) {
     const int rc = decode_wide_mma_launch(FMT, p, ntile, nparts, st);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_wide_merge, dim3(p.Hkv * ntile, p.B, 4), dim3(256), 0, st, p, ntile, nparts, (!K2 && p.vmask != nullptr) ? 1 : 0);
+  hipLaunchKernelGGL(p.share ? k_wide_merge<true> : k_wide_merge<false>, dim3(p.Hkv * ntile, p.B, 4), dim3(256), 0, st, p, ntile, nparts, (!K2 && p.vmask != nullptr) ? 1 : 0);
   return hipPeekAtLastError() == hipSuccess ? 0 : -1;
 }
 
