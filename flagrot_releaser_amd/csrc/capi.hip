@@ -187,12 +187,19 @@ int fr_v2_attn(int fmt, const void* q, long long q_bs, const uint8_t* pool, cons
   // tokens 15.5 / 16.0; 480 of 1664 tokens 68 / 72).
   if (variant & HD256) p.wg_waves = pairs * nparts <= cus && chunk >= 512 ? 8 : 4;
   // ... and where the plan has one and a half workgroups a CU at least, its parts are shared out by the sequences' lengths
-  // (decode_share.hpp).  Decode and merge of uneven lengths down to a quarter, us, fixed ranges / shared out: 512 workgroups
-  // 58.5 / 49.3, 480 41.5 / 38.8, 392 33.7 / 31.3; below, the parts that come on top would sit beside others on their CU and
-  // the merge is 1.4 longer: 352 35.9 / 36.9, 176 20.3 / 20.9.  Even lengths: 512 59.8 / 60.6, 480 44.0 / 44.8.
+  // (decode_share.hpp).  Decode and merge of uneven lengths down to a quarter, us, fixed ranges / shared out: 512 workgroups of
+  // 2048 tokens 54.0 / 44.1, 480 of 1536 43.2 / 37.7, 384 of 1536 43.9 / 37.4; of 1024 tokens 33.6 / 33.7 (down to a 32nd: 31.2 /
+  // 24.5); below, the parts that come on top would sit beside others on their CU: 352 35.9 / 36.9, 176 20.3 / 20.9.  Even lengths:
+  // 512 56.7 / 55.8, 448 42.8 / 43.8, 64 sequences of 2048 tokens 36.3 / 36.8.
+  // With BF16 rows the parts have the places that the rows' workgroups leave of two a CU: more of either would begin when the
+  // first ones end (lengths down to a quarter, rows of 72 tokens, fixed ranges / as many parts as without rows / this: 16
+  // sequences of 8192 56.2 / 65.5 / 52.2, 8 of 8192 34.3 / 44.7 / 35.0, 32 of 4096 42.0 / 50.3 / 42.0, 60 of 4000 44.0 / 47.9 / 39.9).
   const char* const plain = getenv("FLAGROT_WIDE_PLAIN");      // (the plain kernel has fixed ranges; read at every call)
-  p.share = (variant & HD256) && !force_static && !(plain != nullptr && plain[0] == '1') && B >= 2 && B <= 64 && nsplit >= 2 &&
-            chunk >= 512 && chunk % 64 == 0 && static_cast<long long>(nsplit) * chunk <= (1ll << 24) && 2 * pairs * nsplit >= 3 * cus;
+  if ((variant & HD256) && !force_static && !(plain != nullptr && plain[0] == '1') && B >= 2 && B <= 64 && nsplit >= 2 &&
+      chunk >= 512 && chunk % 64 == 0 && static_cast<long long>(nsplit) * chunk <= (1ll << 24) && 2 * pairs * nsplit >= 3 * cus) {
+    const long long places = 2 * cus / (pairs / B) - B;
+    p.share = static_cast<int>(tail == nullptr || places > B * nsplit ? B * nsplit : places < 1 ? 1 : places);
+  }
   if (variant & HD256) return launched(decode_wide_launch(fmt, p, static_cast<hipStream_t>(stream)), "fr_v2_attn (head dim 256)");
   return launched(decode_launch(fmt, p, static_cast<hipStream_t>(stream)), "fr_v2_attn");
 }

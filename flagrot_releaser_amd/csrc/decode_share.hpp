@@ -1,6 +1,7 @@
 // Split ranges of a batch of uneven sequences (head dim 256 decode): the B * nsplit workgroups of a (KV head, q tile) that the
 // plan made for the longest sequence are shared out by the lengths, on the device, since only it knows them.  Every part takes
-// at most m units of 64 tokens, m the smallest number (to 1 / 15 of its range) for which the parts of all sequences fit:
+// at most m units of 64 tokens, m the smallest number (to 1 / 15 of its range) for which the parts of all sequences fit their
+// places (p.share), or the plan's own:
 // 16 sequences of 2048 ... 8192 tokens planned as 4 x 2048 get parts of at most 1472 instead, on 64 workgroups instead of 46.
 // Even lengths give the plan's own ranges.  (Kernel of those 16 sequences, 4 KV heads of 256 in 4-bit pages, 6 query heads
 // each: 53.8 -> 43.6 us; bound by two wavefronts per SIMD either way.)
@@ -40,10 +41,11 @@ DEVI Shares share_parts(const DecodeParams& p, int lane) {
   Shares s;
   s.u = lane < p.B ? max(0, (share_end(p, lane) - share_start(p) + 63) >> 6) : 0;
   const int all = __builtin_amdgcn_readlane(scan_lanes(s.u), 63);
-  // parts of m units: at least all / m of them and fewer than all / m + B, so m lies in [all / S, all / (S - B) + 1]
-  const int S = p.B * p.nsplit;
-  const int lo = max(1, (all + S - 1) / S), hi = max(lo, min(p.chunk >> 6, all / (S - p.B) + 1)), step = max(1, (hi - lo + 14) / 15);
-  int m = min(hi, lo + step * (lane & 15));                        // candidate lane mod 16; the last one always fits
+  // parts of m units: at least all / m of them and fewer than all / m + B, so m lies in [all / S, all / (S - B) + 1], and m of the
+  // plan's own size need no more than its places
+  const int S = p.share, cap = p.chunk >> 6;
+  const int hi = S > p.B ? min(cap, all / (S - p.B) + 1) : cap, lo = min(hi, max(1, (all + S - 1) / S)), step = max(1, (hi - lo + 14) / 15);
+  int m = min(hi, lo + step * (lane & 15));                        // candidate lane mod 16; the last one if none fits
   if (hi > lo) {
     const float r = __builtin_amdgcn_rcpf(static_cast<float>(m));
     int count = 0;

@@ -83,7 +83,8 @@ struct DecodeParams {
   int kv_start;
   int dyn;                 // 1: the nsplit body workgroups of a (sequence, KV head, q tile) share its whole page range and
                            //    draw quads of 4 pages from the slot's counter; 0: split s owns tokens [s, s + 1) * chunk
-  int share;               // 1 (head dim 256): the B * nsplit parts of a (KV head, q tile) are shared out by length (decode_share.hpp)
+  int share;               // > 0 (head dim 256): the B * nsplit parts of a (KV head, q tile) are shared out by length, into this
+                           //    many where the plan's chunk allows that (decode_share.hpp)
   int wg_waves;            // wavefronts per workgroup: 4, or the large workgroup that fills a CU
   int fuse_tail;           // 1: no workgroup of their own for the BF16 rows -- the wavefronts of the first body split take
                            //    them after their pages and fold them into their own partials (k_decode, k_decode8; key-only formats)

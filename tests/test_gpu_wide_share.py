@@ -22,16 +22,18 @@ CASES = {"uneven": (UNEVEN, True), "even": ([1530] * 15, True), "the longest alo
          "few workgroups": ([1537, 300, 700], False)}
 
 
-def parts_by_length(lens, nsplit, chunk, kv_start):
-    """how many parts a (KV head, q tile) has in all: the smallest of 16 candidate lengths whose parts fit"""
+def parts_by_length(lens, nsplit, chunk, kv_start, groups):
+    """how many parts a (KV head, q tile) has in all: of 16 candidate lengths the smallest whose parts fit beside the window rows'
+    workgroups, two a CU; the plan's chunk if none does"""
     start = kv_start & ~63
     units = [max(0, -(-(min(n, nsplit * chunk) - start) // 64)) for n in lens]
-    places, total = len(lens) * nsplit, sum(units)
-    lo = max(1, -(-total // places))
-    hi = max(lo, min(chunk // 64, total // (places - len(lens)) + 1))
+    B, cap, total = len(lens), chunk // 64, sum(units)
+    places = max(1, min(B * nsplit, 512 // groups - B))
+    hi = min(cap, total // (places - B) + 1) if places > B else cap
+    lo = min(hi, max(1, -(-total // places)))
     step = max(1, (hi - lo + 14) // 15)
     count = lambda m: sum(-(-u // m) for u in units)                                                # noqa: E731
-    return next(count(m) for m in (min(hi, lo + step * k) for k in range(16)) if count(m) <= places)
+    return next((count(m) for m in (min(hi, lo + step * k) for k in range(16)) if count(m) <= places), count(hi))
 
 
 def check(dev, fmt, P, G, Hkv, lens, shared, kv_start=3):
@@ -43,7 +45,7 @@ def check(dev, fmt, P, G, Hkv, lens, shared, kv_start=3):
         if nsplit == 1 or not shared:
             assert written.all()
             return
-        n = parts_by_length(lens + [0], nsplit, chunk, kv_start)
+        n = parts_by_length(lens + [0], nsplit, chunk, kv_start, groups)
         want = torch.zeros(B * (nsplit + 1), dtype=torch.bool)
         want[:n] = want[B * nsplit:] = True
         assert n < B * nsplit and (written.view(groups, -1) == want).all()
