@@ -425,6 +425,12 @@ int fr_cb_write_smem(int kind, int tg, int hd) {
   if (fmt_of_kind(kind) < 0 || (hd != 0 && hd != 128 && hd != 256)) return 0;
   return k2_write_lds_bytes(hd);
 }
+int fr_cb_write_tokens(int T, int Hkv, int hd) {
+  if (T <= 0 || Hkv < 1 || (hd != 0 && hd != 128 && hd != 256)) return 0;
+  K2WriteParams p{};
+  p.T = T; p.Hkv = Hkv; p.hd = hd;
+  return k2_is_step(p) ? 1 : k2_screen_tokens(T, Hkv, hd);
+}
 
 const char* fr_last_error(void) { return g_err; }
 

@@ -52,6 +52,7 @@ int k2_step_launch(int kind, const K2WriteParams& p, hipStream_t st);      // on
 
 int k2_screen_launch(int kind, const K2WriteParams& p, bool all_exact, hipStream_t st);   // prompts; same bytes
 int k2_screen_lds_bytes(int hd);
+int k2_screen_tokens(long long T, int Hkv, int hd);      // of a workgroup
 
 int head_fwht_launch(const void* x, long long x_ts, void* out, long long o_ts, int T, int H, const uint8_t* flags,
                      float scale, hipStream_t st, int D);

@@ -310,23 +310,28 @@ __global__ void __launch_bounds__(2 * D, D == 128 ? 3 : 2) k_k2_screen(const K2W
   }
 }
 
-template <int QM, int P, int D>
-int screen(const K2WriteParams& p, float kappa, hipStream_t st) {
+// tokens of a workgroup
+template <int D>
+int tile_tokens(long long T, int Hkv) {
   // Steps per workgroup: all workgroups resident at once (3 per CU at head dim 128, 1 at 256) as far as the list of undecided
   // tokens allows; from five steps on, 128-d heads take workgroups of two, which the dispatcher spreads evenly (8 heads of
   // 128, us for 1 / 2 / 4 / 6 / 8 steps: 8192 tokens 94 / 91 / 101 / 97 / 106, 6000 tokens 70 / 68 / 66 / 79 / 100; 4 heads of
   // 256, 8192 tokens 187 / 166 / 139 / 188 / 131).
   constexpr long long RESIDENT = D == 128 ? 768 : 256;
-  const long long steps = (p.T + SCR_TOK - 1) / SCR_TOK, fit = (steps * p.Hkv + RESIDENT - 1) / RESIDENT;
+  const long long steps = (T + SCR_TOK - 1) / SCR_TOK, fit = (steps * Hkv + RESIDENT - 1) / RESIDENT;
   const long long per = D == 128 && fit > 4 ? 2 : fit < SCR_MAXTILE / SCR_TOK ? fit : SCR_MAXTILE / SCR_TOK;
-  // (A kernel of its own for the half steps: with the number of turns as a value both lose, 8192 tokens 95.1 -> 99.5 us.)
   // Short prompts, half a step a workgroup where that leaves every CU one at most: the candidates of one token instead of two
   // in a row (us, whole / half steps: 8 heads of 128, 130 tokens 18.2 / 15.6, 260 17.9 / 17.3, 520 19.9 / 21.0; 4 heads of 256,
   // 260 tokens 31.2 / 25.9, 400 31.7 / 25.5, 520 33.6 / 37.6).
-  const bool half = static_cast<long long>((p.T + SCR_TOK / 2 - 1) / (SCR_TOK / 2)) * p.Hkv <= 256;
-  const int tile = half ? SCR_TOK / 2 : SCR_TOK * static_cast<int>(per);
+  const bool half = (T + SCR_TOK / 2 - 1) / (SCR_TOK / 2) * Hkv <= 256;
+  return half ? SCR_TOK / 2 : SCR_TOK * static_cast<int>(per);
+}
+template <int QM, int P, int D>
+int screen(const K2WriteParams& p, float kappa, hipStream_t st) {
+  const int tile = tile_tokens<D>(p.T, p.Hkv);
   const dim3 grid(p.Hkv, (p.T + tile - 1) / tile);
-  if (half) hipLaunchKernelGGL((k_k2_screen<QM, P, D, 1>), grid, dim3(2 * D), 0, st, p, tile, kappa);
+  // (A kernel of its own for the half steps: with the number of turns as a value both lose, 8192 tokens 95.1 -> 99.5 us.)
+  if (tile < SCR_TOK) hipLaunchKernelGGL((k_k2_screen<QM, P, D, 1>), grid, dim3(2 * D), 0, st, p, tile, kappa);
   else hipLaunchKernelGGL((k_k2_screen<QM, P, D, 2>), grid, dim3(2 * D), 0, st, p, tile, kappa);
   return hipPeekAtLastError() == hipSuccess ? 0 : -1;
 }
@@ -349,6 +354,7 @@ int k2_screen_launch(int kind, const K2WriteParams& p, bool all_exact, hipStream
   }
   return -4;
 }
+int k2_screen_tokens(long long T, int Hkv, int hd) { return hd == 256 ? tile_tokens<256>(T, Hkv) : tile_tokens<128>(T, Hkv); }
 int k2_screen_lds_bytes(int hd) { return static_cast<int>(hd == 256 ? sizeof(ScreenSmem<256>) : sizeof(ScreenSmem<128>)); }
 
 }  // namespace fr

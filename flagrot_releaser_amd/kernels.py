@@ -50,6 +50,7 @@ NATIVE = Library("kernels", "FLAGROT_LIB", "fr_abi_version", ABI, "fr_last_error
     "fr_cb_occupancy": "i i i i",
     "fr_cb_chunk_bytes": "i i",
     "fr_cb_write_smem": "i i i",
+    "fr_cb_write_tokens": "i i i",
     "fr_last_error": "->s",
     "fr_head_fwht": "p l p l i i p f p i",
     "fr_cb_attn_noalloc": "p l p p i p i i i i i f i p l p p p l l p i i",

@@ -127,6 +127,9 @@ int fr_cb_attn_noalloc(const void* q, long long q_bs, const uint8_t* pool, const
 int fr_cb_occupancy(int kind, int variant, int stages, int page);
 int fr_cb_chunk_bytes(int kind, int page);
 int fr_cb_write_smem(int kind, int tg, int hd);
+/* No counterpart in the reference.  Tokens that a workgroup takes in a call of T tokens that runs the screened writer (8: half
+ * a step of its phases, else whole steps of 16), 1 where the call runs a workgroup per (token, head). */
+int fr_cb_write_tokens(int T, int Hkv, int hd);
 
 /* flagrot_capi.cu:155 */
 const char* fr_last_error(void);

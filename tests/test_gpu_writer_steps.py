@@ -10,15 +10,14 @@ import torch
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-# tokens x heads -> steps of a workgroup: 768 resident workgroups at head dim 128 (two steps from five on), 256 at 256 (at
-# most eight)
+# tokens x heads -> steps of a workgroup (what the library answers): 768 resident workgroups at head dim 128 (two steps from five
+# on), 256 at 256 (at most eight)
 SHAPES = [(128, 8, 2001, 2), (128, 8, 4000, 3), (128, 8, 5005, 4), (128, 8, 6203, 2), (256, 4, 2100, 3), (256, 4, 8201, 8)]
 
 
-def steps_of(D, Hkv, T):
-    resident = 768 if D == 128 else 256
-    fit = -(-(-(-T // 16)) * Hkv // resident)
-    return 2 if D == 128 and fit > 4 else min(fit, 8)
+def tokens_of(D, Hkv, T):
+    from flagrot_releaser_amd import kernels as K
+    return K.NATIVE.ask("fr_cb_write_tokens", T, Hkv, D)
 
 
 def check(kind, D, Hkv, T, page, first=5):
@@ -48,6 +47,7 @@ def check(kind, D, Hkv, T, page, first=5):
     pool = torch.randint(0, 256, (npg, Hkv, K.v2_chunk_bytes(page, D, kind)), dtype=torch.uint8, generator=g).to(dev)
     want, got = pool.clone(), pool.clone()
     small = 1024 // Hkv
+    assert tokens_of(D, Hkv, T) > 1 == tokens_of(D, Hkv, small)
     for a in range(0, T, small):
         K.cb_write(kv[a:a + small], slots[a:a + small].contiguous(), CT, co, kind, want, page)
     if D == 128:
@@ -61,7 +61,7 @@ def check(kind, D, Hkv, T, page, first=5):
 @pytest.mark.parametrize("page", [16, 32])
 @pytest.mark.parametrize("D,Hkv,T,steps", SHAPES)
 def test_steps_write_the_bytes_of_small_calls(dev, kind, D, Hkv, T, steps, page):
-    assert steps_of(D, Hkv, T) == steps
+    assert tokens_of(D, Hkv, T) == 16 * steps
     check(kind, D, Hkv, T, page)
 
 
@@ -71,7 +71,7 @@ def test_steps_write_the_bytes_of_small_calls(dev, kind, D, Hkv, T, steps, page)
                                           (256, 4, 257, True), (256, 2, 1024, True), (256, 2, 1025, False)])
 @pytest.mark.parametrize("kind,page", [("konly", 32), ("konlya2", 16)])
 def test_half_steps_write_the_bytes_of_small_calls(dev, kind, page, D, Hkv, T, half):
-    assert T * Hkv > 1024 and (-(-T // 8) * Hkv <= 256) == half
+    assert (tokens_of(D, Hkv, T) == 8) == half and tokens_of(D, Hkv, 1024 // Hkv) == 1
     check(kind, D, Hkv, T, page)
 
 
