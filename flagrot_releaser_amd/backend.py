@@ -306,9 +306,9 @@ class StepPlanner:
         sp.group_src, sp.group_dst = self._group[0, :n], self._group[1, :n]
 
 
-def as_defined(layer, cls, *methods) -> bool:
-    """none of these methods of cls is overridden, in a subclass or on the object"""
-    return all(getattr(getattr(layer, m), "__func__", None) is getattr(cls, m) for m in methods)
+def runs(method, function) -> bool:
+    """a bound method is this function: overridden neither in a subclass nor on the object"""
+    return getattr(method, "__func__", None) is function
 
 
 class DecodeLayer:
@@ -389,7 +389,8 @@ class DecodeLayer:
 
     def step(self, q, kv, sp: StepPlan, out):
         """what a captured decode step of this layer contains: update, its two launches as one, and decode"""
-        if self.ring is not None and kv.shape[0] == sp.slots.shape[0] and as_defined(self, DecodeLayer, "update", "write_pages"):
+        if (self.ring is not None and kv.shape[0] == sp.slots.shape[0] and runs(self.update, DecodeLayer.update)
+                and runs(self.write_pages, DecodeLayer.write_pages)):
             K.step_write(kv, sp.slots, self.kind, self.pool, PAGE, self.ring, sp.ring_dest, mask=self.wmask, CT=self.CT,
                          kmu=self.kmu)
         else:
@@ -465,7 +466,7 @@ class KiviDecodeLayer:
     def step(self, q, kv, sp: StepPlan, out):
         """update, its first two launches as one where that can read the rows (eight bytes at a time), and decode"""
         if (kv.shape[0] == sp.slots.shape[0] and kv.stride(0) % 4 == 0 and kv.data_ptr() % 8 == 0
-                and as_defined(self, KiviDecodeLayer, "update")):
+                and runs(self.update, KiviDecodeLayer.update)):
             KIVI.step_write(kv, sp.slots, self.co, self.pool, self.ring, sp.ring_dest, f8=self.f8)
             self._encode_completed(sp)
         else:
