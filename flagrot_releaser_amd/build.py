@@ -28,8 +28,10 @@ STRICT = ["-ffp-contract=off", "-fno-fast-math"]
 if os.environ.get("FLAGROT_STRICT_MERGE", "0") not in ("", "0"):
     COMMON = COMMON + ["-DFLAGROT_STRICT_MERGE=1"]
 
-# loops that begin on an instruction cache line: the 256-row kernel of the dense path on static pages 65.2 -> 64.6 us (7 requests
-# of up to 150 tokens over 3000), 129.7 -> 126.5 (5 of 167 over 9000), key-only pages 81.4 -> 82.0; the other sources gain nothing
+# loops that begin on an instruction cache line: the 256-row kernel of the dense path, whose two groups of
+# wavefronts run different loops, is 0.4 to 1.5 % faster on all nine shapes measured (us without / with: static pages, 7 requests of up to
+# 150 tokens over 3000 57.8 / 57.0, over 6000 96.1 / 95.3, 4 of 512 over 2000 185.1 / 184.4; 2-bit 54.8 / 54.3; key-only 64.6 / 64.0);
+# the other sources gain nothing
 LINED = ["-falign-loops=64"]
 
 # library -> [(source, extra flags)]

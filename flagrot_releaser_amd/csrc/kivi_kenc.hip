@@ -14,7 +14,7 @@
 // wavefronts' sums goes through LDS.  More than 64 queries: the products are formed again once the choices are known.  The
 // queries are read straight from L2 (a lane's 16 bytes are four k-steps of one query).
 //
-// Prompt of 4133 tokens x 8 heads, FP8 meta / one group a head / 256-d heads, 9 groups x 4 (us): a wavefront per (matrix, 32
+// Prompt of 4133 tokens x 8 heads, FP8 meta / 16 groups x 8 heads / 256-d heads, 9 groups x 4 (us): a wavefront per (matrix, 32
 // queries) with weights and shares exchanged through LDS and IEEE quotients 62.3 / 15.7 / 26.6; this form 46.5 / 11.4 / 20.8.
 #include <type_traits>
 

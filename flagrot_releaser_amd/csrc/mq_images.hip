@@ -4,10 +4,11 @@
 //
 // k_mq8 (mq_prefill.hip) converts a block for each query tile that reads it: its vector slots are softmax plus conversion,
 // 5.3 k cycles a block where the matrix instructions take 2 k.  Here the conversion is a launch of its own, bound by the
-// images it writes (139 MB 28 to 36 us), and the attention kernel has nothing between the matrix instructions but the
-// softmax: the images go from memory to LDS without passing through registers, two blocks ahead, 3.5 k cycles a block.
-// At that point the card's power is the bound: the clock falls to 1.5 GHz, 1070 TFLOP/s where a large matrix product
-// reaches 1170.  4 requests x 512 tokens x 64 heads over 16 k on 4-bit key-only pages: 1345 us, here 2 x (523 + 36).
+// images it writes (138 MB in 34 us), and the attention kernel has nothing between the matrix instructions but the
+// softmax: the images go from memory to LDS without passing through registers, two blocks ahead, 3.6 k cycles a block, the
+// matrix pipe busy for 57 % of them (k_mq8 40 %).  4 requests x 512 tokens x 64 heads over 16 k on 4-bit key-only pages: 1222
+// us, here 2 x (500 + 34) on a cache that repeats, 1418 and 2 x (551 + 37) on new inputs; 1117 TFLOP/s where a large matrix
+// product reaches 1170, at a clock of 1.9 GHz (cycles a CU is busy over the dispatch's time; k_mq8 2.2).
 #include "mq_launch.hpp"
 #include "mq_rows256.hpp"
 
