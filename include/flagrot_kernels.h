@@ -38,7 +38,7 @@ int fr_abi_version(void);
  * the pool chunk is two 128-d half chunks per (page, KV head), kmask / vmask are [Hkv, 8], partials are GT*256 floats
  * with GT = 4 and the counter words are not used.  Split s owns tokens [s, s+1)*chunk, except in batches of 2 .. 64
  * sequences with nsplit >= 2, chunk >= 512 and a multiple of 64, nsplit*chunk <= 2^24 and B*Hkv*ceil(gqa/4)*nsplit >= 1.5
- * workgroups a CU: there the B*nsplit parts of a (KV head, q tile) are shared out by seq_lens on the device (same
+ * workgroups a CU: there up to B*nsplit parts of a (KV head, q tile) are shared out by seq_lens on the device (same
  * workspace, partials [KV head, q tile][B*nsplit parts, B window-row parts]), seq_lens must not change before the call
  * has ended, and where a sequence is cut -- so the last bit of its output -- depends on the other lengths of the batch. */
 int fr_v2_attn(int fmt, const void* q, long long q_bs, const uint8_t* pool, const int* block_table, int bt_stride,
